@@ -31,6 +31,9 @@ HIPCC_FLAGS = [
     "-Wno-unused-function",
     # Packed-FP32 VALU forms are kept out of every kernel: plain fp32 code only.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # Matrix results in ordinary registers: a kernel that may use the accumulation registers
+    # gets every result there and copies it out and back for each vector operation on it.
+    "-mllvm", "-amdgpu-mfma-vgpr-form",
 ]
 
 

@@ -36,12 +36,6 @@ __device__ __forceinline__ u32 pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(u32, v);
 }
 
-// a.lo*b.lo + a.hi*b.hi + acc on packed bf16 pairs, accumulated in fp32 (v_dot2c_f32_bf16).
-__device__ __forceinline__ float dot2_bf16(u32 a, u32 b, float acc) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a),
-                                         __builtin_bit_cast(bf16x2_t, b), acc, false);
-}
-
 // DPP lane permutes inside a 16-lane row (wave64 = 4 rows).
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float x) {

@@ -4,47 +4,69 @@
 // block_table, softmax_scale, causal=True) as used at
 // kavor/layers/attention/flash_attention_kvcache.py:80-83.
 //
-// Work decomposition (HBM-bound: every KV byte is read exactly once) -- stream-K
-//   Work is counted in steps of 16 tokens of one sequence; the steps of all sequences
-//   are laid end to end (prefix sums of ceil(ctx / 16), built in LDS by every
-//   workgroup from context_lens).  The kernel is persistent: its grid is the number of
-//   workgroups the GPU holds at once, independent of the batch and of the block-table
-//   width, so a captured graph never launches empty workgroups.  A workgroup is 4
-//   waves = 4 kv heads; ceil(Hkv / 4) consecutive workgroups form a group that walks
-//   one contiguous range of steps for all kv heads (kv heads of one token row share HBM
-//   pages and are fetched together).  Every group gets the same number of steps
-//   (exact balance whatever the context lengths), and at least 128 tokens: a large batch
-//   is split by the grid (the range limit does not bind), while a small one is cut into
-//   short ranges so that it still spreads over many CUs (measured with 8 sequences of
-//   500-2000 tokens: 34.6 us per call with 512-token ranges, 19.5 us with 128).
-//   A wave owns all G = Hq / Hkv query heads of its kv head, so GQA costs no extra KV
-//   traffic.  Lane (r = lane/16, c = lane%16) owns dims [8c, 8c+8) of tokens 4i+r of a
-//   step (i = 0..3): 4 dwordx4 loads of K and 4 of V per lane, each 16-lane row
-//   reading one 256-byte head row.  The loads of step n+1 are issued before step n is
-//   computed (register double buffer), so 8-16 KiB per wave stay in flight.  KV rows are
-//   read with the nontemporal hint (each byte is used once; measured +12% on MI355X over
-//   plain loads, which keep the stream in L2 for nothing); addresses
-//   past the context are clamped onto its last token (masked in the softmax), so no
-//   branch guards a load.
-//   Scores: q.k with v_dot2c_f32_bf16 on packed bf16 pairs, then a 4-step DPP sum
-//   across the 16-lane row.  Softmax: online, base 2, scale*log2(e) folded into the
-//   scores, one running (max, sum, acc[8]) per lane row.
-//   Output: where a wave's range ends or a sequence ends, the 4 lane rows are merged
-//   with cross-lane shuffles; a sequence covered by one range writes bf16 directly,
-//   otherwise each range writes (max, sum, unnormalised acc) in fp32 to the workspace
-//   and decode_merge_kernel combines them with the same online-softmax rule.  Partial
-//   traffic is about 2 states per group per sequence boundary: well under 1% of the KV
-//   bytes.
-//   Partial slots: the state that range r writes for sequence b goes to slot r + b.
-//   Sequence b's ranges are first_b .. last_b (first_b = cum_b / spr), and the next
-//   sequence with steps starts at a range >= last_b, so slots are unique, and one
-//   sequence's slots are consecutive.  A launch with R ranges over B sequences uses at
-//   most R + B slots of num_q_heads states each, whatever the context lengths.
+// What bounds it: HBM, since every K/V byte is read exactly once; for the smallest batches
+// the chain of dependent loads and the instructions around it.
+//
+// Work decomposition -- stream-K
+//   Work is counted in steps of 32 tokens of one sequence; the steps of all sequences are
+//   laid end to end (prefix sums of ceil(ctx / 32), built in LDS by every workgroup from
+//   context_lens).  The grid is the number of workgroups the GPU holds at once (one of 4
+//   waves per CU), independent of the batch and of the block-table width, so a captured
+//   graph never launches empty workgroups.  A workgroup's waves are 4 kv heads;
+//   ceil(Hkv / 4) workgroups walk one contiguous range of steps for all kv heads (kv heads
+//   of one token row share HBM pages and are fetched together).  Every range gets the same
+//   number of steps (exact balance whatever the context lengths).  A wave owns all
+//   G = Hq / Hkv query heads of its kv head, so GQA costs no extra KV traffic.
+//
+// Why the matrix cores, although the work is HBM-bound: on the vector ALUs the q.k dot
+// products, their lane sums and the P V products grow with G while the K/V bytes do not.
+// At G = 8 a wave needed more issue cycles for a step than HBM needs to deliver it, and the
+// registers that held the K/V double buffer were short.  Here both products run as
+// v_mfma_f32_16x16x32_bf16 with the G heads as columns, a fixed 24 (G <= 5) or 32 (G = 8)
+// matrix instructions per step.  Measured against the vector-ALU kernel (MI355X, whole
+// calls, the two in turn): 64 sequences of 1000-9000 tokens at G = 8, one-launch step:
+// 382 -> 215 us (3.4 -> 6.1 TB/s); 128 sequences of 1024-32768 tokens at G = 4: 1300 ->
+// 1269 us (7.0 TB/s); 256 sequences of 100-2048 tokens at G = 2, with the append: 182 ->
+// 177 us; 8 sequences of 600-3000 tokens at G = 2: 22.8 -> 21.8 us per layer.
+//
+// K and V rows go from memory into the wave's own LDS tiles (32 tokens x 256 bytes, two of
+// each) with direct-to-LDS buffer loads: no register holds them, no barrier is needed, and
+// a tile is refilled as soon as its step has read it, two steps ahead, so 24-32 KiB per
+// wave are in flight all the time.  They are read with the nontemporal hint; rows past the
+// context are clamped onto its last token (masked in the softmax), so no branch guards a
+// load.
+//
+// Layouts (lane l: n = l % 16, q4 = l / 16).  S = K Q^T: A is the K tile (row n of 16
+// tokens, dims 8 q4 + e of each 32), B is q (column n); the lane gets the scores of tokens
+// 4 q4 + j, j = 0..3, of both 16-token halves for its column.  O^T += V^T P^T: A is V^T by
+// the LDS transpose load, B is P straight from the score registers (the k index of
+// (q4, e) is token 4 q4 + e of the first half for e < 4, of the second for e >= 4), and the
+// lane gets dims 16 mt + 4 q4 + j of its column.
+//
+// P stays exact to fp32: the weight is split into bf16 parts p = p0 + p1 + p2 (8 bits of
+// mantissa each), and the 16 columns hold the parts of the G heads side by side (column n:
+// part n / G of head n % G; q is repeated, so every column forms its own part from its own
+// scores).  Three parts fit for G <= 5; G = 8 holds two and adds the third with a second
+// product.  The parts of a head are summed in fp32 when the state is written.  Tile rows are
+// swizzled by 16-byte chunks, K by row & 15 and V by 2 (row & 7), so neither the 16-byte
+// reads nor the transpose reads share a bank.  Softmax: online, base 2, scale*log2(e)
+// folded into the scores, one running (max, sum) per column and row group.
+//
+// Output: where a wave's range ends or a sequence ends its state is written; a sequence
+// covered by one range gives bf16 directly, otherwise each range writes (max, sum,
+// unnormalised acc) in fp32 to the workspace and decode_merge_kernel combines them with the
+// same online-softmax rule.  Partial traffic is about 2 states per group per sequence
+// boundary: well under 1% of the KV bytes.
+//
+// Partial slots: the state that range r writes for sequence b goes to slot r + b.
+// Sequence b's ranges are first_b .. last_b (first_b = cum_b / spr), and the next
+// sequence with steps starts at a range >= last_b, so slots are unique, and one
+// sequence's slots are consecutive.  A launch with R ranges over B sequences uses at
+// most R + B slots of num_q_heads states each, whatever the context lengths.
 #include <math.h>
 
 #include <algorithm>
 #include <atomic>
-#include <type_traits>
 
 #include "common.h"
 
@@ -53,14 +75,33 @@ namespace kvp {
 constexpr int kDecodeHeadDim = 128;
 constexpr int kDecodeWaves = 4;  // kv heads per workgroup
 constexpr int kDecodeThreads = 64 * kDecodeWaves;
-constexpr int kMinRangeTokens = 128;        // a range covers at least 128 tokens
-constexpr int kMinStepTokens = 16;           // smallest step (G = 8); G <= 4 steps 32 tokens
-constexpr int kG5Step = 32;                  // G = 5 (Qwen3-14B: 40 q heads over 8 kv heads)
-constexpr int kMaxSeqsPerLaunch = 4096;      // size of the LDS prefix-sum table
-constexpr int kHeaderInts = 16;              // workspace header before the prefix table
-// Upper bound of the persistent grid.  The variants hold 1 or 2 workgroups per CU on
-// MI355X (at most 512 in all); the cap makes the workspace bound independent of the device.
+constexpr int kStep = 32;               // tokens per step
+constexpr int kTileBytes = kStep * 256;  // one K or V tile
+constexpr int kMinRangeTokens = 128;  // a range covers at least 128 tokens
+constexpr int kSeqsPerLaunch = 1024;  // sequences per launch (LDS tables); more run as consecutive launches
+constexpr int kHeaderSeqs = 4096;     // sequences the workspace formula counts at most
+constexpr int64_t kMaxDmaRow = 1 << 24;  // row stride (elements) up to which 32 rows are addressed in 32 bits
+constexpr int kHeaderInts = 16;          // workspace header before the prefix table
+// Upper bound of the persistent grid; the cap makes the workspace bound independent of the
+// device.
 constexpr int kMaxDecodeGrid = 1024;
+
+// n / d for 0 <= n < 2^31 by a multiplication (the compiler's division is some 30
+// instructions, most of them executed once per launch from a cold instruction cache).
+// With l = ceil(log2 d) and mul = ceil(2^(31 + l) / d), n * mul / 2^(31 + l) exceeds n / d
+// by less than n / 2^(31 + l) <= 1 / d for n < 2^31, so the floor is exact.
+struct Divisor {
+  uint32_t mul, shift;  // shift = l - 1 beyond the high word; d = 1: mul = 0
+};
+static Divisor divisor(uint32_t d) {
+  if (d <= 1) return Divisor{0, 0};
+  uint32_t l = 0;
+  while ((1ull << l) < d) ++l;
+  return Divisor{static_cast<uint32_t>(((1ull << (31 + l)) + d - 1) / d), l - 1};
+}
+__device__ __forceinline__ int div_by(int n, const Divisor& d) {
+  return d.mul ? static_cast<int>(__umulhi(static_cast<uint32_t>(n), d.mul) >> d.shift) : n;
+}
 
 struct DecodeParams {
   const uint16_t* q;
@@ -72,12 +113,11 @@ struct DecodeParams {
   const int32_t* block_tables;
   int64_t bt_stride;
   const int32_t* context_lens;
-  int32_t num_seqs;  // <= kMaxSeqsPerLaunch
+  int32_t num_seqs;  // <= kSeqsPerLaunch
   int32_t num_q_heads;
   int32_t num_kv_heads;
   int32_t block_size;
   int32_t max_blocks;
-  int32_t step_tokens;  // tokens per step (the kernel's STEP)
   float scale_log2;   // softmax_scale * log2(e)
   uint16_t* out;
   int64_t o_seq_stride, o_head_stride;
@@ -96,6 +136,9 @@ struct DecodeParams {
   float eps;
   const int32_t* slot_mapping;
   int64_t num_cache_slots;
+  Divisor div_block, div_ranges;  // by block_size and by the launch's range count
+  // 32 token rows / the q heads of one kv head fit 32-bit byte offsets
+  bool rows_by_dma, q_by_dma;
 };
 
 __device__ __forceinline__ uint4 load16(const uint16_t* ptr) {
@@ -114,39 +157,42 @@ __device__ __forceinline__ int load_uniform(const int32_t* base, int64_t idx) {
 // Steps of a sequence; 0 for empty or impossible contexts (written separately).
 __device__ __forceinline__ int seq_steps(int ctx, const DecodeParams& p) {
   if (ctx <= 0 || ctx > p.max_blocks * p.block_size) return 0;
-  return (ctx + p.step_tokens - 1) / p.step_tokens;
+  return (ctx + kStep - 1) / kStep;
 }
 
-// s_cum[b] = steps of sequences 0..b-1 (b = 0..num_seqs), built by the whole workgroup:
-// each thread sums a contiguous run of sequences, then the 256 run totals are scanned
-// with DPP within each wave and the 4 wave totals through LDS (one barrier; a
-// Hillis-Steele scan over LDS took 16: 15.0 -> 14.65 us per call for 4 sequences).
-__device__ void build_step_prefix(const DecodeParams& p, int* s_cum, int* s_part) {
+// Rows with nothing to attend (ctx 0: graph padding) read as zeros; impossible lengths read
+// as NaN.  Neither has steps.
+__device__ __forceinline__ void fill_row(const DecodeParams& p, int b, int ctx) {
+  const u32 w = ctx <= 0 ? 0u : 0x7fc07fc0u;
+#pragma unroll 1
+  for (int o = 0; o < p.num_q_heads * kDecodeHeadDim; o += 8)
+    *reinterpret_cast<uint4*>(p.out + b * p.o_seq_stride + (o / kDecodeHeadDim) * p.o_head_stride +
+                              o % kDecodeHeadDim) = make_uint4(w, w, w, w);
+}
+
+// s_ctx[b] = context length, s_cum[b] = steps of sequences 0..b-1 (b = 0..num_seqs), built by
+// the whole workgroup: each thread sums a contiguous run of sequences, then the 256 run
+// totals are scanned with DPP within each wave and the 4 wave totals through LDS.
+__device__ __forceinline__ void build_step_prefix(const DecodeParams& p, int* s_cum, int* s_ctx, int* s_part) {
   const int tid = threadIdx.x;
   const int B = p.num_seqs;
   const int per = (B + kDecodeThreads - 1) / kDecodeThreads;
-  const int j0 = tid * per;
+  const int j0 = tid * per, j1 = min(j0 + per, B);
+  // the first entry of each block-table row, so that the table read that waits for the
+  // lengths finds its line in L2
+  int warm = 0;
+  if (tid < B) warm = p.block_tables[tid * p.bt_stride];
+  const int wg = blockIdx.y * gridDim.x + blockIdx.x, wgs = gridDim.x * gridDim.y;
   int local = 0;
-  for (int i = 0; i < per; ++i) {
-    const int b = j0 + i;
-    if (b < B) local += seq_steps(p.context_lens[b], p);
-  }
-  // Rows with nothing to attend (ctx 0: graph padding) read as zeros; impossible
-  // lengths read as NaN.  Neither has steps.  Workgroup w writes rows b == w (mod grid).
-  for (int i = 0; i < per; ++i) {
-    const int b = j0 + i;
-    if (b >= B || b % static_cast<int>(gridDim.x) != static_cast<int>(blockIdx.x)) continue;
+#pragma unroll 1
+  for (int b = j0; b < j1; ++b) {
     const int ctx = p.context_lens[b];
-    if (ctx > 0 && ctx <= p.max_blocks * p.block_size) continue;
-    const uint16_t fill = ctx <= 0 ? 0 : 0x7fc0;
-    for (int o = 0; o < p.num_q_heads * kDecodeHeadDim; o += 8) {
-      const int h = o / kDecodeHeadDim, d = o - h * kDecodeHeadDim;
-      const uint4 f = make_uint4(fill * 0x10001u, fill * 0x10001u, fill * 0x10001u, fill * 0x10001u);
-      *reinterpret_cast<uint4*>(p.out + b * p.o_seq_stride + h * p.o_head_stride + d) = f;
-    }
+    const int steps = seq_steps(ctx, p);
+    s_ctx[b] = ctx;
+    local += steps;
+    if (steps == 0 && b % wgs == wg) fill_row(p, b, ctx);
   }
-  // Inclusive scan of the run totals within each wave (DPP and lane reads), then across
-  // the 4 waves through LDS: one barrier.
+  asm volatile("" ::"v"(warm));
   const int lane = tid & 63, wave = tid >> 6;
   const int incl = wave_incl_scan(local);
   if (lane == 63) s_part[wave] = incl;
@@ -156,18 +202,16 @@ __device__ void build_step_prefix(const DecodeParams& p, int* s_cum, int* s_part
   for (int w = 0; w < kDecodeWaves - 1; ++w)
     if (w < wave) before += s_part[w];
   int run = before + incl - local;
-  for (int i = 0; i < per; ++i) {
-    const int b = j0 + i;
-    if (b < B) {
-      s_cum[b] = run;
-      run += seq_steps(p.context_lens[b], p);
-    }
+#pragma unroll 1
+  for (int b = j0; b < j1; ++b) {
+    s_cum[b] = run;
+    run += seq_steps(s_ctx[b], p);
   }
   if (tid == kDecodeThreads - 1) s_cum[B] = before + incl;
   __syncthreads();
 }
 
-// Ranges [part_first(b), part_last(b)] touch sequence b's steps [cum_b, cum_b1).
+// Ranges [cum_b / spr, (cum_b1 - 1) / spr] touch sequence b's steps [cum_b, cum_b1).
 __device__ __forceinline__ int num_parts(int cum_b, int cum_b1, int spr) {
   return (cum_b1 - 1) / spr - cum_b / spr + 1;
 }
@@ -181,159 +225,53 @@ struct StepCursor {
   int lblk;     // logical block whose id is cached in blk (-1: none)
   int blk;      // physical block id of lblk
   int pf_blk;   // id of block lblk + 1, loaded one block ahead (-1: not loaded)
-  bool bad;     // a needed block id was out of range
+  int bad;      // a needed block id was out of range (an int: the struct copies stay in registers)
 };
 
-__device__ __forceinline__ void cursor_start_seq(const DecodeParams& p, StepCursor& cur, int b, int j) {
+// The cursor of step S, which belongs to sequence b.
+__device__ __forceinline__ void cursor_start_seq(StepCursor& cur, const int* s_cum, const int* s_ctx, int b, int S) {
+  const int cum = __builtin_amdgcn_readfirstlane(s_cum[b]);
   cur.b = b;
-  cur.j = j;
-  cur.ctx = load_uniform(p.context_lens, b);
-  cur.nsteps = seq_steps(cur.ctx, p);
+  cur.j = S - cum;
+  cur.ctx = __builtin_amdgcn_readfirstlane(s_ctx[b]);
+  cur.nsteps = __builtin_amdgcn_readfirstlane(s_cum[b + 1]) - cum;
   cur.lblk = -1;
   cur.blk = 0;
   cur.pf_blk = -1;
-  cur.bad = false;
+  cur.bad = 0;
 }
 
-// Address (in elements) of this lane's first token of the cursor's step, and the number
-// of valid tokens of the step.  On entering a block it takes the id prefetched one
-// block earlier (or loads it) and prefetches the next block's id, so the scalar load
-// is off the critical path.
-template <int STEP>
-__device__ __forceinline__ int64_t step_base(const DecodeParams& p, StepCursor& cur, int64_t head_off,
-                                            int& nvalid) {
-  const int t0 = cur.j * STEP;
-  const int lblk = t0 / p.block_size;
+// Element offset of the cursor's step in the caches, and the number of valid tokens of the
+// step.  On entering a block it takes the id prefetched one block earlier (or loads it) and
+// prefetches the next block's id, so the scalar load is off the critical path.
+__device__ __forceinline__ int64_t step_base(const DecodeParams& p, StepCursor& cur, int64_t head_off, int& nvalid) {
+  const int t0 = cur.j * kStep;
+  const int lblk = div_by(t0, p.div_block);
   if (lblk != cur.lblk) {
     const int32_t* row = p.block_tables + cur.b * p.bt_stride;
     int blk = (cur.lblk >= 0 && lblk == cur.lblk + 1 && cur.pf_blk != -1) ? cur.pf_blk : load_uniform(row, lblk);
     if (blk < 0 || blk >= p.num_cache_blocks) {
-      cur.bad = true;
+      cur.bad = 1;
       blk = 0;
     }
     cur.blk = blk;
     cur.lblk = lblk;
     cur.pf_blk = (lblk + 1) * p.block_size < cur.ctx ? load_uniform(row, lblk + 1) : -1;
   }
-  nvalid = min(STEP, cur.ctx - t0);
+  nvalid = min(kStep, cur.ctx - t0);
   return static_cast<int64_t>(cur.blk) * p.blk_stride +
          static_cast<int64_t>(t0 - lblk * p.block_size) * p.slot_stride + head_off;
-}
-
-// Token 4i + r of the step, clamped onto the last valid token so every load is in
-// bounds and needs no branch; clamped tokens are masked out of the softmax.
-template <int NL>
-__device__ __forceinline__ void step_load(const DecodeParams& p, int64_t base, int nvalid, int r,
-                                          uint4 (&kr)[NL], uint4 (&vr)[NL]) {
-#pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    const int t = min(4 * i + r, nvalid - 1);
-    kr[i] = load16_nt(p.k_cache + base + t * p.slot_stride);
-    vr[i] = load16_nt(p.v_cache + base + t * p.slot_stride);
-  }
-}
-
-template <int G, int NL>
-__device__ __forceinline__ void step_compute(const DecodeParams& p, const uint4 (&qv)[G],
-                                             const uint4 (&kr)[NL], const uint4 (&vr)[NL],
-                                             int nvalid, int r, float (&m)[G], float (&l)[G],
-                                             float (&acc)[G][8]) {
-  float s[G][NL];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float mx = kMaxFloor;
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      float part = dot2_bf16(qv[g].x, kr[i].x, 0.f);
-      part = dot2_bf16(qv[g].y, kr[i].y, part);
-      part = dot2_bf16(qv[g].z, kr[i].z, part);
-      part = dot2_bf16(qv[g].w, kr[i].w, part);
-      const float sc = row16_sum(part) * p.scale_log2;
-      s[g][i] = (4 * i + r < nvalid) ? sc : -INFINITY;
-      mx = fmaxf(mx, s[g][i]);
-    }
-    const float m_new = fmaxf(m[g], mx);
-    const float alpha = fast_exp2(m[g] - m_new);
-    m[g] = m_new;
-    l[g] *= alpha;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[g][j] *= alpha;
-  }
-  // P V: each V row is widened to fp32 once and feeds all G heads.
-#pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    const float vf[8] = {bf16_lo(vr[i].x), bf16_hi(vr[i].x), bf16_lo(vr[i].y), bf16_hi(vr[i].y),
-                         bf16_lo(vr[i].z), bf16_hi(vr[i].z), bf16_lo(vr[i].w), bf16_hi(vr[i].w)};
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const float pr = fast_exp2(s[g][i] - m[g]);
-      l[g] += pr;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) acc[g][j] += pr * vf[j];
-    }
-  }
-}
-
-// Merges the 4 lane rows of the wave and writes the state of (b, kvh) for this range:
-// the bf16 output when one range covers the sequence, otherwise an fp32 partial.
-template <int G>
-__device__ __forceinline__ void emit_state(const DecodeParams& p, int b, int kvh, int slot, bool single,
-                                           bool bad, int lane, float (&m)[G], float (&l)[G],
-                                           float (&acc)[G][8]) {
-  const int c = lane & 15;
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const float mm = xor32_max(xor16_max(m[g]));
-    const float sc = fast_exp2(m[g] - mm);
-    const float ll0 = xor32_sum(xor16_sum(l[g] * sc));
-    float a[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) a[j] = xor32_sum(xor16_sum(acc[g][j] * sc));
-    float ll = ll0;
-    if (bad) ll = NAN;
-    const int h = kvh * G + g;
-    if (lane < 16) {
-      if (single) {
-        const float inv = 1.f / ll;
-        uint4 o;
-        o.x = pack_bf16x2(a[0] * inv, a[1] * inv);
-        o.y = pack_bf16x2(a[2] * inv, a[3] * inv);
-        o.z = pack_bf16x2(a[4] * inv, a[5] * inv);
-        o.w = pack_bf16x2(a[6] * inv, a[7] * inv);
-        *reinterpret_cast<uint4*>(p.out + b * p.o_seq_stride + h * p.o_head_stride + 8 * c) = o;
-      } else {
-        const int64_t row = static_cast<int64_t>(slot) * p.num_q_heads + h;
-        float4* dst = reinterpret_cast<float4*>(p.part_o + row * kDecodeHeadDim + 8 * c);
-        dst[0] = make_float4(a[0], a[1], a[2], a[3]);
-        dst[1] = make_float4(a[4], a[5], a[6], a[7]);
-        if (c == 0) *reinterpret_cast<float2*>(p.part_ml + row * 2) = make_float2(mm, ll);
-      }
-    }
-  }
 }
 
 // ---- fused q/k norm + RoPE + append (FUSED kernels)
 //
 // The inputs of the q of a sequence (its cos/sin row and raw q heads) and of its new token
-// (cos/sin row, raw k and v heads) reach a per-wave LDS scratch with direct-to-LDS buffer
-// loads (buffer_load_dwordx4 ... lds: lane l writes 16 bytes at M0 + 16 l), issued one
-// step before they are needed, so the wave never waits on a dependent load chain at a
-// sequence boundary and no VGPR holds them meanwhile.  Each kind has two regions, one per
-// copy of the unrolled step loop; a region is read by the step copy that consumes it and
-// written only by the other copy.  A region read at the end of step S was filled during
-// step S - 1, after the K/V loads of step S and before those of step S + 1 (2 NL loads);
-// vector memory operations complete in issue order, so an explicit wait that leaves at
-// most 2 NL of them in flight covers it.  The compiler's own tracking of direct-to-LDS
-// loads does not order these reads, hence the explicit wait.  The token's position is
+// (cos/sin row, raw k and v heads) reach a per-wave LDS region with direct-to-LDS buffer
+// loads one step before they are needed, so the wave never waits on a dependent load chain
+// at a sequence boundary and no VGPR holds them meanwhile.  The token's position is
 // context_lens[b] - 1.
 constexpr int kFzRow = 512;  // bytes: one cos/sin row, 128 fp32
 constexpr int kFzNew = 1024;  // new token: cos/sin row | raw k head | raw v head
-template <int G>
-struct FzSize {  // q of a sequence: cos/sin row | G raw q heads, in 1 KiB loads
-  static constexpr int kLoads = (kFzRow + G * 256 + 1023) / 1024;
-  static constexpr int kBytes = kLoads * 1024;
-};
-
 __device__ __forceinline__ BufferRsrc cos_sin_rsrc(const DecodeParams& p) {
   return buffer_rsrc(p.cos_sin, static_cast<uint32_t>(p.max_position) * kFzRow);
 }
@@ -358,7 +296,7 @@ __device__ __forceinline__ void fz_issue_q(const DecodeParams& p, int b, int ctx
   if (lane < 32) lds_dma16(cos_sin_rsrc(p), fz_row_bytes(p, ctx) + 16 * lane, region);
   const int heads = (b * static_cast<int>(p.qkv_stride) + kvh * G * kRopeDim) * 2;
 #pragma unroll
-  for (int i = 0; i < FzSize<G>::kLoads; ++i) {
+  for (int i = 0; i < (kFzRow + G * 256 + 1023) / 1024; ++i) {
     const int byte = 1024 * i + 16 * lane;  // this lane's destination within the region
     if (byte >= kFzRow && byte < kFzRow + G * 256) lds_dma16(qkv_rsrc(p), heads + byte - kFzRow, region + 1024 * i);
   }
@@ -375,110 +313,229 @@ __device__ __forceinline__ void fz_issue_new(const DecodeParams& p, int b, int c
   }
 }
 
-__device__ __forceinline__ void fz_cos_sin(const char* row, int c, float (&cs)[8], float (&sn)[8]) {
-  const float* f = reinterpret_cast<const float*>(row) + 8 * (c & 7);
-  *reinterpret_cast<float4*>(cs) = *reinterpret_cast<const float4*>(f);
-  *reinterpret_cast<float4*>(cs + 4) = *reinterpret_cast<const float4*>(f + 4);
-  *reinterpret_cast<float4*>(sn) = *reinterpret_cast<const float4*>(f + kRopeDim / 2);
-  *reinterpret_cast<float4*>(sn + 4) = *reinterpret_cast<const float4*>(f + kRopeDim / 2 + 4);
+typedef __bf16 mfma_bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float mfma_f32x4_t __attribute__((ext_vector_type(4)));
+
+
+__device__ __forceinline__ mfma_f32x4_t mfma16(u32x4_t a, u32x4_t b, mfma_f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mfma_bf16x8_t, a),
+                                                 __builtin_bit_cast(mfma_bf16x8_t, b), c, 0, 0, 0);
+}
+// All LDS accesses of the wave are done: what they read may be overwritten.
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// Tile accesses are written out, each block with its own wait: the compiler cannot tell a
+// tile from the one being filled and would wait for every load in flight.
+__device__ __forceinline__ u32 lds_addr(const void* p) {
+  return static_cast<u32>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)(p)));
+}
+// The 16 bytes at a[i] and at a[i] + 4096 (the tile's two 16-token halves), i = 0..3.
+__device__ __forceinline__ void read_k_tile(const u32 (&a)[4], u32x4_t (&k)[8]) {
+  asm volatile(
+      "ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:4096\n\t"
+      "ds_read_b128 %2, %9\n\tds_read_b128 %3, %9 offset:4096\n\t"
+      "ds_read_b128 %4, %10\n\tds_read_b128 %5, %10 offset:4096\n\t"
+      "ds_read_b128 %6, %11\n\tds_read_b128 %7, %11 offset:4096\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(k[0]), "=&v"(k[1]), "=&v"(k[2]), "=&v"(k[3]), "=&v"(k[4]), "=&v"(k[5]), "=&v"(k[6]), "=&v"(k[7])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3])
+      : "memory");
+}
+typedef u32 u32x2_t __attribute__((ext_vector_type(2)));
+// Transposed 8-byte reads at a[i] (first half) and a[i] + 4096 (second half), i = 0..7.
+__device__ __forceinline__ void read_v_tile(const u32 (&a)[8], u32x2_t (&lo)[8], u32x2_t (&hi)[8]) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %16\n\tds_read_b64_tr_b16 %8, %16 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %1, %17\n\tds_read_b64_tr_b16 %9, %17 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %2, %18\n\tds_read_b64_tr_b16 %10, %18 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %3, %19\n\tds_read_b64_tr_b16 %11, %19 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %4, %20\n\tds_read_b64_tr_b16 %12, %20 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %5, %21\n\tds_read_b64_tr_b16 %13, %21 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %6, %22\n\tds_read_b64_tr_b16 %14, %22 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %7, %23\n\tds_read_b64_tr_b16 %15, %23 offset:4096\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(lo[0]), "=&v"(lo[1]), "=&v"(lo[2]), "=&v"(lo[3]), "=&v"(lo[4]), "=&v"(lo[5]), "=&v"(lo[6]),
+        "=&v"(lo[7]), "=&v"(hi[0]), "=&v"(hi[1]), "=&v"(hi[2]), "=&v"(hi[3]), "=&v"(hi[4]), "=&v"(hi[5]),
+        "=&v"(hi[6]), "=&v"(hi[7])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7])
+      : "memory");
+}
+// A head's inputs for norm_rope_head: the lane's norm weights, cos and sin, and two 16-byte
+// chunks x0, x1.
+struct HeadInputs {
+  u32x4_t w, cos[2], sin[2], x0, x1;
+};
+__device__ __forceinline__ HeadInputs read_head(u32 w_at, u32 table_at, u32 x0_at, u32 x1_at) {
+  HeadInputs h;
+  asm volatile(
+      "ds_read_b128 %0, %7\n\tds_read_b128 %1, %8\n\tds_read_b128 %2, %8 offset:16\n\t"
+      "ds_read_b128 %3, %8 offset:256\n\tds_read_b128 %4, %8 offset:272\n\t"
+      "ds_read_b128 %5, %9\n\tds_read_b128 %6, %10\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(h.w), "=&v"(h.cos[0]), "=&v"(h.cos[1]), "=&v"(h.sin[0]), "=&v"(h.sin[1]), "=&v"(h.x0), "=&v"(h.x1)
+      : "v"(w_at), "v"(table_at), "v"(x0_at), "v"(x1_at)
+      : "memory");
+  return h;
+}
+__device__ __forceinline__ uint4 norm_rope_chunk(const HeadInputs& h, u32x4_t raw, int c, bool pos_ok, float eps) {
+  float w[8], x[8], cs[8], sn[8];
+  unpack8(__builtin_bit_cast(uint4, h.w), w);
+  unpack8(__builtin_bit_cast(uint4, raw), x);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    cs[e] = __uint_as_float(h.cos[e >> 2][e & 3]);
+    sn[e] = __uint_as_float(h.sin[e >> 2][e & 3]);
+  }
+  norm_rope_head(x, w, cs, sn, c < 8, pos_ok, eps);
+  return pack8(x);
+}
+// q of one column in the B layout: 16 bytes at a, a + 64, a + 128, a + 192.
+__device__ __forceinline__ void read_q(u32 a, u32x4_t (&q)[4]) {
+  asm volatile(
+      "ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:64\n\t"
+      "ds_read_b128 %2, %4 offset:128\n\tds_read_b128 %3, %4 offset:192\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3])
+      : "v"(a)
+      : "memory");
+}
+__device__ __forceinline__ void write_tile16(u32 addr, uint4 v) {
+  asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(__builtin_bit_cast(u32x4_t, v)) : "memory");
 }
 
-// q of a sequence from its q region: RMS-normalised and rotated, in the decode's q layout
-// (lane c: dims 8c..8c+7 of every head).
+// x of the lane N places up in the 16-lane row (0 past its end).
+template <int N>
+__device__ __forceinline__ float row_up(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x100 + N, 0xf, 0xf, false));
+}
+
+// The lane's parts of the tile fills.  Instruction i fills rows 4 i .. 4 i + 3 of a tile:
+// lane l writes row r = 4 i + l / 16 at physical chunk l % 16, which holds logical chunk
+// (l % 16) ^ (r & 15) of K and (l % 16) ^ 2 (r & 7) of V.
+struct TileLane {
+  int r, c;        // l / 16, l % 16
+  int row_off;     // byte offset of row r
+  int k_chunk[4];  // 16 (c ^ (4 i + r)), i = 0..3
+  int v_chunk[2];  // 16 (c ^ 2 ((4 i + r) & 7)), i = 0..1
+};
+// Rows of a tile from element `base` of the cache: row r is token r, rows past the last one
+// repeat it, so every load is in bounds.  Strides whose 32 rows do not fit 32-bit byte
+// offsets go through registers.
+template <bool V>
+__device__ __forceinline__ void issue_tile(const DecodeParams& p, const TileLane& ln, int64_t base, int rows,
+                                                char* tile) {
+  const uint16_t* src = (V ? p.v_cache : p.k_cache) + base;
+  if (p.rows_by_dma) {  // uniform
+    const int row_bytes = static_cast<int>(p.slot_stride) * 2;
+    const BufferRsrc rsrc = buffer_rsrc(src, static_cast<uint32_t>((kStep - 1) * row_bytes + 256));
+    const int last = (rows - 1) * row_bytes;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)  // nontemporal: every row is read once
+      raw_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(tile + 1024 * i), 16,
+                          min(ln.row_off + 4 * i * row_bytes, last) + (V ? ln.v_chunk[i & 1] : ln.k_chunk[i & 3]), 0,
+                          0, 2);
+  } else {
+#pragma unroll 1
+    for (int row = ln.r; row < kStep; row += 4) {
+      const int chunk = 16 * (ln.c ^ (V ? 2 * (row & 7) : row & 15));
+      const char* at = reinterpret_cast<const char*>(src + min(row, rows - 1) * p.slot_stride) + chunk;
+      write_tile16(lds_addr(tile) + 256 * row + 16 * ln.c, load16_nt(at));
+    }
+  }
+}
+
 template <int G>
-__device__ __forceinline__ void fz_finish_q(const DecodeParams& p, int ctx, int c, const char* region,
-                                            const char* weights, uint4 (&qv)[G]) {
-  const bool pos_ok = ctx - 1 >= 0 && ctx - 1 < p.max_position;
-  float w[8], cs[8], sn[8];
-  unpack8(*reinterpret_cast<const uint4*>(weights + 16 * c), w);
-  fz_cos_sin(region, c, cs, sn);
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float x[8];
-    unpack8(*reinterpret_cast<const uint4*>(region + kFzRow + 256 * g + 16 * c), x);
-    norm_rope_head(x, w, cs, sn, c < 8, pos_ok, p.eps);
-    qv[g] = pack8(x);
-  }
-}
-
-// The new token of sequence b: k normalised and rotated, v as is; both appended at
-// slot_mapping[b] (-1 or a slot outside the pool: not stored) by lanes 0-15, and folded
-// into the wave's online softmax as one more key (counted in lane row 0 only; the step
-// that loaded its slot masked it out).  Only the wave owning the sequence's final step of
-// kv head kvh runs this, so the appended token is never read from the cache in the launch.
+struct State {
+  float m, l;
+  mfma_f32x4_t acc[8];               // column n's part; dims 16 mt + 4 q4 + j
+  mfma_f32x4_t acc2[G > 5 ? 8 : 1];  // G = 8: the third part, in columns 8..15
+};
 template <int G>
-__device__ __forceinline__ void fz_finish_new(const DecodeParams& p, int b, int ctx, int kvh, int r, int c,
-                                              const char* region, const char* weights, const uint4 (&qv)[G],
-                                              float (&m)[G], float (&l)[G], float (&acc)[G][8]) {
-  const bool pos_ok = ctx - 1 >= 0 && ctx - 1 < p.max_position;
-  const int slot = load_uniform(p.slot_mapping, b);
-  float w[8], cs[8], sn[8], x[8];
-  unpack8(*reinterpret_cast<const uint4*>(weights + 256 + 16 * c), w);
-  fz_cos_sin(region, c, cs, sn);
-  unpack8(*reinterpret_cast<const uint4*>(region + kFzRow + 16 * c), x);
-  const uint4 vraw = *reinterpret_cast<const uint4*>(region + kFzRow + 256 + 16 * c);
-  norm_rope_head(x, w, cs, sn, c < 8, pos_ok, p.eps);
-  const uint4 knew = pack8(x);
-  if (r == 0 && slot >= 0 && slot < p.num_cache_slots) {
-    const int blk = slot / p.block_size, off = slot - blk * p.block_size;
-    const int64_t at = static_cast<int64_t>(blk) * p.blk_stride + static_cast<int64_t>(off) * p.slot_stride +
-                       static_cast<int64_t>(kvh) * p.head_stride + 8 * c;
-    *reinterpret_cast<uint4*>(const_cast<uint16_t*>(p.k_cache) + at) = knew;
-    *reinterpret_cast<uint4*>(const_cast<uint16_t*>(p.v_cache) + at) = vraw;
-  }
-  const float vf[8] = {bf16_lo(vraw.x), bf16_hi(vraw.x), bf16_lo(vraw.y), bf16_hi(vraw.y),
-                       bf16_lo(vraw.z), bf16_hi(vraw.z), bf16_lo(vraw.w), bf16_hi(vraw.w)};
+__device__ __forceinline__ void reset_state(State<G>& st) {
+  st.m = kMaxFloor;
+  st.l = 0.f;
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float part = dot2_bf16(qv[g].x, knew.x, 0.f);
-    part = dot2_bf16(qv[g].y, knew.y, part);
-    part = dot2_bf16(qv[g].z, knew.z, part);
-    part = dot2_bf16(qv[g].w, knew.w, part);
-    const float sc = r == 0 ? row16_sum(part) * p.scale_log2 : -INFINITY;
-    const float m_new = fmaxf(m[g], sc);
-    const float alpha = fast_exp2(m[g] - m_new);
-    const float pr = fast_exp2(sc - m_new);
-    m[g] = m_new;
-    l[g] = l[g] * alpha + pr;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[g][j] = acc[g][j] * alpha + pr * vf[j];
+  for (int mt = 0; mt < 8; ++mt) {
+    st.acc[mt] = mfma_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (G > 5) st.acc2[mt] = mfma_f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 }
 
-template <int G, int STEP, bool FUSED>
-__global__ __launch_bounds__(kDecodeThreads) void paged_decode_kernel(const DecodeParams p) {
-  constexpr int NL = STEP / 4;  // dwordx4 loads per lane per tensor per step
-  constexpr int kMinSteps = kMinRangeTokens / STEP;
-  __shared__ int s_cum[kMaxSeqsPerLaunch + 1];
-  __shared__ int s_part[kDecodeThreads];
-  // fused scratch, per wave: norm weights; q inputs and new-token inputs, one region of
-  // each per copy of the unrolled step loop (see the fused helpers)
+// The state of (b, kvh) for this range: the parts of each head summed, then the bf16
+// output when one range covers the sequence, otherwise an fp32 partial.
+template <int G>
+__device__ __forceinline__ void emit_state(const DecodeParams& p, int b, int kvh, int slot, bool single, bool bad,
+                                          int n, int q4, const State<G>& st) {
+  float l = xor32_sum(xor16_sum(st.l));
+  if (bad) l = NAN;
+  float o[8][4];
+  bool nan = false;
+#pragma unroll
+  for (int mt = 0; mt < 8; ++mt) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = st.acc[mt][j];
+      o[mt][j] = a + row_up<G>(a);
+      if (G <= 5) o[mt][j] += row_up<2 * (G <= 5 ? G : 1)>(a);
+      else o[mt][j] += row_up<G>(st.acc2[mt][j]);
+      nan |= o[mt][j] != o[mt][j];
+    }
+  }
+  if (__any(nan)) {  // an infinite value in V: the first part has the result, the others inf - inf
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[mt][j] = __builtin_isfinite(st.acc[mt][j]) ? o[mt][j] : st.acc[mt][j];
+  }
+  const int h = kvh * G + n;
+  if (single) {
+    const float inv = 1.f / l;
+    uint16_t* out = p.out + b * p.o_seq_stride + h * p.o_head_stride + 4 * q4;
+    if (n < G)
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+        *reinterpret_cast<uint2*>(out + 16 * mt) =
+            make_uint2(pack_bf16x2(o[mt][0] * inv, o[mt][1] * inv), pack_bf16x2(o[mt][2] * inv, o[mt][3] * inv));
+  } else if (n < G) {
+    const int64_t row = static_cast<int64_t>(slot) * p.num_q_heads + h;
+    float* part = p.part_o + row * kDecodeHeadDim + 4 * q4;
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt)
+      *reinterpret_cast<float4*>(part + 16 * mt) = make_float4(o[mt][0], o[mt][1], o[mt][2], o[mt][3]);
+    if (q4 == 0) *reinterpret_cast<float2*>(p.part_ml + row * 2) = make_float2(st.m, l);
+  }
+}
+
+template <int G, bool FUSED>
+__global__ __launch_bounds__(kDecodeThreads)
+void paged_decode_kernel(const DecodeParams p) {
+  constexpr int kMinSteps = kMinRangeTokens / kStep;
+  // per wave: K and V tiles of the steps of either parity
+  __shared__ __attribute__((aligned(16))) char s_tile[kDecodeWaves][2][2 * kTileBytes];
+  // per wave: q heads of the next sequence (FUSED: behind its cos/sin row); FUSED: norm
+  // weights, and cos/sin row, raw k and raw v of the new token
+  constexpr int kQRow = FUSED ? kFzRow : 0;
   constexpr int kFzWaves = FUSED ? kDecodeWaves : 1;
-  __shared__ __attribute__((aligned(16))) char s_fw[kFzWaves][1024];
-  __shared__ __attribute__((aligned(16))) char s_fq0[kFzWaves][FUSED ? FzSize<G>::kBytes : 16];
-  __shared__ __attribute__((aligned(16))) char s_fq1[kFzWaves][FUSED ? FzSize<G>::kBytes : 16];
-  __shared__ __attribute__((aligned(16))) char s_fn0[kFzWaves][FUSED ? kFzNew : 16];
-  __shared__ __attribute__((aligned(16))) char s_fn1[kFzWaves][FUSED ? kFzNew : 16];
+  __shared__ __attribute__((aligned(16))) char s_fq[kDecodeWaves][kQRow + 256 * G];
+  __shared__ __attribute__((aligned(16))) char s_fw[kFzWaves][FUSED ? 512 : 16];
+  __shared__ __attribute__((aligned(16))) char s_fn[kFzWaves][FUSED ? kFzNew : 16];
+  __shared__ int s_cum[kSeqsPerLaunch + 1];  // steps of sequences 0 .. b - 1
+  __shared__ int s_ctx[kSeqsPerLaunch];
+  __shared__ int s_part[kDecodeWaves];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
-  const int r = lane >> 4;
-  const int c = lane & 15;
+  const int n = lane & 15, q4 = lane >> 4;
 
-  build_step_prefix(p, s_cum, s_part);
+  build_step_prefix(p, s_cum, s_ctx, s_part);
   const int B = p.num_seqs;
   const int total_steps = s_cum[B];
-  const int groups_per_range = (p.num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
-  const int num_ranges = max(1, static_cast<int>(gridDim.x) / groups_per_range);
-  const int spr = max(kMinSteps, (total_steps + num_ranges - 1) / num_ranges);
-  if (blockIdx.x == 0) {  // for the merge kernel
+  const int spr = max(kMinSteps, div_by(total_steps + static_cast<int>(gridDim.y) - 1, p.div_ranges));
+  if (blockIdx.x == 0 && blockIdx.y == 0) {  // for the merge kernel
     if (tid == 0) p.header[0] = spr;
     for (int b = tid; b <= B; b += kDecodeThreads) p.header[kHeaderInts + b] = s_cum[b];
   }
-
-  const int range = blockIdx.x / groups_per_range;
-  const int kvh = (blockIdx.x - range * groups_per_range) * kDecodeWaves + wave;
+  const int range = blockIdx.y;  // workgroup x of a range: kv heads 4 x .. 4 x + 3
+  const int kvh = blockIdx.x * kDecodeWaves + wave;
   const int S0 = range * spr;
   const int S1 = min(total_steps, S0 + spr);
   if (kvh >= p.num_kv_heads || S0 >= S1) return;  // no barrier follows
@@ -490,164 +547,234 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_decode_kernel(const Deco
     if (s_cum[mid] <= S0) lo = mid;
     else hi = mid;
   }
-  StepCursor cur;
-  lo = __builtin_amdgcn_readfirstlane(lo);  // uniform: the cursor's loads stay scalar
-  cursor_start_seq(p, cur, lo, __builtin_amdgcn_readfirstlane(S0 - s_cum[lo]));
-  const int64_t head_off = static_cast<int64_t>(kvh) * p.head_stride + 8 * c;
-
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  const int64_t head_off = static_cast<int64_t>(kvh) * p.head_stride;
   const int fw = FUSED ? wave : 0;
-  // The next sequence after the one whose steps end at step S (S < S1 - 1): the first
-  // sequence with steps starting at S + 1.
-  auto seq_after = [&](int b, int S) {
+  const int hg = n % G;     // this column's head and the part of P it holds
+  const int part = n / G;
+
+  TileLane ln;
+  ln.r = q4;
+  ln.c = n;
+  ln.row_off = q4 * static_cast<int>(p.rows_by_dma ? p.slot_stride : 0) * 2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ln.k_chunk[i] = 16 * (n ^ (4 * i + q4));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) ln.v_chunk[i] = 16 * (n ^ (2 * ((4 * i + q4) & 7)));
+  // LDS addresses of the lane's operands in a tile at address 0 (see the swizzles)
+  u32 ka[4], va[8];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) ka[kk] = 256 * n + 16 * ((4 * kk + q4) ^ n);
+  const int vrow = 4 * q4 + (n >> 2);
+#pragma unroll
+  for (int mt = 0; mt < 8; ++mt) va[mt] = kTileBytes + 256 * vrow + 8 * (n & 3) + 32 * (mt ^ (vrow & 7));
+
+  auto seq_after = [&](int b, int S) {  // the first sequence with steps starting at S + 1
     int nb = b + 1;
     while (s_cum[nb + 1] == S + 1) ++nb;
     return __builtin_amdgcn_readfirstlane(nb);
   };
-  uint4 qv[G];
-  if (FUSED) {
-    // q of the first sequence (waited for here, once per wave), and, if step S0 ends it,
-    // its new token and the next sequence's q for copy 0 of the step loop
-    fz_issue_weights(p, lane, s_fw[fw]);
-    fz_issue_q<G>(p, cur.b, cur.ctx, kvh, lane, s_fq1[fw]);
-    if (cur.j + 1 == cur.nsteps) {
-      fz_issue_new(p, cur.b, cur.ctx, kvh, lane, s_fn0[fw]);
-      if (S0 + 1 < S1) {
-        const int nb = seq_after(cur.b, S0);
-        fz_issue_q<G>(p, nb, load_uniform(p.context_lens, nb), kvh, lane, s_fq0[fw]);
-      }
-    }
-    wait_vmem<0>();
-    fz_finish_q<G>(p, cur.ctx, c, s_fq1[fw], s_fw[fw], qv);
-  } else {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-      qv[g] = load16(p.q + cur.b * p.q_seq_stride + (kvh * G + g) * p.q_head_stride + 8 * c);
-  }
-  float m[G], l[G], acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = kMaxFloor;
-    l[g] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-  }
 
-  // Tokens a step's loads may touch: with FUSED, a sequence's final step holds the token
-  // this launch appends, whose slot is not written yet; its rows are clamped onto the
-  // last cached token instead (a step with only the new token loads that slot but is
-  // never computed).
-  auto fused_load_count = [](const StepCursor& s, int nv) { return s.j + 1 == s.nsteps && nv > 1 ? nv - 1 : nv; };
-  uint4 kA[NL], vA[NL], kB[NL], vB[NL];
-  int nvA, nvB = 0;
-  if constexpr (FUSED) {
-    const int64_t base = step_base<STEP>(p, cur, head_off, nvA);
-    step_load<NL>(p, base, fused_load_count(cur, nvA), r, kA, vA);
-  } else {
-    step_load<NL>(p, step_base<STEP>(p, cur, head_off, nvA), nvA, r, kA, vA);
-  }
-
-  // One step: prefetch the next step into (kN, vN), compute (kC, vC), emit at the end
-  // of a sequence or of the range.  Returns false when the range is done.
-  // Compute of the step held in (kC, vC), the fused new token at a sequence end, the emit
-  // at the end of a sequence or of the range, and with MORE the switch to the next
-  // sequence's q.  The last step of a range gets its own instance: where the path that
-  // prefetched the next step met the one that did not, the compiler would keep the
-  // smaller wait count of the two and stall on the prefetch.
-  auto finish = [&](const uint4 (&kC)[NL], const uint4 (&vC)[NL], int nvC, bool seq_end, const StepCursor& nxt,
-                    const uint4 (&qn)[G], char* fq_mine, char* fn_mine, auto more_c) {
-    constexpr bool MORE = decltype(more_c)::value;
-    // Fused: the sequence's last token is not read from the cache (it is appended by this
-    // launch) but folded in from the qkv row after the step.  The step's loads were
-    // clamped onto the last cached token (fused_load_count), so no row holds the
-    // unwritten slot; a final step with no cached token is not computed at all.
+  // q of a sequence reaches the wave's region one step ahead, then the B layout (column n is
+  // head hg, dims 32 kk + 8 q4 + e).  FUSED: the raw heads are normalised and rotated in
+  // place first (row group r takes heads r, r + 4).
+  auto issue_q = [&](int b, int ctx) {
     if constexpr (FUSED) {
-      if (!(seq_end && nvC == 1)) step_compute<G, NL>(p, qv, kC, vC, seq_end ? nvC - 1 : nvC, r, m, l, acc);
+      fz_issue_q<G>(p, b, ctx, kvh, lane, s_fq[wave]);
     } else {
-      step_compute<G, NL>(p, qv, kC, vC, nvC, r, m, l, acc);
+      const uint16_t* src = p.q + b * p.q_seq_stride + static_cast<int64_t>(kvh) * G * p.q_head_stride;
+#pragma unroll
+      for (int u = 0; u < (G + 3) / 4; ++u) {
+        const int g = q4 + 4 * u;
+        if (p.q_by_dma) {  // uniform
+          const int head_bytes = static_cast<int>(p.q_head_stride) * 2;
+          const BufferRsrc rsrc = buffer_rsrc(src, static_cast<uint32_t>((G - 1) * head_bytes + 256));
+          if (g < G) lds_dma16(rsrc, g * head_bytes + 16 * n, s_fq[wave] + 1024 * u);
+        } else if (g < G) {
+          write_tile16(lds_addr(s_fq[wave]) + 256 * g + 16 * n, load16(src + g * p.q_head_stride + 8 * n));
+        }
+      }
     }
-    if (FUSED && seq_end) {
-      // this sequence's new-token region and, with MORE, the next one's q region were
-      // filled before the K/V loads of the next step
-      if (MORE) wait_vmem<2 * NL>();
+  };
+  const u32 q_at = lds_addr(s_fq[wave]), w_at = lds_addr(s_fw[fw]), new_at = lds_addr(s_fn[fw]);
+  auto finish_q = [&](int ctx, u32x4_t (&dst)[4]) {
+    if constexpr (FUSED) {
+      const bool pos_ok = ctx - 1 >= 0 && ctx - 1 < p.max_position;
+      const int g0 = min(q4, G - 1), g1 = min(q4 + 4, G - 1);
+      const u32 x0_at = q_at + kQRow + 256 * g0 + 16 * n, x1_at = q_at + kQRow + 256 * g1 + 16 * n;
+      const HeadInputs h = read_head(w_at + 16 * n, q_at + 32 * (n & 7), x0_at, x1_at);
+      const uint4 y0 = norm_rope_chunk(h, h.x0, n, pos_ok, p.eps);
+      if (q4 < G) write_tile16(x0_at, y0);
+      if (G > 4) {
+        const uint4 y1 = norm_rope_chunk(h, h.x1, n, pos_ok, p.eps);
+        if (q4 + 4 < G) write_tile16(x1_at, y1);
+      }
+    }
+    read_q(q_at + kQRow + 256 * hg + 16 * q4, dst);
+  };
+  // FUSED: the new token of the sequence that ends at this step: k normalised and rotated,
+  // both rows appended at the slot and put into the step's tiles, where the loads left them
+  // out; the rows past it are cleared, so that no unwritten slot is multiplied.
+  auto finish_new = [&](const StepCursor& c, int nv, u32 tile) {
+    const bool pos_ok = c.ctx - 1 >= 0 && c.ctx - 1 < p.max_position;
+    const int slot = load_uniform(p.slot_mapping, c.b);
+    const HeadInputs h =
+        read_head(w_at + 256 + 16 * n, new_at + 32 * (n & 7), new_at + kFzRow + 16 * n, new_at + kFzRow + 256 + 16 * n);
+    const uint4 knew = norm_rope_chunk(h, h.x0, n, pos_ok, p.eps);
+    const uint4 vnew = __builtin_bit_cast(uint4, h.x1);
+    if (q4 == 0 && slot >= 0 && slot < p.num_cache_slots) {
+      const int blk = slot / p.block_size, off = slot - blk * p.block_size;
+      const int64_t at = static_cast<int64_t>(blk) * p.blk_stride + static_cast<int64_t>(off) * p.slot_stride +
+                         head_off + 8 * n;
+      *reinterpret_cast<uint4*>(const_cast<uint16_t*>(p.k_cache) + at) = knew;
+      *reinterpret_cast<uint4*>(const_cast<uint16_t*>(p.v_cache) + at) = vnew;
+    }
+#pragma unroll 1
+    for (int row = q4; row < kStep; row += 4) {
+      if (row < nv - 1) continue;
+      const uint4 zero = make_uint4(0, 0, 0, 0);
+      write_tile16(tile + 256 * row + 16 * (n ^ (row & 15)), row == nv - 1 ? knew : zero);
+      write_tile16(tile + kTileBytes + 256 * row + 16 * (n ^ (2 * (row & 7))), row == nv - 1 ? vnew : zero);
+    }
+    wait_lds();
+  };
+
+  // The loop.  Iteration S computes step S and issues the tiles of step S + 2; the first two
+  // iterations (S < S0) only issue.  c0, c1, c2: cursors of steps S, S + 1, S + 2.  Loads
+  // complete in issue order, which is, per iteration: what the sequence end at step S + 1
+  // needs (q of the sequence after it, FUSED its new token), K of S + 2, V of S + 2; the
+  // first sequence's q goes before the tiles of S0.  The waits count from that order; other
+  // operations in flight (stores) only make them stricter.
+  StepCursor c0{}, c1{}, c2{};
+  int nv0 = 0, nv1 = 0, nv2 = 0;
+  u32x4_t qv[4] = {}, qn[4] = {};
+  State<G> st;
+  reset_state<G>(st);
+  if (FUSED) fz_issue_weights(p, lane, s_fw[fw]);
+  const u32 tile_base = lds_addr(s_tile[wave][0]);
+  for (int S = S0 - 2; S < S1; ++S) {
+    const int par = (S - S0) & 1;
+    const u32 tile = tile_base + 2 * kTileBytes * par;
+    const bool live = S >= S0, has1 = S + 1 >= S0 && S + 1 < S1, has2 = S + 2 < S1;
+    const bool seq_end = live && c0.j + 1 == c0.nsteps;
+    const bool end1 = has1 && c1.j + 1 == c1.nsteps;  // a sequence ends at S + 1
+    const bool new_q = has1 && (!live || seq_end);    // S + 1 starts with another q
+    if (seq_end || new_q) {
+      if (has1) wait_vmem<16>();  // all but the tiles of S + 1
       else wait_vmem<0>();
-      fz_finish_new<G>(p, cur.b, cur.ctx, kvh, r, c, fn_mine, s_fw[fw], qv, m, l, acc);
-    }
-    if (!MORE || seq_end) {
-      const int cb = s_cum[cur.b], cb1 = s_cum[cur.b + 1];
-      const int np = num_parts(cb, cb1, spr);
-      emit_state<G>(p, cur.b, kvh, range + cur.b, np == 1, cur.bad, lane, m, l, acc);
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        m[g] = kMaxFloor;
-        l[g] = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-      }
-      if (MORE) {
-        if (FUSED) {
-          fz_finish_q<G>(p, nxt.ctx, c, fq_mine, s_fw[fw], qv);
-        } else {
-#pragma unroll
-          for (int g = 0; g < G; ++g) qv[g] = qn[g];
-        }
-      }
-    }
-  };
-
-  // One step: prefetch the next step into (kN, vN), then finish this one.  Returns false
-  // when the range is done.
-  auto advance = [&](uint4 (&kC)[NL], uint4 (&vC)[NL], int nvC,
-                     uint4 (&kN)[NL], uint4 (&vN)[NL], int& nvN, int S, auto copy) -> bool {
-    constexpr int X = decltype(copy)::value;  // this copy of the step loop (0 or 1)
-    char* fq_mine = X == 0 ? s_fq0[fw] : s_fq1[fw];
-    char* fn_mine = X == 0 ? s_fn0[fw] : s_fn1[fw];
-    char* fq_other = X == 0 ? s_fq1[fw] : s_fq0[fw];
-    char* fn_other = X == 0 ? s_fn1[fw] : s_fn0[fw];
-    const bool seq_end = cur.j + 1 == cur.nsteps;
-    if (S + 1 < S1) {
-      StepCursor nxt = cur;
-      uint4 qn[G];
-      if (seq_end) {
-        // next non-empty sequence: the one whose steps start at S + 1
-        const int nb = seq_after(cur.b, S);
-        cursor_start_seq(p, nxt, nb, 0);
-        if (!FUSED) {
-#pragma unroll
-          for (int g = 0; g < G; ++g)
-            qn[g] = load16(p.q + nb * p.q_seq_stride + (kvh * G + g) * p.q_head_stride + 8 * c);
-        }
-      } else {
-        nxt.j = cur.j + 1;
-      }
       if constexpr (FUSED) {
-        const int64_t base = step_base<STEP>(p, nxt, head_off, nvN);
-        step_load<NL>(p, base, fused_load_count(nxt, nvN), r, kN, vN);
-      } else {
-        step_load<NL>(p, step_base<STEP>(p, nxt, head_off, nvN), nvN, r, kN, vN);
+        if (seq_end) finish_new(c0, nv0, tile);
       }
-      if (FUSED && nxt.j + 1 == nxt.nsteps) {
-        // step S + 1 (the other copy) ends sequence nxt.b: its new token, and the q of the
-        // sequence after it, for that copy
-        fz_issue_new(p, nxt.b, nxt.ctx, kvh, lane, fn_other);
-        if (S + 2 < S1) {
-          const int nb2 = seq_after(nxt.b, S + 1);
-          fz_issue_q<G>(p, nb2, load_uniform(p.context_lens, nb2), kvh, lane, fq_other);
+      if (new_q) finish_q(c1.ctx, qn);
+    } else if (live) {
+      if (has1) wait_vmem<24>();  // all but this step's V and the tiles of S + 1
+      else wait_vmem<8>();
+    }
+    if (end1) {
+      if (FUSED && live) fz_issue_new(p, c1.b, c1.ctx, kvh, lane, s_fn[fw]);
+      if (has2) {
+        const int nb = seq_after(c1.b, S + 1);
+        issue_q(nb, FUSED ? __builtin_amdgcn_readfirstlane(s_ctx[nb]) : 0);
+      }
+    }
+
+    // ---- scores
+    mfma_f32x4_t s[2] = {mfma_f32x4_t{0.f, 0.f, 0.f, 0.f}, mfma_f32x4_t{0.f, 0.f, 0.f, 0.f}};
+    if (live) {
+      u32x4_t k[8];
+      const u32 at[4] = {tile + ka[0], tile + ka[1], tile + ka[2], tile + ka[3]};
+      read_k_tile(at, k);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i & 1] = mfma16(k[i], qv[i >> 1], s[i & 1]);
+    }
+    int64_t base2 = 0;
+    int rows2 = 0;
+    if (has2) {  // K has been read: its tile takes step S + 2
+      if (S + 2 == S0) {
+        cursor_start_seq(c2, s_cum, s_ctx, lo, S0);
+        issue_q(c2.b, c2.ctx);
+        if (FUSED && c2.j + 1 == c2.nsteps) fz_issue_new(p, c2.b, c2.ctx, kvh, lane, s_fn[fw]);
+      } else if (c1.j + 1 == c1.nsteps) {
+        cursor_start_seq(c2, s_cum, s_ctx, seq_after(c1.b, S + 1), S + 2);
+      } else {
+        c2 = c1;
+        c2.j = c1.j + 1;
+      }
+      base2 = step_base(p, c2, head_off, nv2);
+      // FUSED: a sequence's final step holds the token this launch appends, whose slot is
+      // not written yet; its row is filled by finish_new
+      rows2 = FUSED && c2.j + 1 == c2.nsteps && nv2 > 1 ? nv2 - 1 : nv2;
+      issue_tile<false>(p, ln, base2, rows2, s_tile[wave][par]);
+    }
+    u32 pk[4] = {}, pk2[4] = {};
+    if (live) {
+      // ---- online softmax of the lane's 8 tokens and, over the row groups, all 32
+      float sc[8], mx = kMaxFloor;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = s[e >> 2][e & 3] * p.scale_log2;
+        sc[e] = 16 * (e >> 2) + 4 * q4 + (e & 3) < nv0 ? x : -INFINITY;
+        mx = fmaxf(mx, sc[e]);
+      }
+      mx = xor32_max(xor16_max(mx));
+      const float m_new = fmaxf(st.m, mx);
+      const float alpha = fast_exp2(st.m - m_new);
+      st.m = m_new;
+      if (__any(alpha != 1.f)) {
+        st.l *= alpha;
+#pragma unroll
+        for (int mt = 0; mt < 8; ++mt) {
+          st.acc[mt] *= alpha;
+          if (G > 5) st.acc2[mt] *= alpha;
         }
       }
-      finish(kC, vC, nvC, seq_end, nxt, qn, fq_mine, fn_mine, std::true_type{});
-      cur = nxt;
-      return true;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        float v[2], w[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const float p0 = fast_exp2(sc[e + i] - m_new);
+          st.l += p0;
+          const float r1 = p0 - round_bf16(p0);
+          const float r2 = r1 - round_bf16(r1);
+          v[i] = part == 0 ? p0 : (part == 1 ? r1 : r2);
+          w[i] = r2;
+        }
+        pk[e >> 1] = pack_bf16x2(v[0], v[1]);
+        if (G > 5) pk2[e >> 1] = pack_bf16x2(w[0], w[1]);
+      }
+      // ---- O^T += V^T P^T
+      if (has2) wait_vmem<24>();  // all but the tiles of S + 1 and the K tile of S + 2
+      else if (has1) wait_vmem<16>();
+      else wait_vmem<0>();
+      u32x2_t vlo[8], vhi[8];
+      const u32 at[8] = {tile + va[0], tile + va[1], tile + va[2], tile + va[3],
+                         tile + va[4], tile + va[5], tile + va[6], tile + va[7]};
+      read_v_tile(at, vlo, vhi);
+      const u32x4_t pf = {pk[0], pk[1], pk[2], pk[3]}, pf2 = {pk2[0], pk2[1], pk2[2], pk2[3]};
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt) {
+        const u32x4_t vt = {vlo[mt].x, vlo[mt].y, vhi[mt].x, vhi[mt].y};
+        st.acc[mt] = mfma16(vt, pf, st.acc[mt]);
+        if (G > 5) st.acc2[mt] = mfma16(vt, pf2, st.acc2[mt]);
+      }
     }
-    finish(kC, vC, nvC, seq_end, cur, qv, fq_mine, fn_mine, std::false_type{});
-    return false;
-  };
-
-  for (int S = S0;; S += 2) {
-    if (!advance(kA, vA, nvA, kB, vB, nvB, S, std::integral_constant<int, 0>{})) break;
-    if (!advance(kB, vB, nvB, kA, vA, nvA, S + 1, std::integral_constant<int, 1>{})) break;
+    if (has2) issue_tile<true>(p, ln, base2, rows2, s_tile[wave][par] + kTileBytes);
+    if (seq_end || (live && !has1)) {
+      // the whole sequence in this range: it ends here and began here
+      emit_state<G>(p, c0.b, kvh, range + c0.b, seq_end && S + 1 - c0.nsteps >= S0, c0.bad, n, q4, st);
+      reset_state<G>(st);
+    }
+    if (new_q) {
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) qv[kk] = qn[kk];
+    }
+    c0 = c1;
+    nv0 = nv1;
+    c1 = c2;
+    nv1 = nv2;
   }
 }
-
 // Combines the per-range partial states of sequences that span several ranges.
 // grid = (ceil(num_q_heads / 4), num_seqs), 128 threads: 4 query heads x 32 threads,
 // 4 output elements (16-byte partial rows) per thread.  A quarter of the waves of one
@@ -730,7 +857,7 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(const Decod
   *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(oo.x / ll, oo.y / ll), pack_bf16x2(oo.z / ll, oo.w / ll));
 }
 
-constexpr int64_t kHeaderBytes = ((kHeaderInts + kMaxSeqsPerLaunch + 1) * 4 + 255) / 256 * 256;
+constexpr int64_t kHeaderBytes = ((kHeaderInts + kHeaderSeqs + 1) * 4 + 255) / 256 * 256;
 constexpr int64_t kStateBytes = (kDecodeHeadDim + 2) * 4;  // one (acc[128], max, sum) state
 
 // Ranges of one launch: the grid's groups, and no more than minimum-size ranges over the
@@ -751,9 +878,9 @@ static int64_t decode_workspace_bound(int64_t seqs, int64_t q_heads, int64_t max
   return decode_workspace_need(seqs, q_heads, ranges);
 }
 
-// Workgroups of paged_decode_kernel<G, STEP, FUSED> resident on the whole current device
-// (cached per device once the queries succeed), capped at kMaxDecodeGrid.
-template <int G, int STEP, bool FUSED>
+// Workgroups of the kernel resident on the whole current device (cached per device once
+// the queries succeed), capped at kMaxDecodeGrid.
+template <int G, bool FUSED>
 static int resident_workgroups() {
   static std::atomic<int> cached[16];
   int dev = 0;
@@ -763,7 +890,7 @@ static int resident_workgroups() {
   int cus = 0, per_cu = 0;
   bool ok = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0;
   if (!ok) cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, paged_decode_kernel<G, STEP, FUSED>, kDecodeThreads, 0) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, paged_decode_kernel<G, FUSED>, kDecodeThreads, 0) !=
           hipSuccess || per_cu <= 0) {
     per_cu = 1;
     ok = false;
@@ -773,30 +900,29 @@ static int resident_workgroups() {
   return v;
 }
 
-template <int G, int STEP, bool FUSED>
+template <int G, bool FUSED>
 static int64_t decode_ranges(int num_kv_heads, int64_t max_tokens) {
   const int64_t groups_per_range = (num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
-  return std::max<int64_t>(1, std::min<int64_t>(resident_workgroups<G, STEP, FUSED>() / groups_per_range,
+  return std::max<int64_t>(1, std::min<int64_t>(resident_workgroups<G, FUSED>() / groups_per_range,
                                                 range_cap(max_tokens)));
 }
 
 template <bool FUSED>
 static int64_t decode_ranges_for(int G, int num_kv_heads, int64_t max_tokens) {
   switch (G) {
-    case 1: return decode_ranges<1, 32, FUSED>(num_kv_heads, max_tokens);
-    case 2: return decode_ranges<2, 32, FUSED>(num_kv_heads, max_tokens);
-    case 4: return decode_ranges<4, 32, FUSED>(num_kv_heads, max_tokens);
-    case 5: return decode_ranges<5, kG5Step, FUSED>(num_kv_heads, max_tokens);
-    default: return decode_ranges<8, kMinStepTokens, FUSED>(num_kv_heads, max_tokens);
+    case 1: return decode_ranges<1, FUSED>(num_kv_heads, max_tokens);
+    case 2: return decode_ranges<2, FUSED>(num_kv_heads, max_tokens);
+    case 4: return decode_ranges<4, FUSED>(num_kv_heads, max_tokens);
+    case 5: return decode_ranges<5, FUSED>(num_kv_heads, max_tokens);
+    default: return decode_ranges<8, FUSED>(num_kv_heads, max_tokens);
   }
 }
 
-template <int G, int STEP, bool FUSED>
+template <int G, bool FUSED>
 static void launch_decode(DecodeParams p, int64_t ranges, hipStream_t s) {
   const int64_t groups_per_range = (p.num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
-  p.step_tokens = STEP;
-  hipLaunchKernelGGL((paged_decode_kernel<G, STEP, FUSED>), dim3(static_cast<unsigned>(ranges * groups_per_range)),
-                     dim3(kDecodeThreads), 0, s, p);
+  p.div_ranges = divisor(static_cast<uint32_t>(ranges));
+  hipLaunchKernelGGL((paged_decode_kernel<G, FUSED>), dim3(static_cast<unsigned>(groups_per_range), static_cast<unsigned>(ranges)), dim3(kDecodeThreads), 0, s, p);
   hipLaunchKernelGGL(decode_merge_kernel, dim3((p.num_q_heads + kMergeHeads - 1) / kMergeHeads, p.num_seqs),
                      dim3(kMergeThreads), 0, s, p);
 }
@@ -854,14 +980,14 @@ static int check_decode_args(const char* fn, const DecodeArgs& a) {
 
 // Enqueues the decode of a checked batch on `s` with `ws` as workspace (ws_bytes must
 // cover decode_workspace_need of every launch; checked by the callers).  Batches beyond
-// the LDS prefix table run as consecutive launches of up to 4096 sequences; they reuse
+// the LDS prefix table run as consecutive launches of up to 1024 sequences; they reuse
 // the workspace in stream order.
 template <bool FUSED>
 static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, char* ws, hipStream_t s,
                           const DecodeParams* fused = nullptr) {
   const int G = a.num_q_heads / a.num_kv_heads;
-  for (int b0 = 0; b0 < a.num_seqs; b0 += kMaxSeqsPerLaunch) {
-    const int nb = std::min(kMaxSeqsPerLaunch, a.num_seqs - b0);
+  for (int b0 = 0; b0 < a.num_seqs; b0 += kSeqsPerLaunch) {
+    const int nb = std::min(kSeqsPerLaunch, a.num_seqs - b0);
     DecodeParams p = fused ? *fused : DecodeParams{};
     if (FUSED) {  // this chunk's rows of the per-sequence inputs
       p.qkv += b0 * p.qkv_stride;
@@ -875,6 +1001,8 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, c
     p.blk_stride = a.cache_block_stride;
     p.slot_stride = a.cache_slot_stride;
     p.head_stride = a.cache_head_stride;
+    p.rows_by_dma = a.cache_slot_stride >= 0 && a.cache_slot_stride <= kMaxDmaRow;
+    p.q_by_dma = a.q_head_stride >= 0 && a.q_head_stride <= kMaxDmaRow;
     p.num_cache_blocks = a.num_cache_blocks;
     p.block_tables = a.block_tables + b0 * a.block_table_stride;
     p.bt_stride = a.block_table_stride;
@@ -884,6 +1012,7 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, c
     p.num_kv_heads = a.num_kv_heads;
     p.block_size = a.block_size;
     p.max_blocks = a.max_blocks_per_seq;
+    p.div_block = divisor(static_cast<uint32_t>(a.block_size));
     p.scale_log2 = a.softmax_scale * 1.4426950408889634f;
     p.out = static_cast<uint16_t*>(a.out) + b0 * a.out_seq_stride;
     p.o_seq_stride = a.out_seq_stride;
@@ -892,11 +1021,11 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, c
     p.part_o = reinterpret_cast<float*>(ws + kHeaderBytes);
     p.part_ml = p.part_o + static_cast<size_t>(ranges + nb) * a.num_q_heads * kDecodeHeadDim;
     switch (G) {
-      case 1: launch_decode<1, 32, FUSED>(p, ranges, s); break;
-      case 2: launch_decode<2, 32, FUSED>(p, ranges, s); break;
-      case 4: launch_decode<4, 32, FUSED>(p, ranges, s); break;
-      case 5: launch_decode<5, kG5Step, FUSED>(p, ranges, s); break;
-      default: launch_decode<8, kMinStepTokens, FUSED>(p, ranges, s); break;
+      case 1: launch_decode<1, FUSED>(p, ranges, s); break;
+      case 2: launch_decode<2, FUSED>(p, ranges, s); break;
+      case 4: launch_decode<4, FUSED>(p, ranges, s); break;
+      case 5: launch_decode<5, FUSED>(p, ranges, s); break;
+      default: launch_decode<8, FUSED>(p, ranges, s); break;
     }
     const int rc = launch_status(fn);
     if (rc != KVP_OK) return rc;
@@ -907,7 +1036,7 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, c
 // Launch ranges for the batch's first (largest) launch.
 template <bool FUSED = false>
 static int64_t batch_ranges(const DecodeArgs& a) {
-  const int nb = std::min(a.num_seqs, kMaxSeqsPerLaunch);
+  const int nb = std::min(a.num_seqs, kSeqsPerLaunch);
   const int64_t max_tokens = static_cast<int64_t>(nb) * a.max_blocks_per_seq * a.block_size;
   return decode_ranges_for<FUSED>(a.num_q_heads / a.num_kv_heads, a.num_kv_heads, max_tokens);
 }
@@ -962,7 +1091,7 @@ extern "C" size_t kvp_decode_workspace_bytes(int32_t max_num_seqs, int32_t num_q
   if (max_num_seqs <= 0 || num_q_heads <= 0 || head_dim != kDecodeHeadDim || max_blocks_per_seq <= 0 ||
       block_size <= 0)
     return 0;
-  const int64_t seqs = std::min<int64_t>(max_num_seqs, kMaxSeqsPerLaunch);
+  const int64_t seqs = std::min<int64_t>(max_num_seqs, kHeaderSeqs);
   return static_cast<size_t>(decode_workspace_bound(seqs, num_q_heads, max_blocks_per_seq, block_size));
 }
 
@@ -987,7 +1116,7 @@ extern "C" int kvp_paged_decode_bf16(const void* q, int64_t q_seq_stride, int64_
   int rc = check_decode_args(fn, a);
   if (rc != KVP_OK) return rc;
   if (num_seqs == 0) return KVP_OK;
-  const int chunk_seqs = std::min(num_seqs, kMaxSeqsPerLaunch);
+  const int chunk_seqs = std::min(num_seqs, kHeaderSeqs);
   const size_t need =
       static_cast<size_t>(decode_workspace_bound(chunk_seqs, num_q_heads, max_blocks_per_seq, block_size));
   if (!workspace || workspace_bytes < need)
@@ -1020,12 +1149,12 @@ extern "C" int kvp_paged_decode_bf16_noalloc(const void* q, int64_t q_seq_stride
   if (rc != KVP_OK) return rc;
   if (num_seqs == 0) return KVP_OK;
   const int64_t ranges = batch_ranges(a);
-  const int64_t need = decode_workspace_need(std::min(num_seqs, kMaxSeqsPerLaunch), num_q_heads, ranges);
+  const int64_t need = decode_workspace_need(std::min(num_seqs, kHeaderSeqs), num_q_heads, ranges);
   if (need > static_cast<int64_t>(kScratchBytes))
     return fail(KVP_EWORKSPACE,
                 "%s: %d sequences x %d query heads need %lld bytes of decode scratch; the static scratch "
                 "holds %zu (use kvp_paged_decode_bf16 with a caller workspace)",
-                fn, std::min(num_seqs, kMaxSeqsPerLaunch), num_q_heads, static_cast<long long>(need), kScratchBytes);
+                fn, std::min(num_seqs, kHeaderSeqs), num_q_heads, static_cast<long long>(need), kScratchBytes);
   char* ws = nullptr;
   rc = scratch_address(fn, static_cast<hipStream_t>(stream), &ws);
   if (rc != KVP_OK) return rc;
@@ -1063,7 +1192,7 @@ extern "C" int kvp_paged_decode_fused_bf16(
     return fail(KVP_EINVAL, "%s: qkv row stride %lld is shorter than (hq + 2 hkv) * head_dim", fn,
                 static_cast<long long>(qkv_tok_stride));
   if (num_seqs == 0) return KVP_OK;
-  const int chunk_seqs = std::min(num_seqs, kMaxSeqsPerLaunch);
+  const int chunk_seqs = std::min(num_seqs, kHeaderSeqs);
   // the kernel addresses the table and one launch's qkv rows with 32-bit byte offsets
   if (static_cast<int64_t>(max_position) * kRopeDim * 4 > INT32_MAX ||
       static_cast<int64_t>(chunk_seqs) * qkv_tok_stride * 2 > INT32_MAX)

@@ -1,0 +1,97 @@
+"""Paged decode at the edges of its work split and of its LDS tiles, against the fp32 oracle:
+contexts around the 32-token step and the 16-token half, pages whose size is not a power of
+two, more sequences than one launch's tables hold, row strides beyond 32-bit offsets, and
+values that a split of the softmax weights into parts could spoil (infinities in V).
+
+Tolerance (TOL, atol 2e-2): outputs are bf16 averages of N(0, 1) values, |o| < 4, whose
+rounding is at most 2^-7; the fp32 sums and the exact three-part weights add below 1e-4.
+"""
+
+import math
+
+import pytest
+import torch
+
+from oracle import kvpath_oracle as ref
+from tests.helpers import TOL, contiguous_caches, gen, random_block_tables, randn_bf16
+from tests.test_fused_decode import _case as fused_case, _fused, _separate
+from tests.test_paged_decode import SCALE, _check, _decode
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 191, 192, 193, 383, 385]
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("bs", [64, 192])
+def test_step_and_page_edges(cuda_device, G, bs):
+    g = gen(700 + G + bs)
+    hkv = 3 if G < 8 else 5  # waves past the last kv head, one and two head groups
+    nb = sum(math.ceil(c / bs) for c in EDGES) + 2
+    kc, vc = contiguous_caches(nb, bs, hkv, 128, g)
+    bt = random_block_tables(EDGES, bs, nb, g)
+    q = randn_bf16((len(EDGES), G * hkv, 128), g)
+    _check(cuda_device, q, kc, vc, bt, torch.tensor(EDGES, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 5, 8])
+def test_one_launch_step_at_the_edges(cuda_device, G):
+    """Append, q and attention of the one-launch step where the new token opens, fills or
+    closes a step, a page or a range."""
+    hkv, bs = 3, 64
+    host, d1 = fused_case(cuda_device, 800 + G, G * hkv, hkv, bs, EDGES, pad=2)
+    d2 = {k: v.clone() for k, v in d1.items()}
+    sep, one = _separate(d1, G * hkv, hkv, bs), _fused(d2, G * hkv, hkv, bs)
+    torch.cuda.synchronize()
+    assert torch.equal(d1["pool"].cpu(), d2["pool"].cpu())
+    torch.testing.assert_close(one.cpu().float(), sep.cpu().float(), **TOL)
+
+
+def test_more_sequences_than_one_launch(cuda_device):
+    B, hkv, bs = 1030, 2, 64
+    g = gen(9)
+    ctx = torch.randint(0, 90, (B,), generator=g, dtype=torch.int32)
+    nb = sum(math.ceil(int(c) / bs) for c in ctx) + 2
+    kc, vc = contiguous_caches(nb, bs, hkv, 128, g)
+    bt = random_block_tables([int(c) for c in ctx], bs, nb, g)
+    _check(cuda_device, randn_bf16((B, 4 * hkv, 128), g), kc, vc, bt, ctx)
+
+
+def test_strides_beyond_32_bit_offsets(cuda_device):
+    """Token rows and q heads further apart than 32 rows of 32-bit byte offsets reach: the
+    tiles are filled through registers and give the same bits."""
+    g, d = gen(10), cuda_device
+    hkv, G, bs, far = 1, 2, 64, (1 << 24) + 8
+    kc, vc = contiguous_caches(1, bs, hkv, 128, g)
+    q = randn_bf16((1, G, 128), g)
+    ctx, bt = torch.tensor([61], dtype=torch.int32), torch.zeros(1, 1, dtype=torch.int32)
+    near = _decode(q.to(d), kc.to(d), vc.to(d), ctx.to(d), bt.to(d))
+    big = [torch.empty(bs * far, dtype=torch.bfloat16, device=d).as_strided((1, bs, hkv, 128), (bs * far, far, 128, 1))
+           for _ in range(2)]
+    big[0].copy_(kc)
+    big[1].copy_(vc)
+    qf = torch.empty(G * far, dtype=torch.bfloat16, device=d).as_strided((1, G, 128), (G * far, far, 1))
+    qf.copy_(q)
+    out = _decode(qf, big[0], big[1], ctx.to(d), bt.to(d))
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), near.view(torch.int16))
+
+
+@pytest.mark.parametrize("G", [2, 5, 8])
+def test_infinite_values_stay_infinite(cuda_device, G):
+    """An infinity in V gives that infinity (a weight's lower parts times it are inf - inf),
+    and touches no other dim."""
+    g, d = gen(11), cuda_device
+    hkv, bs = 2, 64
+    ctx = torch.tensor([50, 40], dtype=torch.int32)
+    kc, vc = contiguous_caches(3, bs, hkv, 128, g)
+    vc[1, 20, 0, 5] = float("inf")
+    vc[1, 21, 1, 77] = float("-inf")
+    bt = torch.tensor([[1], [2]], dtype=torch.int32)
+    q = randn_bf16((2, G * hkv, 128), g)
+    out = _decode(q.to(d), kc.to(d), vc.to(d), ctx.to(d), bt.to(d)).cpu().float()
+    want = ref.paged_decode(q, kc, vc, bt, ctx, SCALE)
+    assert torch.equal(torch.isinf(out), torch.isinf(want)) and not torch.isnan(out).any()
+    assert torch.all(out[0, :G, 5] == float("inf")) and torch.all(out[0, G:, 77] == float("-inf"))
+    fin = torch.isfinite(want)
+    torch.testing.assert_close(out[fin], want[fin], **TOL)
