@@ -77,7 +77,13 @@ constexpr int kDecodeWaves = 4;  // kv heads per workgroup
 constexpr int kDecodeThreads = 64 * kDecodeWaves;
 constexpr int kStep = 32;               // tokens per step
 constexpr int kTileBytes = kStep * 256;  // one K or V tile
-constexpr int kMinRangeTokens = 128;  // a range covers at least 128 tokens
+// A range covers at least one step.  The workspace formula counts ranges of 128 tokens, so a
+// workspace of just that size may be too small for a narrow block table's one-step ranges;
+// then a range covers at least 128 tokens.  A small batch wants the shortest ranges, because
+// its waves run their steps one after the other while most CUs idle: per call, one sequence
+// of 611 tokens 15.0 us with 128-token ranges, 12.2 us with one-step ranges; 37 sequences of
+// 17-118 tokens 20.9 and 12.5 us.  A large batch is split by the grid and sees no difference.
+constexpr int kWorkspaceRangeTokens = 128;
 constexpr int kSeqsPerLaunch = 1024;  // sequences per launch (LDS tables); more run as consecutive launches
 constexpr int kHeaderSeqs = 4096;     // sequences the workspace formula counts at most
 constexpr int64_t kMaxDmaRow = 1 << 24;  // row stride (elements) up to which 32 rows are addressed in 32 bits
@@ -118,6 +124,7 @@ struct DecodeParams {
   int32_t num_kv_heads;
   int32_t block_size;
   int32_t max_blocks;
+  int32_t min_steps;  // least steps of a range
   float scale_log2;   // softmax_scale * log2(e)
   uint16_t* out;
   int64_t o_seq_stride, o_head_stride;
@@ -507,7 +514,6 @@ __device__ __forceinline__ void emit_state(const DecodeParams& p, int b, int kvh
 template <int G, bool FUSED>
 __global__ __launch_bounds__(kDecodeThreads)
 void paged_decode_kernel(const DecodeParams p) {
-  constexpr int kMinSteps = kMinRangeTokens / kStep;
   // per wave: K and V tiles of the steps of either parity
   __shared__ __attribute__((aligned(16))) char s_tile[kDecodeWaves][2][2 * kTileBytes];
   // per wave: q heads of the next sequence (FUSED: behind its cos/sin row); FUSED: norm
@@ -529,7 +535,7 @@ void paged_decode_kernel(const DecodeParams p) {
   build_step_prefix(p, s_cum, s_ctx, s_part);
   const int B = p.num_seqs;
   const int total_steps = s_cum[B];
-  const int spr = max(kMinSteps, div_by(total_steps + static_cast<int>(gridDim.y) - 1, p.div_ranges));
+  const int spr = max(p.min_steps, div_by(total_steps + static_cast<int>(gridDim.y) - 1, p.div_ranges));
   if (blockIdx.x == 0 && blockIdx.y == 0) {  // for the merge kernel
     if (tid == 0) p.header[0] = spr;
     for (int b = tid; b <= B; b += kDecodeThreads) p.header[kHeaderInts + b] = s_cum[b];
@@ -862,8 +868,8 @@ constexpr int64_t kStateBytes = (kDecodeHeadDim + 2) * 4;  // one (acc[128], max
 
 // Ranges of one launch: the grid's groups, and no more than minimum-size ranges over the
 // largest possible work (max_tokens = sequences * table width * block_size).
-static int64_t range_cap(int64_t max_tokens) {
-  return std::max<int64_t>(1, (max_tokens + kMinRangeTokens - 1) / kMinRangeTokens);
+static int64_t range_cap(int64_t max_tokens, int64_t range_tokens) {
+  return std::max<int64_t>(1, (max_tokens + range_tokens - 1) / range_tokens);
 }
 
 // Workspace bytes for a launch of `seqs` sequences over `ranges` ranges.
@@ -874,7 +880,7 @@ static int64_t decode_workspace_need(int64_t seqs, int64_t q_heads, int64_t rang
 // Workspace bytes that cover every launch of up to `seqs` sequences, on any device:
 // a launch has at most kMaxDecodeGrid ranges.
 static int64_t decode_workspace_bound(int64_t seqs, int64_t q_heads, int64_t max_blocks, int64_t block_size) {
-  const int64_t ranges = std::min<int64_t>(kMaxDecodeGrid, range_cap(seqs * max_blocks * block_size));
+  const int64_t ranges = std::min<int64_t>(kMaxDecodeGrid, range_cap(seqs * max_blocks * block_size, kWorkspaceRangeTokens));
   return decode_workspace_need(seqs, q_heads, ranges);
 }
 
@@ -900,21 +906,14 @@ static int resident_workgroups() {
   return v;
 }
 
-template <int G, bool FUSED>
-static int64_t decode_ranges(int num_kv_heads, int64_t max_tokens) {
-  const int64_t groups_per_range = (num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
-  return std::max<int64_t>(1, std::min<int64_t>(resident_workgroups<G, FUSED>() / groups_per_range,
-                                                range_cap(max_tokens)));
-}
-
 template <bool FUSED>
-static int64_t decode_ranges_for(int G, int num_kv_heads, int64_t max_tokens) {
+static int resident_for(int G) {
   switch (G) {
-    case 1: return decode_ranges<1, FUSED>(num_kv_heads, max_tokens);
-    case 2: return decode_ranges<2, FUSED>(num_kv_heads, max_tokens);
-    case 4: return decode_ranges<4, FUSED>(num_kv_heads, max_tokens);
-    case 5: return decode_ranges<5, FUSED>(num_kv_heads, max_tokens);
-    default: return decode_ranges<8, FUSED>(num_kv_heads, max_tokens);
+    case 1: return resident_workgroups<1, FUSED>();
+    case 2: return resident_workgroups<2, FUSED>();
+    case 4: return resident_workgroups<4, FUSED>();
+    case 5: return resident_workgroups<5, FUSED>();
+    default: return resident_workgroups<8, FUSED>();
   }
 }
 
@@ -922,7 +921,8 @@ template <int G, bool FUSED>
 static void launch_decode(DecodeParams p, int64_t ranges, hipStream_t s) {
   const int64_t groups_per_range = (p.num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
   p.div_ranges = divisor(static_cast<uint32_t>(ranges));
-  hipLaunchKernelGGL((paged_decode_kernel<G, FUSED>), dim3(static_cast<unsigned>(groups_per_range), static_cast<unsigned>(ranges)), dim3(kDecodeThreads), 0, s, p);
+  const dim3 grid(static_cast<unsigned>(groups_per_range), static_cast<unsigned>(ranges));
+  hipLaunchKernelGGL((paged_decode_kernel<G, FUSED>), grid, dim3(kDecodeThreads), 0, s, p);
   hipLaunchKernelGGL(decode_merge_kernel, dim3((p.num_q_heads + kMergeHeads - 1) / kMergeHeads, p.num_seqs),
                      dim3(kMergeThreads), 0, s, p);
 }
@@ -978,14 +978,32 @@ static int check_decode_args(const char* fn, const DecodeArgs& a) {
   return KVP_OK;
 }
 
+// How the batch is cut: the ranges of its first (largest) launch and the least steps of one.
+// One-step ranges where `capacity` bytes hold their states, else ranges of 128 tokens.
+struct Split {
+  int64_t ranges;
+  int min_steps;
+};
+template <bool FUSED = false>
+static Split batch_split(const DecodeArgs& a, int64_t capacity) {
+  const int nb = std::min(a.num_seqs, kSeqsPerLaunch);
+  const int64_t max_tokens = static_cast<int64_t>(nb) * a.max_blocks_per_seq * a.block_size;
+  const int64_t groups = (a.num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
+  const int64_t most = std::max<int64_t>(1, resident_for<FUSED>(a.num_q_heads / a.num_kv_heads) / groups);
+  const int64_t fine = std::min(most, range_cap(max_tokens, kStep));
+  if (decode_workspace_need(nb, a.num_q_heads, fine) <= capacity) return Split{fine, 1};
+  return Split{std::min(most, range_cap(max_tokens, kWorkspaceRangeTokens)), kWorkspaceRangeTokens / kStep};
+}
+
 // Enqueues the decode of a checked batch on `s` with `ws` as workspace (ws_bytes must
 // cover decode_workspace_need of every launch; checked by the callers).  Batches beyond
 // the LDS prefix table run as consecutive launches of up to 1024 sequences; they reuse
 // the workspace in stream order.
 template <bool FUSED>
-static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, char* ws, hipStream_t s,
+static int enqueue_decode(const char* fn, const DecodeArgs& a, const Split& split, char* ws, hipStream_t s,
                           const DecodeParams* fused = nullptr) {
   const int G = a.num_q_heads / a.num_kv_heads;
+  const int64_t ranges = split.ranges;
   for (int b0 = 0; b0 < a.num_seqs; b0 += kSeqsPerLaunch) {
     const int nb = std::min(kSeqsPerLaunch, a.num_seqs - b0);
     DecodeParams p = fused ? *fused : DecodeParams{};
@@ -1012,6 +1030,7 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, c
     p.num_kv_heads = a.num_kv_heads;
     p.block_size = a.block_size;
     p.max_blocks = a.max_blocks_per_seq;
+    p.min_steps = split.min_steps;
     p.div_block = divisor(static_cast<uint32_t>(a.block_size));
     p.scale_log2 = a.softmax_scale * 1.4426950408889634f;
     p.out = static_cast<uint16_t*>(a.out) + b0 * a.out_seq_stride;
@@ -1031,14 +1050,6 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, c
     if (rc != KVP_OK) return rc;
   }
   return KVP_OK;
-}
-
-// Launch ranges for the batch's first (largest) launch.
-template <bool FUSED = false>
-static int64_t batch_ranges(const DecodeArgs& a) {
-  const int nb = std::min(a.num_seqs, kSeqsPerLaunch);
-  const int64_t max_tokens = static_cast<int64_t>(nb) * a.max_blocks_per_seq * a.block_size;
-  return decode_ranges_for<FUSED>(a.num_q_heads / a.num_kv_heads, a.num_kv_heads, max_tokens);
 }
 
 // ---------------------------------------------------------------- no-allocation variant
@@ -1123,7 +1134,7 @@ extern "C" int kvp_paged_decode_bf16(const void* q, int64_t q_seq_stride, int64_
     return fail(KVP_EWORKSPACE, "%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, need);
   if (reinterpret_cast<uintptr_t>(workspace) & 255u)
     return fail(KVP_EINVAL, "%s: workspace must be 256-byte aligned", fn);
-  return enqueue_decode<false>(fn, a, batch_ranges(a), static_cast<char*>(workspace),
+  return enqueue_decode<false>(fn, a, batch_split(a, static_cast<int64_t>(workspace_bytes)), static_cast<char*>(workspace),
                                static_cast<hipStream_t>(stream));
 }
 
@@ -1148,8 +1159,11 @@ extern "C" int kvp_paged_decode_bf16_noalloc(const void* q, int64_t q_seq_stride
   int rc = check_decode_args(fn, a);
   if (rc != KVP_OK) return rc;
   if (num_seqs == 0) return KVP_OK;
-  const int64_t ranges = batch_ranges(a);
-  const int64_t need = decode_workspace_need(std::min(num_seqs, kHeaderSeqs), num_q_heads, ranges);
+  // cut as with a workspace of the formula's size, so that both entry points agree bit for bit
+  const int64_t formula =
+      decode_workspace_bound(std::min(num_seqs, kHeaderSeqs), num_q_heads, max_blocks_per_seq, block_size);
+  const Split split = batch_split(a, formula);
+  const int64_t need = decode_workspace_need(std::min(num_seqs, kHeaderSeqs), num_q_heads, split.ranges);
   if (need > static_cast<int64_t>(kScratchBytes))
     return fail(KVP_EWORKSPACE,
                 "%s: %d sequences x %d query heads need %lld bytes of decode scratch; the static scratch "
@@ -1158,7 +1172,7 @@ extern "C" int kvp_paged_decode_bf16_noalloc(const void* q, int64_t q_seq_stride
   char* ws = nullptr;
   rc = scratch_address(fn, static_cast<hipStream_t>(stream), &ws);
   if (rc != KVP_OK) return rc;
-  return enqueue_decode<false>(fn, a, ranges, ws, static_cast<hipStream_t>(stream));
+  return enqueue_decode<false>(fn, a, split, ws, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int kvp_paged_decode_fused_bf16(
@@ -1213,6 +1227,6 @@ extern "C" int kvp_paged_decode_fused_bf16(
   f.eps = eps;
   f.slot_mapping = slot_mapping;
   f.num_cache_slots = static_cast<int64_t>(num_cache_blocks) * block_size;
-  return enqueue_decode<true>(fn, a, batch_ranges<true>(a), static_cast<char*>(workspace),
+  return enqueue_decode<true>(fn, a, batch_split<true>(a, static_cast<int64_t>(workspace_bytes)), static_cast<char*>(workspace),
                               static_cast<hipStream_t>(stream), &f);
 }

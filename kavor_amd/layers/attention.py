@@ -104,8 +104,10 @@ def reserve_decode_workspace(max_num_seqs: int, num_q_heads: int, head_dim: int,
                              device: torch.device | str | int) -> torch.Tensor:
     """Allocates (or grows) the per-device decode workspace.  Call before graph capture
     with the largest batch a captured graph will use; an eager call that needs more grows
-    the workspace without freeing the one the graphs hold."""
-    nbytes = decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim, max_blocks_per_seq, block_size)
+    the workspace without freeing the one the graphs hold.  It holds the states of
+    one-step (32-token) ranges, four times as many as kvp_decode_workspace_bytes counts
+    for the same block table: a small batch runs faster in them."""
+    nbytes = decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim, 4 * max_blocks_per_seq, block_size)
     dev = torch.device(device) if not isinstance(device, int) else torch.device("cuda", device)
     if dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())

@@ -15,7 +15,7 @@ import torch
 from oracle import kvpath_oracle as ref
 from tests.helpers import TOL, contiguous_caches, gen, random_block_tables, randn_bf16
 from tests.test_fused_decode import _case as fused_case, _fused, _separate
-from tests.test_paged_decode import SCALE, _check, _decode
+from tests.test_paged_decode import SCALE, _case as decode_case, _check, _decode
 
 pytestmark = pytest.mark.gpu
 
@@ -32,6 +32,13 @@ def test_step_and_page_edges(cuda_device, G, bs):
     bt = random_block_tables(EDGES, bs, nb, g)
     q = randn_bf16((len(EDGES), G * hkv, 128), g)
     _check(cuda_device, q, kc, vc, bt, torch.tensor(EDGES, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("steps", [2, 4, 5, 19, 20, 21, 100])
+def test_one_sequence_in_many_ranges(cuda_device, steps):
+    """A lone sequence is cut into one-step ranges: its states merge in rounds of 4 and 16."""
+    q, kc, vc, bt, _ = decode_case(900 + steps, 1, 8, 2, 64, 32 * steps - 5, 32 * steps - 5)
+    _check(cuda_device, q, kc, vc, bt, torch.tensor([32 * steps - 5], dtype=torch.int32))
 
 
 @pytest.mark.parametrize("G", [1, 2, 4, 5, 8])
