@@ -782,25 +782,22 @@ void paged_decode_kernel(const DecodeParams p) {
   }
 }
 // Combines the per-range partial states of sequences that span several ranges.
-// grid = (ceil(num_q_heads / 4), num_seqs), 128 threads: 4 query heads x 32 threads,
-// 4 output elements (16-byte partial rows) per thread.  A quarter of the waves of one
-// thread per element: 175.0 -> 174.2 us per decode call on 256 sequences, and about
-// 1 us less for small batches.
-// The kernel is latency-bound: it reads the sequence's step span and the steps per range
-// from the header (one round trip), then its first kSpecParts slots together (a second
-// one: the slots are consecutive and start at slot first_b + b); rows past the part count
-// are clamped onto the last part and ignored.
+// grid = (ceil(num_q_heads / 4), num_seqs), one wave per query head: the four 16-lane rows
+// take the sequence's slots (consecutive, from first_b + b) round robin, 8 dims per lane,
+// and are merged across the wave at the end.
+// Latency-bound: the header words (one round trip), then one slot per row (a second one,
+// which ends it for up to 4 parts), then 16 slots per round trip, so that a sequence cut
+// into many short ranges does not wait for its slots a few at a time.  Against 32 lanes per
+// head with 4, then 8 slots per round trip (whole calls): 2 sequences of 3000-4000 tokens
+// (up to 62 parts) 21.7 -> 17.4 us, 8 of 600-3000 21.9 -> 20.6 us, one of 611 12.2 -> 11.2 us.
+// Rows past the part count are clamped onto the last part and ignored.
 constexpr int kMergeHeads = 4;
-constexpr int kSpecParts = 4;
-constexpr int kMergeThreads = kMergeHeads * kDecodeHeadDim / 4;  // 4 dims per thread
-__device__ __forceinline__ float4 fma4(float w, float4 o, float4 acc) {
-  return make_float4(acc.x + w * o.x, acc.y + w * o.y, acc.z + w * o.z, acc.w + w * o.w);
-}
+constexpr int kMergeThreads = 64 * kMergeHeads;
 __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(const DecodeParams p) {
   constexpr int D = kDecodeHeadDim;
-  const int h = blockIdx.x * kMergeHeads + static_cast<int>(threadIdx.x) / (D / 4);
+  const int h = blockIdx.x * kMergeHeads + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = blockIdx.y;
-  const int d = 4 * (threadIdx.x % (D / 4));
+  const int r = (threadIdx.x >> 4) & 3, d = 8 * (threadIdx.x & 15);
   if (h >= p.num_q_heads) return;
   const int cb = load_uniform(p.header, kHeaderInts + b), cb1 = load_uniform(p.header, kHeaderInts + b + 1);
   const int spr = load_uniform(p.header, 0);
@@ -811,56 +808,42 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(const Decod
   const int64_t hq = p.num_q_heads;  // rows between consecutive slots
   const float* ml = p.part_ml + row0 * 2;
   const float* po = p.part_o + row0 * D + d;
-  float2 st0[kSpecParts];
-  float4 ov0[kSpecParts];
+  float m = kMaxFloor, l = 0.f, o[8] = {};
+  auto add = [&](float2 s, float4 x, float4 y) {
+    const float m_new = fmaxf(m, s.x), alpha = fast_exp2(m - m_new), w = fast_exp2(s.x - m_new);
+    const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+    m = m_new;
+    l = l * alpha + w * s.y;
 #pragma unroll
-  for (int k = 0; k < kSpecParts; ++k) {
-    const int s = min(k, np - 1);
-    st0[k] = *reinterpret_cast<const float2*>(ml + 2 * s * hq);
-    ov0[k] = *reinterpret_cast<const float4*>(po + s * hq * D);
+    for (int j = 0; j < 8; ++j) o[j] = o[j] * alpha + w * v[j];
+  };
+  {
+    const int64_t s = min(r, np - 1) * hq;
+    const float2 st = *reinterpret_cast<const float2*>(ml + 2 * s);
+    const float4 x = *reinterpret_cast<const float4*>(po + s * D), y = *reinterpret_cast<const float4*>(po + s * D + 4);
+    if (r < np) add(st, x, y);
   }
-  float mm = kMaxFloor;
+#pragma unroll 1
+  for (int k0 = 4 + r; k0 - r < np; k0 += 16) {
+    float2 st[4];
+    float4 x[4], y[4];
 #pragma unroll
-  for (int k = 0; k < kSpecParts; ++k)
-    if (k < np) mm = fmaxf(mm, st0[k].x);
-  float ll = 0.f;
-  float4 oo = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-  for (int k = 0; k < kSpecParts; ++k) {
-    if (k < np) {
-      const float w = fast_exp2(st0[k].x - mm);
-      ll += w * st0[k].y;
-      oo = fma4(w, ov0[k], oo);
+    for (int u = 0; u < 4; ++u) {
+      const int64_t s = min(k0 + 4 * u, np - 1) * hq;
+      st[u] = *reinterpret_cast<const float2*>(ml + 2 * s);
+      x[u] = *reinterpret_cast<const float4*>(po + s * D);
+      y[u] = *reinterpret_cast<const float4*>(po + s * D + 4);
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (k0 + 4 * u < np) add(st[u], x[u], y[u]);
   }
-  // Further parts (long sequences): batches of 8, all loads of a batch issued first.
-  for (int s0 = kSpecParts; s0 < np; s0 += 8) {
-    float2 st[8];
-    float4 ov[8];
+  const float mm = xor32_max(xor16_max(m));
+  const float w = fast_exp2(m - mm);
+  const float inv = 1.f / xor32_sum(xor16_sum(l * w));
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int s = min(s0 + k, np - 1);
-      st[k] = *reinterpret_cast<const float2*>(ml + 2 * s * hq);
-      ov[k] = *reinterpret_cast<const float4*>(po + s * hq * D);
-    }
-    float bm = mm;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) bm = fmaxf(bm, st[k].x);
-    const float alpha = fast_exp2(mm - bm);
-    ll *= alpha;
-    oo = make_float4(oo.x * alpha, oo.y * alpha, oo.z * alpha, oo.w * alpha);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      if (s0 + k < np) {
-        const float w = fast_exp2(st[k].x - bm);
-        ll += w * st[k].y;
-        oo = fma4(w, ov[k], oo);
-      }
-    }
-    mm = bm;
-  }
-  uint16_t* o = p.out + b * p.o_seq_stride + h * p.o_head_stride + d;
-  *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(oo.x / ll, oo.y / ll), pack_bf16x2(oo.z / ll, oo.w / ll));
+  for (int j = 0; j < 8; ++j) o[j] = xor32_sum(xor16_sum(o[j] * w)) * inv;
+  if (r == 0) *reinterpret_cast<uint4*>(p.out + b * p.o_seq_stride + h * p.o_head_stride + d) = pack8(o);
 }
 
 constexpr int64_t kHeaderBytes = ((kHeaderInts + kHeaderSeqs + 1) * 4 + 255) / 256 * 256;
