@@ -241,6 +241,15 @@ int kvp_varlen_prefill_bf16(const void* q, int64_t q_tok_stride, int64_t q_head_
 size_t kvp_prefill_workspace_bytes(int32_t num_seqs, int32_t max_seqlen_q, int32_t num_q_heads,
                                    int32_t num_kv_heads);
 
+/*
+ * Bytes of device workspace with which kvp_varlen_prefill_bf16, for up to num_seqs sequences
+ * and max_seqlen_q query tokens, may also split the keys of a batch of few query tiles over
+ * idle workgroups: kvp_prefill_workspace_bytes and 69 MB of partial states.  Such a batch
+ * gives the same results within rounding in the smaller workspace, only slower.
+ */
+size_t kvp_prefill_split_workspace_bytes(int32_t num_seqs, int32_t max_seqlen_q, int32_t num_q_heads,
+                                         int32_t num_kv_heads);
+
 /* ------------------------------------------------------------------------------
  * The layer work on either side of the path (the engine's Qwen3 layers).  Same
  * conventions as above.

@@ -89,6 +89,7 @@ SIGNATURES: dict[str, tuple] = {
         _c_void_p, _size_t, _c_void_p,    # workspace, workspace_bytes, stream
     ]),
     "kvp_prefill_workspace_bytes": (_size_t, [_i32, _i32, _i32, _i32]),
+    "kvp_prefill_split_workspace_bytes": (_size_t, [_i32, _i32, _i32, _i32]),
     "kvp_rmsnorm_bf16": (ctypes.c_int, [
         _c_void_p, _i64, _i64,            # x, x_stride0, x_stride1
         _c_void_p, _i64, _i64,            # residual, residual_stride0, residual_stride1

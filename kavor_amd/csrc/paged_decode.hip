@@ -534,7 +534,7 @@ void paged_decode_kernel(const DecodeParams p) {
 
   build_step_prefix(p, s_cum, s_ctx, s_part);
   const int B = p.num_seqs;
-  const int total_steps = s_cum[B];
+  const int total_steps = __builtin_amdgcn_readfirstlane(s_cum[B]);  // uniform, and a scalar
   const int spr = max(p.min_steps, div_by(total_steps + static_cast<int>(gridDim.y) - 1, p.div_ranges));
   if (blockIdx.x == 0 && blockIdx.y == 0) {  // for the merge kernel
     if (tid == 0) p.header[0] = spr;

@@ -58,6 +58,16 @@ constexpr int kPlanSeqsPerThread = kMaxPrefillSeqs / kPlanThreads;
 constexpr int kPlanLevels = 2048;          // cost levels (64-key tiles) ranked apart; longer units tie at the top
 constexpr int kPlanGroupSlots = 4096;      // first-block hash slots, more than kMaxPrefillSeqs: a probe always ends
 static_assert(kPlanLevels % kPlanThreads == 0 && kMaxPrefillSeqs % kPlanThreads == 0, "plan shape");
+// Split launches (few query tiles on long keys; see prefill_split_plan_kernel).
+constexpr int kSplitTiles = 512;      // query tiles x kv heads of a launch that may be split, at most
+constexpr int kSplitItems = 1024;     // units of a split launch at most (and partial states)
+constexpr int kSplitMinChunk = 8;     // key tiles of a chunk at least
+constexpr int kSplitMinKeys = 1024;   // keys from which a launch may be split
+constexpr int kSplitLevels = 512;     // unit lengths ranked apart
+constexpr int kSplitUnitsInt = 64;    // in the split area: counts, then units, then merges
+constexpr int kSplitMergesInt = kSplitUnitsInt + kUnitInts * kSplitItems;
+constexpr int kSplitInts = kSplitMergesInt + kUnitInts * kSplitTiles;
+constexpr int kPartFloats = kPrefillRows * (kPrefillHeadDim + 2);  // one partial state: O, then (max, sum) per row
 // A tile's row sum of P above this re-bases the running max (P itself stays <= 2^16).
 constexpr float kSpecSumLimit = 65536.f;
 
@@ -85,6 +95,9 @@ struct PrefillParams {
   uint16_t* out;
   int64_t o_tok_stride, o_head_stride;
   int* ws;  // launch workspace: claim counters, unit count, ranked unit pairs
+  int32_t tile_slots;  // split launches: query tiles per sequence the plan covers
+  int* split;          // split launches: [0] unit count, [1] merge count, units, merges
+  float* part;         // split launches: partial states
 };
 
 // Ranks the launch's units for the persistent attention workgroups.  A unit is a pair of
@@ -219,6 +232,183 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const Prefil
   if (tid == 0) p.ws[kWsCountInt] = total * p.num_kv_heads;
 }
 
+// The plan of a split launch: too few query tiles to fill the chip, on long keys (the next
+// turn of a chat: a few hundred new tokens on thousands of cached ones; one long prompt).
+// One workgroup per tile would leave CUs idle while each tile walks all its keys; here the
+// key range of a tile is cut into chunks, each a unit of its own that writes its
+// unnormalised O and (max, sum) in fp32, and prefill_merge_kernel combines them with the
+// online-softmax rule.  A sequence's tiles share their chunk boundaries, so that they read
+// the same keys at about the same time.  A tile of one chunk writes its output directly.
+// The chunk length C is the one of least estimated cost, in key tiles: the longest unit
+// where every unit has a workgroup slot (two per CU), otherwise the mean load of a slot and
+// half the longest unit (units go out longest first), plus the partial states' traffic
+// (66 KB written and read each, about 1/48 key tile) and the merge.
+// Measured against the uncut launch, whole calls with the append: 3 sequences of 17-300 new
+// tokens on 2048-8192 cached (32q/8kv) 156 -> 64 us; 32 new on 4096 (16q/8kv) 83 -> 32 us; 4 of
+// 200-700 on 500-3000 81 -> 60 us; one prompt of 2000 without a prefix 60 -> 46 us, of 3000
+// 82 -> 69 us.
+// A unit: s, tile, q start, q length, k start, k length, first key tile | end << 16 (-1: all
+// key tiles, and the tiles tile_slots apart), partial slot (-1: none).
+// A merge: tile, q start, q length, first partial slot, parts.
+template <int G>
+__global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const PrefillParams p) {
+  constexpr int TOK = kPrefillRows / G;
+  constexpr int U = kSplitTiles / kPlanThreads;
+  constexpr int kCandidates = 20;
+  __shared__ int wtot[2][kPlanThreads / 64];
+  __shared__ int hist[kSplitLevels];
+  __shared__ int s_n[kSplitTiles], s_nm[kSplitTiles];  // key tiles of a tile, and of its sequence
+  __shared__ int s_cost[kCandidates];
+  __shared__ int s_longest;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int J = p.tile_slots, T = p.num_seqs * J;
+  const int slots = kSplitTiles / p.num_kv_heads, most = kSplitItems / p.num_kv_heads;  // T <= slots
+  int flip = 0;
+  // exclusive prefix sum over the threads and the total (a barrier; the buffers alternate)
+  auto scan = [&](u32 x, u32& sum) {
+    const u32 incl = static_cast<u32>(wave_incl_scan(static_cast<int>(x)));
+    if (lane == 63) wtot[flip][wave] = static_cast<int>(incl);
+    __syncthreads();
+    u32 before = incl - x;
+    sum = 0;
+#pragma unroll
+    for (int w = 0; w < kPlanThreads / 64; ++w) {
+      if (w < wave) before += static_cast<u32>(wtot[flip][w]);
+      sum += static_cast<u32>(wtot[flip][w]);
+    }
+    // a scalar: with totals in vector registers the compiler gave a loop that ended on one a
+    // condition code that was not the comparison's
+    sum = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(sum)));
+    flip ^= 1;
+    return before;
+  };
+  if (tid < 8) p.ws[kClaimStride * tid] = 0;
+  if (tid == 0) s_longest = 1;
+  if (tid < kCandidates) s_cost[tid] = 0x7fffffff;
+  for (int i = tid; i < kSplitLevels; i += kPlanThreads) hist[i] = 0;
+  int sq[U], ti[U], q0[U], ql[U], k0[U], kl[U], n[U], nm[U];
+  int work = 0, longest = 1;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int idx = U * tid + u;
+    sq[u] = idx / J;
+    ti[u] = idx - sq[u] * J;
+    q0[u] = ql[u] = k0[u] = kl[u] = n[u] = 0;
+    nm[u] = 1;
+    if (idx < T) {
+      q0[u] = p.cu_q[sq[u]];
+      ql[u] = p.cu_q[sq[u] + 1] - q0[u];
+      k0[u] = p.cu_k[sq[u]];
+      kl[u] = p.cu_k[sq[u] + 1] - k0[u];
+    }
+    const int nt = (ql[u] + TOK - 1) / TOK;
+    if (idx < T && ti[u] < nt) {
+      const int end = min(kl[u], min(ql[u], (ti[u] + 1) * TOK) + kl[u] - ql[u]);  // keys the tile sees
+      n[u] = max(1, (end + kKeyTile - 1) / kKeyTile);
+      nm[u] = max(1, (kl[u] + kKeyTile - 1) / kKeyTile);
+      if (nt > J || nm[u] > 0x7fff) n[u] = nm[u] = 1;  // one unit
+    }
+    s_n[idx] = n[u];
+    s_nm[idx] = nm[u];
+    work += n[u];
+    longest = max(longest, nm[u]);
+  }
+  __syncthreads();
+  if (longest > 1) atomicMax(&s_longest, longest);
+  u32 total;
+  scan(static_cast<u32>(work), total);
+  longest = __builtin_amdgcn_readfirstlane(s_longest);
+  // chunks of a tile at chunk length C: the sequence's keys in equal chunks of at most C
+  auto chunk_of = [](int nm, int C) { const int k = (nm + C - 1) / C; return (nm + k - 1) / k; };
+  // Candidates for C: half the longest, then down by quarters while C stays above a quarter
+  // of the mean load and the units fit; each wave weighs every fourth of them.  The uncut
+  // launch (C = longest, one unit per tile, T <= slots) costs its longest unit.
+  const int floor_c = max(kSplitMinChunk, static_cast<int>(total) / (4 * slots));
+  {
+    int C = (longest + 1) / 2;
+    for (int k = 0; k < kCandidates && C >= floor_c; ++k, C -= max(1, C >> 2)) {
+      if ((k & 3) != __builtin_amdgcn_readfirstlane(wave)) continue;
+      int packed = 0;  // units | partial states << 16: at most T + 8 slots < 2^13 of either
+      for (int i = lane; i < T; i += 64) {
+        const int cs = chunk_of(s_nm[i], C), np = (s_n[i] + cs - 1) / cs;
+        packed += np + (np > 1 ? np << 16 : 0);
+      }
+      const int sum = __builtin_amdgcn_readlane(wave_incl_scan(packed), 63);
+      const int units = sum & 0xffff, partial = sum >> 16;
+      const int cost =
+          (units <= slots ? C : static_cast<int>(total) / slots + C / 2) + partial * p.num_kv_heads / 48 + 4;
+      if (lane == 0 && units <= most) s_cost[k] = cost;
+    }
+  }
+  __syncthreads();
+  int C = longest;
+  {
+    int best_cost = longest, c = (longest + 1) / 2;
+    for (int k = 0; k < kCandidates && c >= floor_c; ++k, c -= max(1, c >> 2)) {
+      const int cost = __builtin_amdgcn_readfirstlane(s_cost[k]);
+      if (cost < best_cost) {
+        best_cost = cost;
+        C = c;
+      }
+    }
+  }
+  int np[U], cs[U];
+  u32 mine = 0;  // units | partial states << 11 | cut tiles << 22: at most 1024, 1024 and 512
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    cs[u] = chunk_of(nm[u], C);
+    np[u] = (n[u] + cs[u] - 1) / cs[u];
+    mine += static_cast<u32>(np[u]);
+    if (np[u] > 1) {
+      mine += (static_cast<u32>(np[u]) << 11) + (1u << 22);
+      // the tile's units by length: np - 1 of cs key tiles, and the rest
+      atomicAdd(&hist[min(cs[u], kSplitLevels - 1)], np[u] - 1);
+    }
+    if (np[u] > 0) atomicAdd(&hist[min(n[u] - (np[u] - 1) * cs[u], kSplitLevels - 1)], 1);
+  }
+  u32 sums;
+  const u32 mark = scan(mine, sums);
+  int slot = static_cast<int>(mark >> 11) & 0x7ff, mat = static_cast<int>(mark >> 22);
+  const int units = static_cast<int>(sums & 0x7ff), all_cuts = static_cast<int>(sums >> 22);
+  // offsets in decreasing length: thread t owns the levels just below thread t - 1's
+  constexpr int LPT = kSplitLevels / kPlanThreads;
+  const int top = kSplitLevels - 1 - LPT * tid;
+  int h[LPT], run = 0;
+  u32 unused;
+#pragma unroll
+  for (int e = 0; e < LPT; ++e) {
+    h[e] = hist[top - e];
+    run += h[e];
+  }
+  int before = static_cast<int>(scan(static_cast<u32>(run), unused));
+#pragma unroll
+  for (int e = 0; e < LPT; ++e) {
+    hist[top - e] = before;
+    before += h[e];
+  }
+  __syncthreads();
+  int* const list = p.split + kSplitUnitsInt;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (np[u] > 1) {
+      int* const m = p.split + kSplitMergesInt + kUnitInts * mat++;
+      *reinterpret_cast<int4*>(m) = make_int4(ti[u], q0[u], ql[u], slot);
+      m[4] = np[u];
+    }
+    for (int i = 0; i < np[u]; ++i) {
+      const int t0 = i * cs[u], t1 = min(n[u], t0 + cs[u]);
+      const int at = atomicAdd(&hist[min(t1 - t0, kSplitLevels - 1)], 1);
+      *reinterpret_cast<int4*>(list + kUnitInts * at) = make_int4(sq[u], ti[u], q0[u], ql[u]);
+      *reinterpret_cast<int4*>(list + kUnitInts * at + 4) =
+          make_int4(k0[u], kl[u], np[u] > 1 ? t0 | (t1 << 16) : -1, np[u] > 1 ? slot++ : -1);
+    }
+  }
+  if (tid == 0) {
+    p.split[0] = units * p.num_kv_heads;
+    p.split[1] = all_cuts;
+  }
+}
+
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 
 // ds_read_b64_tr_b16: 8 bytes per lane, transposed as 16-bit elements across each
@@ -245,12 +435,59 @@ __device__ __forceinline__ f32x16_t mfma32(uint4 a, uint4 b, f32x16_t c) {
                                                  __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+// Writes one wave's 32 query rows: O (scaled by inv) through the LDS area `stg` of 32 rows.
+// The lane holds dims 32mb + 8(j/4) + 4hf + (j%4) of its query row, so a direct store writes
+// 16 bytes into each of 32 rows; staged (in the finished tile buffers of the attention kernel,
+// each wave its own 32 rows, rewritten by the next query tile's second key tile only after
+// that tile's barrier), every store instruction writes whole rows.  A row's 16-byte chunk c
+// sits at chunk c ^ (row & 15) and its 8-byte halves swap for rows 16..31, so neither the
+// 8-byte writes nor the 16-byte reads share a bank.  Dense 32-sequence prefill 92.9 -> 88.1
+// us, prefix-cached 343.0 -> 341.1 us, same outputs.
+template <int G>
+__device__ __forceinline__ void write_rows(const PrefillParams& p, uint16_t* const stg,
+                                           const f32x16_t (&oacc)[kPrefillHeadDim / 32], float inv, int lane, int wave,
+                                           int q0, int q_start, int qlen, int kvh) {
+  constexpr int D = kPrefillHeadDim;
+  constexpr int TOK = kPrefillRows / G;
+  // lane index recomputed here: offsets derived from it are not hoisted out of the
+  // unit loop (where they would hold 24 registers through the key loop)
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  const int nn = ln & 31, hh = ln >> 5;
+  const int hsw = (nn >> 4) & 1;
+#pragma unroll
+  for (int mb = 0; mb < D / 32; ++mb)
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq) {
+      const int c = 4 * mb + jq;
+      const uint2 w = make_uint2(pack_bf16x2(oacc[mb][4 * jq] * inv, oacc[mb][4 * jq + 1] * inv),
+                                 pack_bf16x2(oacc[mb][4 * jq + 2] * inv, oacc[mb][4 * jq + 3] * inv));
+      *reinterpret_cast<uint2*>(stg + nn * kPrefillHeadDim + 8 * (c ^ (nn & 15)) + 4 * (hh ^ hsw)) = w;
+    }
+  __builtin_amdgcn_wave_barrier();  // a wave's LDS accesses run in order
+  const int chunk = ln & 15;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int row = 4 * i + (ln >> 4);
+    uint4 v = *reinterpret_cast<const uint4*>(stg + row * kPrefillHeadDim + 8 * (chunk ^ (row & 15)));
+    if ((row >> 4) & 1) v = make_uint4(v.z, v.w, v.x, v.y);
+    const int rho_o = 32 * wave + row;
+    const int tq_o = rho_o / G;
+    const int qi_o = q0 + tq_o;
+    if (tq_o < TOK && qi_o < qlen) {
+      uint16_t* op = p.out + static_cast<int64_t>(q_start + qi_o) * p.o_tok_stride +
+                     static_cast<int64_t>(kvh * G + rho_o - tq_o * G) * p.o_head_stride + 8 * chunk;
+      *reinterpret_cast<uint4*>(op) = v;
+    }
+  }
+}
+
 // Two workgroups per CU (2 waves per SIMD, <= 256 registers per wave): the workgroups'
 // barriers are independent, so one's MFMAs overlap the other's softmax (measured
 // 1.45 -> 0.83 ms on the prefix-cached prefill workload vs one 4-wave workgroup per CU,
 // 0.97 ms with one 8-wave workgroup).
 
-template <int G, bool PAGED, bool CAUSAL>
+template <int G, bool PAGED, bool CAUSAL, bool SPLIT>
 __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu(2))) void varlen_prefill_kernel(const PrefillParams p) {
   constexpr int D = kPrefillHeadDim;
   constexpr int TOK = kPrefillRows / G;  // query tokens per tile
@@ -285,17 +522,17 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   const int J = p.pair_slots;  // tile pairs per (sequence, kv head) the plan covers
   const int xcd = blockIdx.x & 7;
   int* const ctr = p.ws + kClaimStride * xcd;
-  const int num_units = __builtin_amdgcn_readfirstlane(p.ws[kWsCountInt]);
+  const int num_units = __builtin_amdgcn_readfirstlane(SPLIT ? p.split[0] : p.ws[kWsCountInt]);
   if (tid == 0) s_claim[0] = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   int claim = __builtin_amdgcn_readfirstlane(s_claim[0]);
   int cslot = 1;
 
   for (;;) {
-  const int r = 8 * (claim / kXcdGroup) + xcd;  // rank in decreasing cost
-  const int member = claim % kXcdGroup;         // which tile of the unit
+  const int r = SPLIT ? 8 * claim + xcd : 8 * (claim / kXcdGroup) + xcd;  // rank in decreasing cost
+  const int member = SPLIT ? 0 : claim % kXcdGroup;  // which tile of the unit
   if (r >= num_units) break;             // uniform
-  const int* ent = p.ws + kWsUnitsInt + kUnitInts * (r / p.num_kv_heads);
+  const int* ent = (SPLIT ? p.split + kSplitUnitsInt : p.ws + kWsUnitsInt) + kUnitInts * (r / p.num_kv_heads);
   const int kvh = r % p.num_kv_heads;
   const int s = __builtin_amdgcn_readfirstlane(ent[0]);
   const int jj = __builtin_amdgcn_readfirstlane(ent[1]);
@@ -304,6 +541,8 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   const int k_start = __builtin_amdgcn_readfirstlane(ent[4]);
   const int klen = __builtin_amdgcn_readfirstlane(ent[5]);
   const int diag = klen - qlen;  // bottom-right causal offset
+  const int key_range = SPLIT ? __builtin_amdgcn_readfirstlane(ent[6]) : -1;
+  const int part_slot = SPLIT ? __builtin_amdgcn_readfirstlane(ent[7]) : -1;
 
   bool bad = false;
   if (PAGED && klen > p.max_blocks * p.block_size) bad = true;
@@ -359,30 +598,26 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   const uint16_t* v_tile = nullptr;
   const int64_t k_tile_step = PAGED ? static_cast<int64_t>(kKeyTile) * p.k_tok_stride : 0;
   const int64_t v_tile_step = PAGED ? static_cast<int64_t>(kKeyTile) * p.v_tok_stride : 0;
+  auto start_block = [&](int lblk) __attribute__((always_inline)) {
+    const int w = lblk >> 6;
+    if (w != bt_win) {  // uniform
+      bt_lane = 64 * w + lane < p.max_blocks ? p.block_tables[s * p.bt_stride + 64 * w + lane] : -1;
+      bt_win = w;
+    }
+    int blk = lblk < p.max_blocks ? __builtin_amdgcn_readlane(bt_lane, lblk & 63) : -1;
+    if (blk < 0 || blk >= p.num_cache_blocks) {
+      bad = true;
+      blk = 0;
+    }
+    k_tile = p.k + static_cast<int64_t>(blk) * p.k_blk_stride + static_cast<int64_t>(kvh) * p.k_head_stride;
+    v_tile = p.v + static_cast<int64_t>(blk) * p.v_blk_stride + static_cast<int64_t>(kvh) * p.v_head_stride;
+  };
   auto issue_kv = [&](int kv0, uint16_t* dk, uint16_t* dv) __attribute__((always_inline)) {
-    if (kv0 == 0) {  // uniform: a query tile's first key tile
+    if (!SPLIT && kv0 == 0) {  // uniform: a query tile's first key tile (SPLIT: set by the caller)
       nx_lblk = 0;
       nx_boff = 0;
-      if (!PAGED) {
-        k_tile = p.k + static_cast<int64_t>(k_start) * p.k_tok_stride + static_cast<int64_t>(kvh) * p.k_head_stride;
-        v_tile = p.v + static_cast<int64_t>(k_start) * p.v_tok_stride + static_cast<int64_t>(kvh) * p.v_head_stride;
-      }
     }
-    if (PAGED && nx_boff == 0) {  // uniform: the tile starts a block
-      const int lblk = nx_lblk;
-      const int w = lblk >> 6;
-      if (w != bt_win) {  // uniform
-        bt_lane = 64 * w + lane < p.max_blocks ? p.block_tables[s * p.bt_stride + 64 * w + lane] : -1;
-        bt_win = w;
-      }
-      int blk = lblk < p.max_blocks ? __builtin_amdgcn_readlane(bt_lane, lblk & 63) : -1;
-      if (blk < 0 || blk >= p.num_cache_blocks) {
-        bad = true;
-        blk = 0;
-      }
-      k_tile = p.k + static_cast<int64_t>(blk) * p.k_blk_stride + static_cast<int64_t>(kvh) * p.k_head_stride;
-      v_tile = p.v + static_cast<int64_t>(blk) * p.v_blk_stride + static_cast<int64_t>(kvh) * p.v_head_stride;
-    }
+    if (nx_boff == 0) start_block(nx_lblk);  // uniform: the tile starts a block
     const BufferRsrc krs = buffer_rsrc(k_tile, static_cast<uint32_t>(kKeyTile * k_row_bytes));
     const BufferRsrc vrs = buffer_rsrc(v_tile, static_cast<uint32_t>(kKeyTile * v_row_bytes));
     if (kv0 + kKeyTile <= klen) {  // uniform: every row of the tile is a key
@@ -410,7 +645,7 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
     k_tile += k_tile_step;
     v_tile += v_tile_step;
     nx_boff += kKeyTile;
-    if (PAGED && nx_boff == p.block_size) {
+    if (nx_boff == p.block_size) {
       nx_boff = 0;
       ++nx_lblk;
     }
@@ -485,8 +720,9 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   // This unit's tile pairs jj, jj + J, jj + 2J, ... counted from the last tile (more
   // than one only when max_seqlen_q understates the sequence); member 0 takes the later
   // tile of each pair, member 1 the earlier one.
-  for (int t = kXcdGroup * jj + member; t < ntiles_seq; t += kXcdGroup * J) {
-    const int tile = ntiles_seq - 1 - t;
+  // SPLIT: query tile jj, and the ones tile_slots apart if there are any
+  for (int t = SPLIT ? jj : kXcdGroup * jj + member; t < ntiles_seq; t += SPLIT ? p.tile_slots : kXcdGroup * J) {
+    const int tile = SPLIT ? t : ntiles_seq - 1 - t;
     const int q0 = tile * TOK;
 
     // This lane's query row.
@@ -508,7 +744,10 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
 
     const int q_last = min(qlen, q0 + TOK) - 1;
     const int kv_end = CAUSAL ? min(klen, q_last + diag + 1) : klen;
-    const int nkv = kv_end > 0 ? (kv_end + kKeyTile - 1) / kKeyTile : 0;
+    const int nkv_all = kv_end > 0 ? (kv_end + kKeyTile - 1) / kKeyTile : 0;
+    // the unit's key tiles [it0, nkv)
+    const int it0 = SPLIT && key_range >= 0 ? key_range & 0xffff : 0;
+    const int nkv = SPLIT && key_range >= 0 ? min(nkv_all, key_range >> 16) : nkv_all;
 
     f32x16_t oacc[D / 32];
 #pragma unroll
@@ -524,12 +763,21 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
     const int wave_max_limit = CAUSAL ? q0 + (32 * wave + 31) / G + diag : klen - 1;
     const bool wave_live = q0 + (32 * wave) / G < qlen;
 
-    if (nkv > 0) {
+    if (nkv > it0) {
       if constexpr (PAGED) {
-        issue_kv(0, s_k0, s_v0);
+        if (SPLIT) {  // the unit's first key tile may lie inside a block
+          nx_lblk = it0 * kKeyTile / p.block_size;
+          nx_boff = it0 * kKeyTile - nx_lblk * p.block_size;
+          if (nx_boff != 0) {
+            start_block(nx_lblk);
+            k_tile += nx_boff * p.k_tok_stride;
+            v_tile += nx_boff * p.v_tok_stride;
+          }
+        }
+        issue_kv(it0 * kKeyTile, s_k0, s_v0);
       } else {
-        issue_k(0, s_k0);
-        issue_v(0, s_v0);
+        issue_k(it0 * kKeyTile, s_k0);
+        issue_v(it0 * kKeyTile, s_v0);
       }
     }
     auto tile_step = [&](int it, const uint16_t* sk, const uint16_t* sv, uint16_t* nk, uint16_t* nv)
@@ -619,7 +867,7 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
           for (int j = 0; j < 16; ++j) mx = fmaxf(mx, sacc[mb][j]);
         return half_swap_max(mx) * p.scale_log2;
       };
-      if (it == 0) m_run = tile_max();  // uniform; O and l are still zero
+      if (it == it0) m_run = tile_max();  // uniform; O and l are still zero
       float rsum = 0.f;
       u32 pk[2][8];  // P as packed bf16 pairs: [mb][pair]
       auto make_p = [&]() __attribute__((always_inline)) {
@@ -688,55 +936,30 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
         __builtin_amdgcn_sched_group_barrier(0x008, D / 32, 0);
       }
     };
-    for (int it = 0; it < nkv; it += 2) {
+    for (int it = it0; it < nkv; it += 2) {
       tile_step(it, s_k0, s_v0, s_k1, s_v1);
       if (it + 1 < nkv) tile_step(it + 1, s_k1, s_v1, s_k0, s_v0);
     }
     __builtin_amdgcn_s_setprio(0);
     __syncthreads();  // every wave is done with the tile buffers (the next unit restages them)
 
-    // ---- write O through LDS.  The lane holds dims 32mb + 8(j/4) + 4hf + (j%4) of its
-    // query row, so a direct store writes 16 bytes into each of 32 rows; staged in the
-    // finished tile buffers (each wave its own 32 rows, rewritten by the next query tile's
-    // second key tile only after that tile's barrier), every store instruction writes
-    // whole rows.  A row's 16-byte chunk c sits at chunk c ^ (row & 15) and its 8-byte
-    // halves swap for rows 16..31, so neither the 8-byte writes nor the 16-byte reads
-    // share a bank.  Dense 32-sequence prefill 92.9 -> 88.1 us, prefix-cached 343.0 ->
-    // 341.1 us, same outputs.
-    {
-      const float inv = bad ? NAN : (l_run > 0.f ? 1.f / l_run : 0.f);
-      uint16_t* const stg = (wave < 2 ? s_k1 : s_v1) + (wave & 1) * 32 * kPrefillHeadDim;
-      // lane index recomputed here: offsets derived from it are not hoisted out of the
-      // unit loop (where they would hold 24 registers through the key loop)
-      int ln = lane;
+    if (SPLIT && part_slot >= 0) {  // a partial state, laid out as the lanes hold it
+      float* const po = p.part + static_cast<int64_t>(part_slot * p.num_kv_heads + kvh) * kPartFloats;
+      int ln = lane;  // recomputed here, as in write_rows
       asm volatile("" : "+v"(ln));
-      const int nn = ln & 31, hh = ln >> 5;
-      const int hsw = (nn >> 4) & 1;
+      float* const at = po + 4 * (1024 * wave + ln);
 #pragma unroll
       for (int mb = 0; mb < D / 32; ++mb)
 #pragma unroll
-        for (int jq = 0; jq < 4; ++jq) {
-          const int c = 4 * mb + jq;
-          const uint2 w = make_uint2(pack_bf16x2(oacc[mb][4 * jq] * inv, oacc[mb][4 * jq + 1] * inv),
-                                     pack_bf16x2(oacc[mb][4 * jq + 2] * inv, oacc[mb][4 * jq + 3] * inv));
-          *reinterpret_cast<uint2*>(stg + nn * kPrefillHeadDim + 8 * (c ^ (nn & 15)) + 4 * (hh ^ hsw)) = w;
-        }
-      __builtin_amdgcn_wave_barrier();  // a wave's LDS accesses run in order
-      const int chunk = ln & 15;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int row = 4 * i + (ln >> 4);
-        uint4 v = *reinterpret_cast<const uint4*>(stg + row * kPrefillHeadDim + 8 * (chunk ^ (row & 15)));
-        if ((row >> 4) & 1) v = make_uint4(v.z, v.w, v.x, v.y);
-        const int rho_o = 32 * wave + row;
-        const int tq_o = rho_o / G;
-        const int qi_o = q0 + tq_o;
-        if (tq_o < TOK && qi_o < qlen) {
-          uint16_t* op = p.out + static_cast<int64_t>(q_start + qi_o) * p.o_tok_stride +
-                         static_cast<int64_t>(kvh * G + rho_o - tq_o * G) * p.o_head_stride + 8 * chunk;
-          *reinterpret_cast<uint4*>(op) = v;
-        }
-      }
+        for (int jq = 0; jq < 4; ++jq)
+          *reinterpret_cast<float4*>(at + 256 * (4 * mb + jq)) =
+              make_float4(oacc[mb][4 * jq], oacc[mb][4 * jq + 1], oacc[mb][4 * jq + 2], oacc[mb][4 * jq + 3]);
+      if (ln < 32)
+        *reinterpret_cast<float2*>(po + kPrefillRows * D + 2 * (32 * wave + ln)) = make_float2(m_run, bad ? NAN : l_run);
+    } else {
+      const float inv = bad ? NAN : (l_run > 0.f ? 1.f / l_run : 0.f);
+      write_rows<G>(p, (wave < 2 ? s_k1 : s_v1) + (wave & 1) * 32 * kPrefillHeadDim, oacc, inv, lane, wave, q0, q_start,
+                    qlen, kvh);
     }
   }
   // The next claim is taken only now, when the workgroup is ready to start it: the two
@@ -752,9 +975,67 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   }  // next unit
 }
 
+// Combines the chunks of the query tiles that a split launch cut: a workgroup takes 32 rows
+// of a tile and kv head, each of its waves 32 dims of them, its lanes holding the same
+// elements as the attention kernel's.  The loads of four parts are in flight together: for
+// 3 sequences of 17-300 new tokens on 2048-8192 cached (32q/8kv, 440 parts) 7.4 us, against
+// 14.2 us with one wave walking all 128 dims of its rows part by part.
+// A part that saw no key has weight zero; a part of a bad block table has a NaN sum.
+template <int G>
+__global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(const PrefillParams p) {
+  constexpr int D = kPrefillHeadDim;
+  constexpr int TOK = kPrefillRows / G;
+  const int hk = blockIdx.x >> 2, quarter = blockIdx.x & 3;  // rows 32 quarter .. + 31
+  const int e = hk / p.num_kv_heads, kvh = hk - e * p.num_kv_heads;
+  if (e >= p.split[1]) return;
+  const int lane = threadIdx.x & 63, mb = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int* cut = p.split + kSplitMergesInt + kUnitInts * e;
+  const int np = __builtin_amdgcn_readfirstlane(cut[4]);
+  const float* base = p.part + static_cast<int64_t>(cut[3] * p.num_kv_heads + kvh) * kPartFloats;
+  const int64_t step = static_cast<int64_t>(p.num_kv_heads) * kPartFloats;  // between a tile's parts
+  const int row = 32 * quarter + (lane & 31);
+  const float* ml = base + kPrefillRows * D + 2 * row;
+  const float* po = base + 4 * (64 * (16 * quarter + 4 * mb) + lane);
+  float m = kMaxFloor, l = 0.f, o[16] = {};
+#pragma unroll 1
+  for (int i = 0; i < np; i += 4) {
+    float2 st[4];
+    float4 x[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t at = min(i + u, np - 1) * step;
+      st[u] = *reinterpret_cast<const float2*>(ml + at);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[u][c] = *reinterpret_cast<const float4*>(po + at + 256 * c);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (i + u >= np) break;
+      const float m_new = fmaxf(m, st[u].x), alpha = fast_exp2(m - m_new), w = fast_exp2(st[u].x - m_new);
+      m = m_new;
+      l = l * alpha + w * st[u].y;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float v[4] = {x[u][c].x, x[u][c].y, x[u][c].z, x[u][c].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[4 * c + j] = o[4 * c + j] * alpha + w * v[j];
+      }
+    }
+  }
+  const float inv = l != l ? NAN : (l > 0.f ? 1.f / l : 0.f);
+  const int tq = row / G, qi = cut[0] * TOK + tq;
+  if (tq >= TOK || qi >= cut[2]) return;
+  uint16_t* op = p.out + static_cast<int64_t>(cut[1] + qi) * p.o_tok_stride +
+                 static_cast<int64_t>(kvh * G + row - tq * G) * p.o_head_stride + 32 * mb + 4 * (lane >> 5);
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    *reinterpret_cast<uint2*>(op + 8 * c) = make_uint2(pack_bf16x2(o[4 * c] * inv, o[4 * c + 1] * inv),
+                                                       pack_bf16x2(o[4 * c + 2] * inv, o[4 * c + 3] * inv));
+}
+
 // Workgroups of one kernel variant resident on the current device (cached per variant and
 // device), rounded down to whole groups of 16 (one pair on each XCD).
-template <int G, bool PAGED, bool CAUSAL>
+template <int G, bool PAGED, bool CAUSAL, bool SPLIT>
 static int64_t prefill_resident() {
   static std::atomic<int64_t> cache[64];
   int dev = 0;
@@ -762,7 +1043,7 @@ static int64_t prefill_resident() {
   int64_t v = cache[dev].load(std::memory_order_relaxed);
   if (v > 0) return v;
   int per_cu = 0, cus = 0;
-  bool ok = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, varlen_prefill_kernel<G, PAGED, CAUSAL>,
+  bool ok = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, varlen_prefill_kernel<G, PAGED, CAUSAL, SPLIT>,
                                                          kPrefillThreads, 0) == hipSuccess && per_cu >= 1;
   if (!ok) per_cu = 1;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
@@ -779,13 +1060,30 @@ static int64_t prefill_resident() {
 template <int G, bool PAGED, bool CAUSAL>
 static void launch_variant(hipStream_t s, const PrefillParams& p) {
   hipLaunchKernelGGL((prefill_plan_kernel<G>), dim3(1), dim3(kPlanThreads), 0, s, p);
-  const int64_t grid = prefill_resident<G, PAGED, CAUSAL>();
-  hipLaunchKernelGGL((varlen_prefill_kernel<G, PAGED, CAUSAL>), dim3(static_cast<unsigned>(grid)),
+  const int64_t grid = prefill_resident<G, PAGED, CAUSAL, false>();
+  hipLaunchKernelGGL((varlen_prefill_kernel<G, PAGED, CAUSAL, false>), dim3(static_cast<unsigned>(grid)),
                      dim3(kPrefillThreads), 0, s, p);
+}
+
+// A split launch: its plan, the units (causal instances only), and the merge of the tiles
+// that were cut (a workgroup per quarter of every tile there can be; the others return).
+template <int G, bool PAGED>
+static void launch_split(hipStream_t s, const PrefillParams& p) {
+  const int64_t tiles = static_cast<int64_t>(p.num_seqs) * p.tile_slots * p.num_kv_heads;
+  hipLaunchKernelGGL((prefill_split_plan_kernel<G>), dim3(1), dim3(kPlanThreads), 0, s, p);
+  const int64_t grid = prefill_resident<G, PAGED, true, true>();
+  hipLaunchKernelGGL((varlen_prefill_kernel<G, PAGED, true, true>), dim3(static_cast<unsigned>(grid)),
+                     dim3(kPrefillThreads), 0, s, p);
+  hipLaunchKernelGGL((prefill_merge_kernel<G>), dim3(static_cast<unsigned>(4 * tiles)), dim3(kPrefillThreads), 0, s, p);
 }
 
 template <int G>
 static void launch_prefill(bool paged, bool causal, hipStream_t s, const PrefillParams& p) {
+  if (p.split) {
+    if (paged) launch_split<G, true>(s, p);
+    else launch_split<G, false>(s, p);
+    return;
+  }
   if (paged) {
     if (causal) launch_variant<G, true, true>(s, p);
     else launch_variant<G, true, false>(s, p);
@@ -805,6 +1103,21 @@ static int64_t prefill_pair_slots(int64_t max_seqlen_q, int g) {
 static int64_t prefill_workspace_need(int64_t seqs, int64_t pair_slots) {
   return 4 * static_cast<int64_t>(kWsUnitsInt) + 4 * kUnitInts * seqs * pair_slots;
 }
+
+// Query tiles per sequence that cover max_seqlen_q tokens, where a launch may be split: its
+// tiles leave workgroup slots free.  0 otherwise.
+static int64_t split_tile_slots(int64_t seqs, int64_t max_seqlen_q, int g, int64_t kv_heads) {
+  const int64_t tok = kPrefillRows / g, tiles = (max_seqlen_q + tok - 1) / tok;
+  return seqs * tiles * kv_heads <= kSplitTiles ? tiles : 0;
+}
+
+// The split area behind the work list: its byte offset, and the workspace that holds it.
+static int64_t split_offset(int64_t need) { return (need + 255) / 256 * 256; }
+static int64_t split_workspace_need(int64_t need) {
+  return split_offset(need) + 4 * static_cast<int64_t>(kSplitInts) +
+         4 * static_cast<int64_t>(kSplitItems) * kPartFloats;
+}
+static_assert(4 * kSplitInts % 256 == 0, "partial states follow the lists, aligned");
 
 }  // namespace kvp
 
@@ -896,6 +1209,23 @@ extern "C" int kvp_varlen_prefill_bf16(const void* q, int64_t q_tok_stride, int6
   p.o_tok_stride = out_tok_stride;
   p.o_head_stride = out_head_stride;
   p.ws = static_cast<int*>(workspace);
+  // Split where the tiles leave workgroups idle, the keys are long (a block table's width
+  // bounds them; without one they are taken to be the queries) and the workspace holds the
+  // partial states.  The tile count is a bound, exact for one sequence: its tiles all walk a
+  // long cached prefix, and from about 3/4 of the slots on two halves of each take as long as
+  // the whole (1500 new tokens on 15000 cached, 376 tiles: 406 us unsplit, 413 us with the
+  // split plan, which then cuts nothing).
+  const int64_t most_keys = paged ? static_cast<int64_t>(max_blocks_per_seq) * block_size : max_seqlen_q;
+  p.tile_slots = static_cast<int32_t>(split_tile_slots(num_seqs, max_seqlen_q, G, num_kv_heads));
+  p.split = nullptr;
+  p.part = nullptr;
+  const bool even = num_seqs == 1 && most_keys >= 3 * static_cast<int64_t>(max_seqlen_q) &&
+                    static_cast<int64_t>(p.tile_slots) * num_kv_heads > kSplitTiles * 11 / 16;
+  if (causal && p.tile_slots > 0 && most_keys >= kSplitMinKeys && !even &&
+      workspace_bytes >= static_cast<size_t>(split_workspace_need(need))) {
+    p.split = p.ws + split_offset(need) / 4;
+    p.part = reinterpret_cast<float*>(p.split + kSplitInts);
+  }
 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool c = causal != 0;
@@ -929,4 +1259,10 @@ extern "C" size_t kvp_prefill_workspace_bytes(int32_t num_seqs, int32_t max_seql
   if (g != 1 && g != 2 && g != 4 && g != 5 && g != 8) return 0;
   return static_cast<size_t>(
       prefill_workspace_need(std::min(num_seqs, kMaxPrefillSeqs), prefill_pair_slots(max_seqlen_q, g)));
+}
+
+extern "C" size_t kvp_prefill_split_workspace_bytes(int32_t num_seqs, int32_t max_seqlen_q, int32_t num_q_heads,
+                                                    int32_t num_kv_heads) {
+  const size_t need = kvp_prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads);
+  return need == 0 ? 0 : static_cast<size_t>(split_workspace_need(static_cast<int64_t>(need)));
 }

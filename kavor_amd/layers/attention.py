@@ -114,6 +114,9 @@ def reserve_decode_workspace(max_num_seqs: int, num_q_heads: int, head_dim: int,
     ws = _workspaces.get(dev.index)
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
+            least = decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim, max_blocks_per_seq, block_size)
+            if ws is not None and ws.numel() >= least:
+                return ws  # enough for longer ranges
             raise RuntimeError(
                 "the paged-decode workspace must be reserved before graph capture "
                 f"({nbytes} bytes needed): call reserve_decode_workspace() first")
@@ -135,23 +138,27 @@ def prefill_workspace_bytes(num_seqs: int, max_seqlen_q: int, num_q_heads: int, 
 
 def reserve_prefill_workspace(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int,
                               device: torch.device | str | int) -> torch.Tensor:
-    """Allocates (or grows) the per-device prefill workspace: the work list of a launch
-    (kvp_prefill_workspace_bytes).  A caller that captures prefill into a graph reserves
+    """Allocates (or grows) the per-device prefill workspace: the work list of a launch and
+    the partial states of a batch whose keys are split
+    (kvp_prefill_split_workspace_bytes).  A caller that captures prefill into a graph reserves
     the largest batch first; an eager call that needs more grows the workspace without
     freeing the one a graph holds."""
-    nbytes = prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads)
+    nbytes = int(lib().kvp_prefill_split_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
     dev = torch.device(device) if not isinstance(device, int) else torch.device("cuda", device)
     if dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
     ws = _prefill_workspaces.get(dev.index)
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
+            if ws is not None and ws.numel() >= prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads):
+                return ws  # enough without the partial states
             raise RuntimeError(
                 "the prefill workspace must be reserved before graph capture "
                 f"({nbytes} bytes needed): call reserve_prefill_workspace() first")
         if ws is not None:
             _retired_workspaces.append(ws)
-        ws = torch.empty(max(nbytes, 4096), dtype=torch.uint8, device=dev)
+        # a power of two, so that batches of growing size retire few buffers
+        ws = torch.empty(1 << (nbytes - 1).bit_length(), dtype=torch.uint8, device=dev)
         _prefill_workspaces[dev.index] = ws
     return ws
 

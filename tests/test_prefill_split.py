@@ -1,0 +1,169 @@
+"""Prefill of few query tiles on long keys, whose key ranges the launch cuts into chunks
+(prefill_split_plan_kernel, prefill_merge_kernel), against the fp32 oracle and against the
+uncut launch, which a workspace without the split area gives.
+
+Tolerance against the uncut launch: both form P in bf16 against their own running maxima and
+sum in fp32, so the bf16 outputs (|o| < 4) differ by roundings of P (2^-9 relative, averaged
+over the keys) and one bf16 rounding, at most 2^-7: TOL's atol 2e-2 covers both.
+"""
+
+import itertools
+import math
+
+import pytest
+import torch
+
+from kavor_amd import _lib
+from kavor_amd.layers import attention
+from oracle import kvpath_oracle as ref
+from tests.helpers import TOL, gen, interleaved_pool, randn_bf16
+
+pytestmark = pytest.mark.gpu
+SCALE = 128 ** -0.5
+
+
+def _cu(lens):
+    return torch.tensor([0] + list(itertools.accumulate(lens)), dtype=torch.int32)
+
+
+def _paged(seed, qlens, prefixes, G, hkv, bs):
+    g = gen(seed)
+    klens = [a + b for a, b in zip(qlens, prefixes)]
+    need = [math.ceil(k / bs) for k in klens]
+    nb = sum(need) + 2
+    _, kc, vc = interleaved_pool(nb, bs, hkv, 128, g)
+    ids = torch.randperm(nb, generator=g).tolist()
+    bt = torch.full((len(qlens), max(need)), -1, dtype=torch.int32)
+    for s, n in enumerate(need):
+        bt[s, :n] = torch.tensor(ids[:n], dtype=torch.int32)
+        ids = ids[n:]
+    return randn_bf16((sum(qlens), G * hkv, 128), g), kc, vc, bt, _cu(qlens), _cu(klens)
+
+
+def _run(dev, q, k, v, bt, cq, ck, max_q, small=False):
+    """varlen_prefill; `small`: with just the workspace that a launch without splits needs."""
+    args = [t.to(dev) for t in (q, k, v)]
+    hq, hkv = q.shape[1], k.shape[-2]
+    kept = attention._prefill_workspaces.pop(dev.index, None)
+    if small:
+        n = attention.prefill_workspace_bytes(cq.numel() - 1, max_q, hq, hkv)
+        real = attention.reserve_prefill_workspace
+        attention.reserve_prefill_workspace = lambda *a: torch.empty(n, dtype=torch.uint8, device=dev)
+    try:
+        out = attention.varlen_prefill(*args, max_q, cq.to(dev), 0, ck.to(dev), SCALE, causal=True,
+                                       block_table=None if bt is None else bt.to(dev))
+        torch.cuda.synchronize()
+    finally:
+        if small:
+            attention.reserve_prefill_workspace = real
+        if kept is not None:
+            attention._prefill_workspaces[dev.index] = kept
+    return out.cpu()
+
+
+CASES = [
+    # one tile on many keys, one row past a tile, a tile of one row; chunks off block borders
+    (2, 8, 256, [64], [4000]), (2, 8, 64, [65], [1500]), (4, 8, 192, [1], [3000]),
+    # ragged turns, an empty sequence, a short one beside long ones
+    (4, 8, 256, [300, 17, 0, 158], [6000, 2048, 700, 5]), (5, 8, 64, [100, 30], [2500, 64]),
+    (8, 4, 64, [70, 33], [1111, 4096]), (1, 4, 256, [200, 129], [1024, 0]),
+    # no prefix: causal tiles of 1 .. n key tiles, some cut and some not
+    (2, 8, 256, [1500], [0]), (2, 2, 64, [2100, 700], [0, 900]),
+]
+
+
+@pytest.mark.parametrize("G,hkv,bs,qlens,prefixes", CASES)
+def test_split_paged_matches_oracle(cuda_device, G, hkv, bs, qlens, prefixes):
+    q, kc, vc, bt, cq, ck = _paged(40 + G + len(qlens), qlens, prefixes, G, hkv, bs)
+    out = _run(cuda_device, q, kc, vc, bt, cq, ck, max(qlens))
+    d = cuda_device
+    want = ref.varlen_prefill(q.to(d), kc.to(d), vc.to(d), cq, ck, SCALE, block_tables=bt.to(d)).cpu()
+    torch.testing.assert_close(out.float(), want, **TOL)
+    uncut = _run(cuda_device, q, kc, vc, bt, cq, ck, max(qlens), small=True)
+    torch.testing.assert_close(out.float(), uncut.float(), **TOL)
+
+
+def test_split_dense_matches_oracle(cuda_device):
+    g, d = gen(60), cuda_device
+    qlens, hkv, G = [1400, 321], 8, 2
+    cu = _cu(qlens)
+    q, k, v = (randn_bf16((sum(qlens), h, 128), g) for h in (G * hkv, hkv, hkv))
+    out = _run(d, q, k, v, None, cu, cu, max(qlens))
+    want = ref.varlen_prefill(q.to(d), k.to(d), v.to(d), cu, cu, SCALE).cpu()
+    torch.testing.assert_close(out.float(), want, **TOL)
+
+
+def test_split_understated_max_seqlen_and_rows_without_keys(cuda_device):
+    """A sequence longer than max_seqlen_q is computed in full (its units stride over tiles);
+    rows before the first key (more queries than keys) are zeros; a bad block id poisons its
+    own sequence only."""
+    qlens, klens, bs, hkv, G = [500, 90, 40], [3000, 50, 2000], 64, 8, 2
+    q, kc, vc, bt, cq, ck = _paged(70, qlens, [k - a for a, k in zip(qlens, klens)], G, hkv, bs)
+    bt[2, 20] = 10 ** 6
+    out = _run(cuda_device, q, kc, vc, bt, cq, ck, 100)
+    good = slice(0, 590)
+    want = ref.varlen_prefill(q[good], kc, vc, cq[:3], ck[:3], SCALE, block_tables=bt[:2])
+    torch.testing.assert_close(out[good].float(), want, **TOL)
+    assert torch.count_nonzero(out[500:540]) == 0
+    assert torch.isnan(out[590:].float()).all()
+
+
+def test_split_replays_in_a_graph(cuda_device):
+    """Captured with one batch's lengths, replayed with others: plan, units and merge follow
+    the lengths on the device."""
+    d, hkv, G, bs, width = cuda_device, 8, 2, 64, 80
+    g = gen(80)
+    _, kc, vc = interleaved_pool(width, bs, hkv, 128, g)
+    kc, vc = kc.to(d), vc.to(d)
+    bt = torch.randperm(width, generator=g).to(torch.int32)[None].to(d)
+    q = randn_bf16((256, G * hkv, 128), g).to(d)
+    cq, ck = torch.zeros(2, dtype=torch.int32, device=d), torch.zeros(2, dtype=torch.int32, device=d)
+    out = torch.zeros_like(q)
+    attention.reserve_prefill_workspace(1, 256, G * hkv, hkv, d)
+
+    def call(o):
+        return attention.varlen_prefill(q, kc, vc, 256, cq, 0, ck, SCALE, causal=True, block_table=bt, out=o)
+
+    cq[1], ck[1] = 256, 4000
+    call(out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out)
+    for ql, kl in ((30, 5000), (256, 1200), (1, 64), (200, 4444)):
+        cq[1], ck[1] = ql, kl
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out[:ql].clone()
+        eager = call(torch.zeros_like(q))[:ql]
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), eager.view(torch.int16))
+        want = ref.varlen_prefill(q[:ql], kc, vc, cq, ck, SCALE, block_tables=bt)
+        torch.testing.assert_close(got.float(), want, **TOL)
+
+
+def test_smaller_workspace_is_accepted_inside_a_capture(cuda_device):
+    """A workspace that holds the work list but no split area (reserved for a wide batch by an
+    older caller) still serves a captured call."""
+    d = cuda_device
+    kept = attention._prefill_workspaces.pop(d.index, None)
+    q, kc, vc, bt, cq, ck = (t.to(d) for t in _paged(90, [100], [2000], 2, 8, 64))
+    base = attention.prefill_workspace_bytes(1, 100, 16, 8)
+    assert _lib.lib().kvp_prefill_split_workspace_bytes(1, 100, 16, 8) > base
+    try:
+        attention._prefill_workspaces[d.index] = torch.empty(base, dtype=torch.uint8, device=d)
+        out = torch.zeros_like(q)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            attention.varlen_prefill(q, kc, vc, 100, cq, 0, ck, SCALE, causal=True, block_table=bt, out=out)
+        for _ in range(2):
+            graph.replay()
+            torch.cuda.synchronize()
+        want = ref.varlen_prefill(q, kc, vc, cq, ck, SCALE, block_tables=bt)
+        torch.testing.assert_close(out.float(), want, **TOL)
+    finally:
+        attention._prefill_workspaces.pop(d.index, None)
+        if kept is not None:
+            attention._prefill_workspaces[d.index] = kept
