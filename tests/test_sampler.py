@@ -115,3 +115,44 @@ def test_sample_in_a_graph_draws_new_noise_each_replay(cuda_device):
     for k, got in enumerate(draws):
         _check_against_oracle(logits, temps.numpy(), 601 + k, got)
     assert not np.array_equal(draws[0], draws[1])
+
+
+@pytest.mark.parametrize("rows,vocab", [(200, 8192 + 3), (3, 151936), (2, 2048 * 8 + 8)])
+def test_values_passed_over_never_win(cuda_device, rows, vocab):
+    """Rows whose shape tests the bound by which values are passed over: flat, peaked, all
+    equal (the noise alone decides), masked with -inf, all -inf, with +inf, with one
+    finite value, huge logits; temperatures from 1e-38 (logit / T overflows) to 1e30."""
+    g = torch.Generator().manual_seed(rows + vocab)
+    logits = torch.randn(rows, vocab, generator=g) * 2
+    temps = torch.empty(rows)
+    shapes = ["flat", "peaked", "equal", "masked", "dead", "inf", "one", "huge"]
+    for r in range(rows):
+        kind = shapes[r % len(shapes)] if rows > 8 else ["peaked", "equal", "masked"][r]
+        temps[r] = [0.7, 1.0, 1e-3, 1e30, 50.0, 1e-38, 0.05][r % 7]
+        if kind == "flat":
+            logits[r] *= 0.1
+        elif kind == "peaked":
+            logits[r, torch.randint(0, vocab, (5,), generator=g)] = 25.0
+        elif kind == "equal":
+            logits[r] = 1.5
+        elif kind == "masked":
+            logits[r, torch.rand(vocab, generator=g) < 0.95] = float("-inf")
+        elif kind == "dead":
+            logits[r] = float("-inf")
+        elif kind == "inf":
+            logits[r, [vocab // 2, vocab - 1]] = float("inf")
+        elif kind == "one":
+            logits[r] = float("-inf")
+            logits[r, vocab - 3] = -7.0
+        else:
+            logits[r] *= 1e37
+    logits = logits.to(torch.bfloat16)
+    buf = torch.zeros(rows, (vocab + 7) // 8 * 8, dtype=torch.bfloat16)
+    buf[:, :vocab] = logits
+    seed = torch.tensor([900], dtype=torch.int32, device=cuda_device)
+    got = sample(buf.to(cuda_device)[:, :vocab], temps.to(cuda_device), seed).cpu()
+    scores = lref.gumbel_scores(logits, temps.numpy(), 901)
+    want = lref.first_argmax(scores)
+    for r in np.flatnonzero(got.numpy() != want):  # a tie to float32 rounding, as above
+        a, b = scores[r, got[r]], scores[r, want[r]]
+        assert abs(a - b) <= 4e-7 * max(1.0, abs(b)), (r, shapes[r % 8], got[r], want[r], a, b)
