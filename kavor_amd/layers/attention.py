@@ -14,6 +14,8 @@ on the current stream; nothing computes on the host and there is no fallback.
 
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 from torch import nn
 
@@ -29,7 +31,8 @@ __all__ = [
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream's handle (building a torch.cuda.Stream for it takes 3.5 us)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _require_cuda_bf16(name: str, t: torch.Tensor) -> None:
@@ -63,24 +66,26 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
     """
     N, num_heads, head_dim = key.shape
     D = num_heads * head_dim
-    assert key.stride(-1) == 1 and value.stride(-1) == 1
-    assert key.stride(1) == head_dim and value.stride(1) == head_dim
-    assert k_cache.stride(1) == D and v_cache.stride(1) == D
+    key_str, value_str, cache_str = key.stride(), value.stride(), k_cache.stride()
+    assert key_str[-1] == 1 and value_str[-1] == 1
+    assert key_str[1] == head_dim and value_str[1] == head_dim
     assert slot_mapping.numel() == N
     assert value.shape == key.shape
-    assert k_cache.shape == v_cache.shape and k_cache.stride() == v_cache.stride()
-    assert k_cache.shape[2:] == (num_heads, head_dim)
+    assert k_cache.shape == v_cache.shape and cache_str == v_cache.stride()
+    assert cache_str[1] == D
+    assert k_cache.dim() == 4
+    num_blocks, block_size, cache_heads, cache_dim = k_cache.shape
+    assert (cache_heads, cache_dim) == (num_heads, head_dim)
     _require_cuda_bf16("key", key)
     _require_cuda_bf16("value", value)
     _require_cuda_bf16("k_cache", k_cache)
     _require_cuda_bf16("v_cache", v_cache)
     _require_int32("slot_mapping", slot_mapping, key.device)
-    num_blocks, block_size = k_cache.shape[0], k_cache.shape[1]
     rc = lib().kvp_append_bf16(
-        key.data_ptr(), key.stride(0), key.stride(1),
-        value.data_ptr(), value.stride(0), value.stride(1),
+        key.data_ptr(), key_str[0], key_str[1],
+        value.data_ptr(), value_str[0], value_str[1],
         k_cache.data_ptr(), v_cache.data_ptr(),
-        k_cache.stride(0), k_cache.stride(1), k_cache.stride(2), num_blocks * block_size,
+        cache_str[0], cache_str[1], cache_str[2], num_blocks * block_size,
         slot_mapping.data_ptr(), N, num_heads, head_dim, block_size, _stream(key))
     check("kvp_append_bf16", rc)
 
@@ -93,6 +98,7 @@ _workspaces: dict[int, torch.Tensor] = {}
 _retired_workspaces: list[torch.Tensor] = []
 
 
+@lru_cache(maxsize=1024)  # arithmetic on the sizes
 def decode_workspace_bytes(max_num_seqs: int, num_q_heads: int, head_dim: int,
                            max_blocks_per_seq: int, block_size: int) -> int:
     return int(lib().kvp_decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim,
@@ -132,8 +138,14 @@ def reserve_decode_workspace(max_num_seqs: int, num_q_heads: int, head_dim: int,
 _prefill_workspaces: dict[int, torch.Tensor] = {}
 
 
+@lru_cache(maxsize=1024)
 def prefill_workspace_bytes(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int) -> int:
     return int(lib().kvp_prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
+
+
+@lru_cache(maxsize=1024)
+def _prefill_split_bytes(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int) -> int:
+    return int(lib().kvp_prefill_split_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
 
 
 def reserve_prefill_workspace(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int,
@@ -143,7 +155,7 @@ def reserve_prefill_workspace(num_seqs: int, max_seqlen_q: int, num_q_heads: int
     (kvp_prefill_split_workspace_bytes).  A caller that captures prefill into a graph reserves
     the largest batch first; an eager call that needs more grows the workspace without
     freeing the one a graph holds."""
-    nbytes = int(lib().kvp_prefill_split_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
+    nbytes = _prefill_split_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads)
     dev = torch.device(device) if not isinstance(device, int) else torch.device("cuda", device)
     if dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
@@ -187,10 +199,11 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     _require_cuda_bf16("q", q3)
     _require_cuda_bf16("k_cache", k_cache)
     _require_cuda_bf16("v_cache", v_cache)
-    if k_cache.shape != v_cache.shape or k_cache.stride() != v_cache.stride():
+    cache_str, q_str = k_cache.stride(), q3.stride()
+    if k_cache.shape != v_cache.shape or cache_str != v_cache.stride():
         raise ValueError("k_cache and v_cache must share shape and strides")
     num_blocks, block_size, Hkv, Dk = k_cache.shape
-    if Dk != D or k_cache.stride(3) != 1 or q3.stride(2) != 1:
+    if Dk != D or cache_str[3] != 1 or q_str[2] != 1:
         raise ValueError("head_dim mismatch or non-contiguous head_dim")
     _require_int32("cache_seqlens", cache_seqlens, q3.device)
     if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.stride(1) != 1:
@@ -207,9 +220,9 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     max_blocks = block_table.shape[1]
     ws = reserve_decode_workspace(B, Hq, D, max_blocks, block_size, q3.device)
     rc = lib().kvp_paged_decode_bf16(
-        q3.data_ptr(), q3.stride(0), q3.stride(1),
+        q3.data_ptr(), q_str[0], q_str[1],
         k_cache.data_ptr(), v_cache.data_ptr(),
-        k_cache.stride(0), k_cache.stride(1), k_cache.stride(2), num_blocks,
+        cache_str[0], cache_str[1], cache_str[2], num_blocks,
         block_table.data_ptr(), block_table.stride(0),
         cache_seqlens.data_ptr(), B, Hq, Hkv, D, block_size, max_blocks,
         float(softmax_scale),

@@ -21,7 +21,7 @@ __all__ = ["rms_norm", "add_rms_norm", "qk_norm_rope_append", "qk_norm_rope", "s
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _check_bf16(name: str, t: torch.Tensor) -> None:
