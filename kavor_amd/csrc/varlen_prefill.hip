@@ -54,9 +54,7 @@ constexpr int kWsCountInt = 8 * kClaimStride;  // the unit count (int index)
 constexpr int kWsUnitsInt = 512;           // first unit pair (int index; byte 2048)
 constexpr int kUnitInts = 8;               // s, pair index, q start, q length, k start, k length, 0, 0
 constexpr int kPlanThreads = 256;
-constexpr int kPlanSeqsPerThread = kMaxPrefillSeqs / kPlanThreads;
 constexpr int kPlanLevels = 2048;          // cost levels (64-key tiles) ranked apart; longer units tie at the top
-constexpr int kPlanGroupSlots = 4096;      // first-block hash slots, more than kMaxPrefillSeqs: a probe always ends
 static_assert(kPlanLevels % kPlanThreads == 0 && kMaxPrefillSeqs % kPlanThreads == 0, "plan shape");
 // Split launches (few query tiles on long keys; see prefill_split_plan_kernel).
 constexpr int kSplitTiles = 512;      // query tiles x kv heads of a launch that may be split, at most
@@ -123,9 +121,15 @@ struct PrefillParams {
 // the group rather than once per sequence (316 -> 278 MB per call on the prefix-cached
 // workload, same time).  An LDS hash table keyed by the first block id holds each group's
 // largest level.
-template <int G>
+// SPT sequences per thread: 1 up to kPlanThreads sequences, otherwise as many as a launch
+// may have.  With one, the hash table is small and the placement, a chain of LDS atomics per
+// sequence, is spread over a wave: 32 sequences of up to 8 pairs 6.3 -> 5.2 us, 2 of 128 pairs
+// 11.0 -> 4.8 us (the whole call of two 8192-token prompts 1002 -> 995 us).
+template <int G, int SPT>
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const PrefillParams p) {
   constexpr int TOK = kPrefillRows / G;
+  constexpr int kPlanSeqsPerThread = SPT;
+  constexpr int kPlanGroupSlots = 2 * SPT * kPlanThreads;  // more than the sequences: a probe always ends
   __shared__ int hist[kPlanLevels];
   __shared__ int wsum[kPlanThreads / 64];
   __shared__ int total;
@@ -166,7 +170,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const Prefil
   // the hash slot of a first block id, inserted if absent (linear probing; fewer ids than
   // slots, so a free or matching slot is always found)
   auto group_slot = [&](int key) {
-    int h = static_cast<int>((static_cast<uint32_t>(key) * 2654435769u) >> 20) & (kPlanGroupSlots - 1);
+    int h = static_cast<int>((static_cast<uint32_t>(key) * 2654435769u) >> 16) & (kPlanGroupSlots - 1);
     for (int probe = 0; probe < kPlanGroupSlots; ++probe) {
       const int prev = atomicCAS(&grp_key[h], -1, key);
       if (prev == -1 || prev == key) return h;
@@ -219,14 +223,37 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const Prefil
   }
   __syncthreads();
   int* units = p.ws + kWsUnitsInt;
+  if constexpr (SPT == 1) {
+    __shared__ int s_seq[6][kPlanThreads];
+    const int mine_n = min(J, ((ql[0] + TOK - 1) / TOK + kXcdGroup - 1) / kXcdGroup);
+    const int fields[6] = {q0[0], ql[0], k0[0], kl[0], lv[0], mine_n};
 #pragma unroll
-  for (int u = 0; u < kPlanSeqsPerThread; ++u) {
-    const int sq = tid + kPlanThreads * u;
-    const int nu = min(J, ((ql[u] + TOK - 1) / TOK + kXcdGroup - 1) / kXcdGroup);
-    for (int j = 0; j < nu; ++j) {
-      const int pos = atomicAdd(&hist[lv[u]], 1);
-      *reinterpret_cast<int4*>(units + kUnitInts * pos) = make_int4(sq, j, q0[u], ql[u]);
-      *reinterpret_cast<int4*>(units + kUnitInts * pos + 4) = make_int4(k0[u], kl[u], 0, 0);
+    for (int f = 0; f < 6; ++f) s_seq[f][tid] = fields[f];
+    __syncthreads();
+    // Up to 64 sequences: one wave, 2^sh >= num_seqs sequences side by side and 64 / 2^sh of
+    // its lanes on each one's pairs, so that a level's pairs still land in the order of their
+    // index (all four waves at once were as fast here, but mixed long and short pairs:
+    // two prompts of 8192 tokens 1036 -> 1043 us).  More: a thread per sequence.
+    const bool wide = p.num_seqs > 64;
+    const int sh = wide ? 8 : (p.num_seqs > 1 ? 32 - __clz(p.num_seqs - 1) : 0);
+    const int sq = tid & ((1 << sh) - 1);
+    const int nu = sq < p.num_seqs && (wide || tid < 64) ? s_seq[5][sq] : 0;
+    const int stride = wide ? 1 : 64 >> sh;
+    for (int j = tid >> sh; j < nu; j += stride) {
+      const int pos = atomicAdd(&hist[s_seq[4][sq]], 1);
+      *reinterpret_cast<int4*>(units + kUnitInts * pos) = make_int4(sq, j, s_seq[0][sq], s_seq[1][sq]);
+      *reinterpret_cast<int4*>(units + kUnitInts * pos + 4) = make_int4(s_seq[2][sq], s_seq[3][sq], 0, 0);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < kPlanSeqsPerThread; ++u) {
+      const int sq = tid + kPlanThreads * u;
+      const int nu = min(J, ((ql[u] + TOK - 1) / TOK + kXcdGroup - 1) / kXcdGroup);
+      for (int j = 0; j < nu; ++j) {
+        const int pos = atomicAdd(&hist[lv[u]], 1);
+        *reinterpret_cast<int4*>(units + kUnitInts * pos) = make_int4(sq, j, q0[u], ql[u]);
+        *reinterpret_cast<int4*>(units + kUnitInts * pos + 4) = make_int4(k0[u], kl[u], 0, 0);
+      }
     }
   }
   if (tid == 0) p.ws[kWsCountInt] = total * p.num_kv_heads;
@@ -1059,7 +1086,10 @@ static int64_t prefill_resident() {
 // persistent workgroups (a multiple of 16, so each XCD holds the same number) claims them.
 template <int G, bool PAGED, bool CAUSAL>
 static void launch_variant(hipStream_t s, const PrefillParams& p) {
-  hipLaunchKernelGGL((prefill_plan_kernel<G>), dim3(1), dim3(kPlanThreads), 0, s, p);
+  if (p.num_seqs <= kPlanThreads)
+    hipLaunchKernelGGL((prefill_plan_kernel<G, 1>), dim3(1), dim3(kPlanThreads), 0, s, p);
+  else
+    hipLaunchKernelGGL((prefill_plan_kernel<G, kMaxPrefillSeqs / kPlanThreads>), dim3(1), dim3(kPlanThreads), 0, s, p);
   const int64_t grid = prefill_resident<G, PAGED, CAUSAL, false>();
   hipLaunchKernelGGL((varlen_prefill_kernel<G, PAGED, CAUSAL, false>), dim3(static_cast<unsigned>(grid)),
                      dim3(kPrefillThreads), 0, s, p);
