@@ -45,11 +45,21 @@ struct NormParams {
   float eps;
 };
 
-// LANES (16 or 64) lanes normalise one row; each lane owns up to MAXC 8-element chunks.
+// LANES lanes normalise one row (16 or 64: several rows per workgroup; 128 to 512: the
+// workgroup is one row, its waves' sums meet in LDS); each lane owns up to MAXC 8-element
+// chunks.  Wide rows take several waves: a wave with 8 or 16 chunks per lane holds them all
+// in registers until the sum is known, so few waves fit a CU and one row is a long serial
+// chain.  One wave per row against the workgroups below (graph-replayed, rotating inputs):
+// 4096 x 5120 40.5 -> 18.9 us, 12000 x 5120 112.7 -> 48.0, 4096 x 4096 19.8 -> 14.5, 1 x 5120
+// 4.7 -> 2.4, 48 x 4096 3.9 -> 2.4, 48 x 2048 2.8 -> 2.2, 48 x 1024 with a residual 2.86 -> 2.50.
+// From kNormManyRows rows of up to 1024 columns a wave per row is the better: 16384 x 1024 with
+// a residual 27.6 against 28.5 us.
+constexpr int kNormManyRows = 8192;
 template <int LANES, int MAXC>
-__global__ __launch_bounds__(kThreads) void rmsnorm_kernel(NormParams p) {
+__global__ __launch_bounds__(LANES > 64 ? LANES : kThreads) void rmsnorm_kernel(NormParams p) {
+  constexpr int THREADS = LANES > 64 ? LANES : kThreads;
   const int lane = threadIdx.x % LANES;
-  const int row = (blockIdx.x * kThreads + threadIdx.x) / LANES;
+  const int row = (blockIdx.x * THREADS + threadIdx.x) / LANES;
   if (row >= p.num_rows) return;  // uniform across the lanes of a row
   const int t = row / p.rows_inner, h = row - t * p.rows_inner;
   const uint16_t* xr = p.x + t * p.x_s0 + h * p.x_s1;
@@ -87,7 +97,15 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(NormParams p) {
     }
   }
   ss = row16_sum(ss);
-  if (LANES == 64) ss = xor32_sum(xor16_sum(ss));
+  if (LANES >= 64) ss = xor32_sum(xor16_sum(ss));
+  if constexpr (LANES > 64) {
+    __shared__ float s_sum[LANES / 64];
+    if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = ss;
+    __syncthreads();  // one row per workgroup: no thread has left
+    ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < LANES / 64; ++w) ss += s_sum[w];
+  }
   const float rstd = rsqrtf(ss / static_cast<float>(p.cols) + p.eps);
 #pragma unroll
   for (int i = 0; i < MAXC; ++i) {
@@ -104,9 +122,10 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(NormParams p) {
 
 template <int LANES, int MAXC>
 void launch_norm(const NormParams& p, hipStream_t stream) {
-  const int rows_per_block = kThreads / LANES;
+  constexpr int threads = LANES > 64 ? LANES : kThreads;
+  const int rows_per_block = threads / LANES;
   const int grid = (p.num_rows + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL((rmsnorm_kernel<LANES, MAXC>), dim3(grid), dim3(kThreads), 0, stream, p);
+  hipLaunchKernelGGL((rmsnorm_kernel<LANES, MAXC>), dim3(grid), dim3(threads), 0, stream, p);
 }
 
 // ------------------------------------------------------------------ q/k norm + RoPE + append
@@ -145,7 +164,10 @@ struct QkParams {
 // and each wave normalises one head per row instead of several in sequence (measured for
 // one token: 6.3 us with NB = 8).
 
-constexpr int kQkWideTokens = 2048;  // token count from which NB = 4 is used
+// Head rows from which NB = 4 is used.  In rows, not tokens: what fills the chip is waves, and
+// 56 rows per token (40 + 8 + 8 heads) fill it with fewer tokens than 32.  1500 x 56 rows: NB = 1
+// 11.5 us, NB = 4 10.7; 600 x 56 rows: 6.45 against 7.38.
+constexpr int kQkWideRows = 65536;
 
 template <int NB>
 __global__ __launch_bounds__(kThreads) void qk_norm_rope_append_kernel(QkParams p) {
@@ -639,17 +661,19 @@ extern "C" int kvp_rmsnorm_bf16(const void* x, int64_t x_stride0, int64_t x_stri
   auto s = static_cast<hipStream_t>(stream);
   const int nch = cols / 8;
   if (nch <= 16) launch_norm<16, 1>(p, s);
+  else if (nch <= 128 && rows < kNormManyRows) launch_norm<128, 1>(p, s);
   else if (nch <= 128) launch_norm<64, 2>(p, s);
-  else if (nch <= 256) launch_norm<64, 4>(p, s);
-  else if (nch <= 512) launch_norm<64, 8>(p, s);
-  else launch_norm<64, 16>(p, s);
+  else if (nch <= 256) launch_norm<256, 1>(p, s);
+  else if (nch <= 512) launch_norm<256, 2>(p, s);
+  else if (nch <= 768) launch_norm<256, 3>(p, s);
+  else launch_norm<512, 2>(p, s);
   return launch_status("rmsnorm_kernel");
 }
 
 // Prefill-sized inputs: 4 head rows per 16-lane row (two waves per token for Qwen3);
 // decode-sized ones: one head row per 16-lane row, several waves per token.
 static int launch_qk(const QkParams& p, hipStream_t s) {
-  const bool wide = p.num_tokens >= kQkWideTokens;
+  const bool wide = static_cast<int64_t>(p.num_tokens) * p.rows >= kQkWideRows;
   const int nb = wide ? 4 : 1;
   const int64_t groups = (p.rows + 4 * nb - 1) / (4 * nb);
   const int64_t waves = static_cast<int64_t>(p.num_tokens) * groups;

@@ -240,3 +240,22 @@ def test_greedy_argmax_tiny_vocab(cuda_device, vocab):
     got = greedy_argmax(buf.to(cuda_device)[:, :vocab]).cpu()
     assert torch.equal(got, ref.greedy(logits))
     assert got[1].item() == vocab - 1
+
+
+@pytest.mark.parametrize("cols", [136, 1016, 1024, 1032, 2048, 2056, 4096, 4104, 5120, 6144, 6152, 8192])
+def test_norm_at_the_edges_of_its_row_shapes(cuda_device, cols):
+    """The widths around which a row's lanes change, in place, with and without a residual, on
+    few rows and on the many from which narrow rows take one wave each."""
+    g = torch.Generator().manual_seed(cols)
+    for rows in (1, 7) + ((8192,) if cols in (136, 1024) else ()):
+        x, r, w = _randn(rows, cols, gen=g), _randn(rows, cols, gen=g), _randn(cols, gen=g)
+        plain = x.to(cuda_device)
+        rms_norm(plain, w.to(cuda_device), EPS, out=plain)
+        res = r.to(cuda_device)
+        got, _ = add_rms_norm(x.to(cuda_device), res, w.to(cuda_device), EPS)
+        torch.cuda.synchronize()
+        want, want_res = ref.add_rms_norm(x, r, w, EPS)
+        assert torch.equal(res.cpu(), want_res)
+        # two roundings to bf16 (2^-9 each) of a value whose fp32 sum is in another order
+        torch.testing.assert_close(got.cpu().float(), want.float(), atol=1e-3, rtol=1e-2)
+        torch.testing.assert_close(plain.cpu().float(), ref.rms_norm(x, w, EPS).float(), atol=1e-3, rtol=1e-2)
