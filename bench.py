@@ -776,7 +776,7 @@ def summarize_prefill_pmc(dir_a: str, dir_b: str, dir_c: str) -> int:
     import csv
     from collections import defaultdict
 
-    name = "void kvp::varlen_prefill_kernel<2, true, true>"
+    name = "void kvp::varlen_prefill_kernel<2, true, true, false>"
     vals = defaultdict(lambda: defaultdict(float))
     agent = {}
     for d in (dir_a, dir_b, dir_c):
@@ -861,12 +861,12 @@ def summarize_prefill_pmc(dir_a: str, dir_b: str, dir_c: str) -> int:
 
 # (profile file, kernel-name prefix, which occurrence group, algorithmic bytes or flops, unit)
 PROFILE_KERNELS = [
-    ("paged_decode_qwen3_0.6b", "void kvp::paged_decode_kernel<2, 32, false>", "decode_0.6b"),
-    ("paged_decode_fused_qwen3_0.6b", "void kvp::paged_decode_kernel<2, 32, true>", "decode_fused_0.6b"),
-    ("paged_decode_qwen3_8b", "void kvp::paged_decode_kernel<4, 32, false>", "decode_8b"),
+    ("paged_decode_qwen3_0.6b", "void kvp::paged_decode_kernel<2, false>", "decode_0.6b"),
+    ("paged_decode_fused_qwen3_0.6b", "void kvp::paged_decode_kernel<2, true>", "decode_fused_0.6b"),
+    ("paged_decode_qwen3_8b", "void kvp::paged_decode_kernel<4, false>", "decode_8b"),
     ("kv_append_4096tok", "void kvp::kv_append_kernel<128", "append"),
-    ("varlen_prefill_prefix_32seq", "void kvp::varlen_prefill_kernel<2, true, true>", "prefill"),
-    ("varlen_prefill_dense_32seq", "void kvp::varlen_prefill_kernel<2, false, true>", "prefill_dense"),
+    ("varlen_prefill_prefix_32seq", "void kvp::varlen_prefill_kernel<2, true, true, false>", "prefill"),
+    ("varlen_prefill_dense_32seq", "void kvp::varlen_prefill_kernel<2, false, true, false>", "prefill_dense"),
     ("qk_norm_rope_append_16384tok", "void kvp::(anonymous namespace)::qk_norm_rope_append_kernel<4>", "qk_norm_rope_append"),
     ("add_rmsnorm_16384x1024", "void kvp::(anonymous namespace)::rmsnorm_kernel<64, 2>", "add_rmsnorm"),
     ("silu_mul_16384x3072", "kvp::(anonymous namespace)::silu_mul_kernel", "silu_mul"),

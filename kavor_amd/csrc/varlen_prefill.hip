@@ -29,6 +29,8 @@
 //   claim them in that order from per-XCD counters, so the most expensive sequences start
 //   first, a sequence's query tiles run together and stream its K/V through one XCD's L2,
 //   and the cheap ones fill in behind them.
+//   A batch of few query tiles on long keys is cut along the keys as well, so that it fills
+//   the chip (prefill_split_plan_kernel).
 #include <math.h>
 
 #include <algorithm>
