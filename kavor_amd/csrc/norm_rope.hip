@@ -11,7 +11,7 @@
 //
 // All are HBM / latency bound elementwise work: every thread moves 16-byte vectors of 8
 // bf16, reductions stay in registers (DPP inside a 16-lane row, lane swaps across rows),
-// nothing goes through LDS except the argmax's cross-wave step.  Numerics follow the
+// nothing goes through LDS except the cross-wave step of the argmax and of a wide row's sum.  Numerics follow the
 // reference's eager formulas: statistics in fp32, the normalised value rounded to bf16
 // before the weight multiply (double rounding, layernorm.py:32-33), RoPE rotated in fp32
 // and rounded once.
