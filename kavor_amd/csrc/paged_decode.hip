@@ -177,6 +177,9 @@ __device__ __forceinline__ void fill_row(const DecodeParams& p, int b, int ctx) 
                               o % kDecodeHeadDim) = make_uint4(w, w, w, w);
 }
 
+// Keeps a load whose value is not used.
+__device__ __forceinline__ void keep(int x) { asm volatile("" ::"v"(x)); }
+
 // s_ctx[b] = context length, s_cum[b] = steps of sequences 0..b-1 (b = 0..num_seqs), built by
 // the whole workgroup: each thread sums a contiguous run of sequences, then the 256 run
 // totals are scanned with DPP within each wave and the 4 wave totals through LDS.
@@ -185,10 +188,7 @@ __device__ __forceinline__ void build_step_prefix(const DecodeParams& p, int* s_
   const int B = p.num_seqs;
   const int per = (B + kDecodeThreads - 1) / kDecodeThreads;
   const int j0 = tid * per, j1 = min(j0 + per, B);
-  // the first entry of each block-table row, so that the table read that waits for the
-  // lengths finds its line in L2
   int warm = 0;
-  if (tid < B) warm = p.block_tables[tid * p.bt_stride];
   const int wg = blockIdx.y * gridDim.x + blockIdx.x, wgs = gridDim.x * gridDim.y;
   int local = 0;
 #pragma unroll 1
@@ -198,8 +198,10 @@ __device__ __forceinline__ void build_step_prefix(const DecodeParams& p, int* s_
     s_ctx[b] = ctx;
     local += steps;
     if (steps == 0 && b % wgs == wg) fill_row(p, b, ctx);
+    // the first entry of a sequence's block-table row, so that the table read behind the
+    // prefix finds its line in L2; no entry is read of a row without steps
+    if (steps > 0 && per == 1) warm = p.block_tables[b * p.bt_stride];
   }
-  asm volatile("" ::"v"(warm));
   const int lane = tid & 63, wave = tid >> 6;
   const int incl = wave_incl_scan(local);
   if (lane == 63) s_part[wave] = incl;
@@ -215,6 +217,7 @@ __device__ __forceinline__ void build_step_prefix(const DecodeParams& p, int* s_
     run += seq_steps(s_ctx[b], p);
   }
   if (tid == kDecodeThreads - 1) s_cum[B] = before + incl;
+  keep(warm);
   __syncthreads();
 }
 
