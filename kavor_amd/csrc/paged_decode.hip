@@ -648,6 +648,15 @@ void paged_decode_kernel(const DecodeParams p) {
     wait_lds();
   };
 
+  // The rows of V past a sequence's end repeat its last token (see issue_tile); their weights
+  // are 0, but 0 times an infinity is not: they are cleared.  (finish_new clears its own.)
+  auto clear_past = [&](int nv, u32 tile) {
+#pragma unroll 1
+    for (int row = q4; row < kStep; row += 4)
+      if (row >= nv) write_tile16(tile + kTileBytes + 256 * row + 16 * n, make_uint4(0, 0, 0, 0));
+    wait_lds();
+  };
+
   // The loop.  Iteration S computes step S and issues the tiles of step S + 2; the first two
   // iterations (S < S0) only issue.  c0, c1, c2: cursors of steps S, S + 1, S + 2.  Loads
   // complete in issue order, which is, per iteration: what the sequence end at step S + 1
@@ -671,8 +680,9 @@ void paged_decode_kernel(const DecodeParams p) {
     if (seq_end || new_q) {
       if (has1) wait_vmem<16>();  // all but the tiles of S + 1
       else wait_vmem<0>();
-      if constexpr (FUSED) {
-        if (seq_end) finish_new(c0, nv0, tile);
+      if (seq_end) {
+        if constexpr (FUSED) finish_new(c0, nv0, tile);
+        else if (nv0 < kStep) clear_past(nv0, tile);
       }
       if (new_q) finish_q(c1.ctx, qn);
     } else if (live) {

@@ -102,3 +102,21 @@ def test_infinite_values_stay_infinite(cuda_device, G):
     assert torch.all(out[0, :G, 5] == float("inf")) and torch.all(out[0, G:, 77] == float("-inf"))
     fin = torch.isfinite(want)
     torch.testing.assert_close(out[fin], want[fin], **TOL)
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 5, 8])
+def test_infinity_in_the_last_token(cuda_device, G):
+    """Rows of a step past the context carry weight 0; an infinity in the context's last token
+    stays that infinity in its own dim and touches no other, from both entry points."""
+    hkv, bs, ctxs = 2, 64, [1, 17, 31, 32, 33, 48, 63, 64, 80, 129]
+    hq = G * hkv
+    host, d = fused_case(cuda_device, 820 + G, hq, hkv, bs, ctxs)
+    v = host["qkv"].view(len(ctxs), hq + 2 * hkv, 128)[:, hq + hkv:]
+    v[:, 0, 9], v[:, 1, 100] = float("inf"), float("-inf")
+    d["qkv"].copy_(host["qkv"])
+    d2 = {k: t.clone() for k, t in d.items()}
+    for out in (_separate(d, hq, hkv, bs), _fused(d2, hq, hkv, bs)):
+        out = out.cpu().float()
+        want = torch.zeros(out.shape)
+        want[:, :G, 9], want[:, G:, 100] = float("inf"), float("-inf")
+        assert torch.equal(torch.where(torch.isfinite(out), 0.0, out), want)
