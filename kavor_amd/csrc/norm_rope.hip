@@ -59,7 +59,9 @@ template <int LANES, int MAXC>
 __global__ __launch_bounds__(LANES > 64 ? LANES : kThreads) void rmsnorm_kernel(NormParams p) {
   constexpr int THREADS = LANES > 64 ? LANES : kThreads;
   const int lane = threadIdx.x % LANES;
-  const int row = (blockIdx.x * THREADS + threadIdx.x) / LANES;
+  // LANES > 64: the rows go over a two-dimensional grid, since a dimension counts its
+  // threads in 32 bits (2^24 rows of 256 threads reach that)
+  const int row = LANES > 64 ? blockIdx.y * gridDim.x + blockIdx.x : (blockIdx.x * THREADS + threadIdx.x) / LANES;
   if (row >= p.num_rows) return;  // uniform across the lanes of a row
   const int t = row / p.rows_inner, h = row - t * p.rows_inner;
   const uint16_t* xr = p.x + t * p.x_s0 + h * p.x_s1;
@@ -124,8 +126,10 @@ template <int LANES, int MAXC>
 void launch_norm(const NormParams& p, hipStream_t stream) {
   constexpr int threads = LANES > 64 ? LANES : kThreads;
   const int rows_per_block = threads / LANES;
-  const int grid = (p.num_rows + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL((rmsnorm_kernel<LANES, MAXC>), dim3(grid), dim3(threads), 0, stream, p);
+  const int blocks = (p.num_rows + rows_per_block - 1) / rows_per_block;
+  constexpr int kMostX = 1 << 22;  // times 512 threads: 2^31
+  const int y = LANES > 64 ? (blocks + kMostX - 1) / kMostX : 1;
+  hipLaunchKernelGGL((rmsnorm_kernel<LANES, MAXC>), dim3((blocks + y - 1) / y, y), dim3(threads), 0, stream, p);
 }
 
 // ------------------------------------------------------------------ q/k norm + RoPE + append

@@ -259,3 +259,20 @@ def test_norm_at_the_edges_of_its_row_shapes(cuda_device, cols):
         # two roundings to bf16 (2^-9 each) of a value whose fp32 sum is in another order
         torch.testing.assert_close(got.cpu().float(), want.float(), atol=1e-3, rtol=1e-2)
         torch.testing.assert_close(plain.cpu().float(), ref.rms_norm(x, w, EPS).float(), atol=1e-3, rtol=1e-2)
+
+
+def test_norm_of_more_rows_than_a_grid_dimension_counts_threads(cuda_device):
+    """2^24 + 5 rows at one workgroup of 256 threads each: 2^32 threads and more.  The input rows
+    overlap (8 elements apart) to stay small; the output (35 GB) holds every row on its own."""
+    rows, cols = (1 << 24) + 5, 1032
+    x = torch.randn(8 * (rows - 1) + cols, device=cuda_device, dtype=torch.bfloat16).as_strided((rows, cols), (8, 1))
+    w = torch.randn(cols, device=cuda_device, dtype=torch.bfloat16)
+    out = torch.full((rows, cols), float("nan"), device=cuda_device, dtype=torch.bfloat16)
+    rms_norm(x, w, 1e-6, out=out)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(out[:, 0]).all())
+    some = torch.tensor([0, 1, (1 << 22) - 1, 1 << 22, (1 << 24) - 1, 1 << 24, rows - 1], device=cuda_device)
+    want = rms_norm(x[some].contiguous(), w, 1e-6)
+    assert torch.equal(out[some].view(torch.int16), want.view(torch.int16))
+    del out
+    torch.cuda.empty_cache()
