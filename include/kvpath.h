@@ -80,9 +80,10 @@ int kvp_append_bf16(const void* key, int64_t key_tok_stride, int64_t key_head_st
  * batch's step prefix sums and the fp32 partial states of sequences that the
  * work split divides: at most (ranges + sequences) states per query head, with at most
  * 1024 ranges per launch, whatever the context lengths (Qwen3-0.6B, 512 sequences:
- * 12.8 MB).  Small batches are cut into ranges of one 32-token step where the workspace
- * holds their states, which the size for four times max_blocks_per_seq always does, and
- * into ranges of 128 tokens otherwise: the same results within rounding, only slower.
+ * 12.8 MB).  kvp_paged_decode_bf16 cuts a batch the same way in any workspace of this size
+ * or more.  kvp_paged_decode_fused_bf16 cuts a small batch into more ranges, down to one
+ * 32-token step each, where the workspace holds their states, which the size for four times
+ * max_blocks_per_seq always does: the same results within rounding, only faster.
  * Returns 0 for arguments the decode does not support.
  */
 size_t kvp_decode_workspace_bytes(int32_t max_num_seqs, int32_t num_q_heads, int32_t head_dim,
@@ -157,9 +158,7 @@ int kvp_paged_decode_fused_bf16(const void* qkv, int64_t qkv_tok_stride,
  * ends), so the call allocates nothing and needs no caller buffer.  No counterpart in
  * the reference: it is for callers that cannot allocate device memory (code under
  * hipGraph capture, tight serving loops, harnesses that forbid hipMalloc).  Same
- * arguments, semantics and results as kvp_paged_decode_bf16 (bit for bit where that has a
- * workspace of kvp_decode_workspace_bytes for the call's own shape; a larger one may cut a
- * small batch finer).  A batch
+ * arguments, semantics and results as kvp_paged_decode_bf16 (bit for bit).  A batch
  * whose partial states do not fit (about (R + num_seqs) * num_q_heads * 520 bytes, where
  * R is the launch's range count: one workgroup per CU divided by ceil(num_kv_heads / 4), so
  * 128 with 8 kv heads and up to 256 with 4 or fewer on MI355X; Qwen3-0.6B at 512 sequences

@@ -77,9 +77,9 @@ constexpr int kDecodeWaves = 4;  // kv heads per workgroup
 constexpr int kDecodeThreads = 64 * kDecodeWaves;
 constexpr int kStep = 32;               // tokens per step
 constexpr int kTileBytes = kStep * 256;  // one K or V tile
-// A range covers at least one step.  The workspace formula counts ranges of 128 tokens, so a
-// workspace of just that size may be too small for a narrow block table's one-step ranges;
-// then a range covers at least 128 tokens.  A small batch wants the shortest ranges, because
+// The workspace formula counts the ranges a launch may have: one per 128 tokens of its block
+// tables.  The kernel cuts the actual steps into that many ranges, so a table wider than its
+// contexts gives shorter ones, down to one step.  A small batch wants the shortest, because
 // its waves run their steps one after the other while most CUs idle: per call, one sequence
 // of 611 tokens 15.0 us with 128-token ranges, 12.2 us with one-step ranges; 37 sequences of
 // 17-118 tokens 20.9 and 12.5 us.  A large batch is split by the grid and sees no difference.
@@ -124,8 +124,7 @@ struct DecodeParams {
   int32_t num_kv_heads;
   int32_t block_size;
   int32_t max_blocks;
-  int32_t min_steps;  // least steps of a range
-  float scale_log2;   // softmax_scale * log2(e)
+  float scale_log2;  // softmax_scale * log2(e)
   uint16_t* out;
   int64_t o_seq_stride, o_head_stride;
   int32_t* header;  // [0] steps per range, [kHeaderInts ..] step prefix sums (B + 1)
@@ -538,7 +537,7 @@ void paged_decode_kernel(const DecodeParams p) {
   build_step_prefix(p, s_cum, s_ctx, s_part);
   const int B = p.num_seqs;
   const int total_steps = __builtin_amdgcn_readfirstlane(s_cum[B]);  // uniform, and a scalar
-  const int spr = max(p.min_steps, div_by(total_steps + static_cast<int>(gridDim.y) - 1, p.div_ranges));
+  const int spr = max(1, div_by(total_steps + static_cast<int>(gridDim.y) - 1, p.div_ranges));
   if (blockIdx.x == 0 && blockIdx.y == 0) {  // for the merge kernel
     if (tid == 0) p.header[0] = spr;
     for (int b = tid; b <= B; b += kDecodeThreads) p.header[kHeaderInts + b] = s_cum[b];
@@ -974,21 +973,19 @@ static int check_decode_args(const char* fn, const DecodeArgs& a) {
   return KVP_OK;
 }
 
-// How the batch is cut: the ranges of its first (largest) launch and the least steps of one.
-// One-step ranges where `capacity` bytes hold their states, else ranges of 128 tokens.
-struct Split {
-  int64_t ranges;
-  int min_steps;
-};
+// The ranges of the batch's first (largest) launch: no more than workgroups resident at once,
+// nor than the workspace formula counts, so that the plain decode cuts a batch the same way,
+// and gives the same bits, whatever workspace it has.  The one-launch step takes a range for
+// every step of its tables where `capacity` bytes hold their states.
 template <bool FUSED = false>
-static Split batch_split(const DecodeArgs& a, int64_t capacity) {
+static int64_t batch_ranges(const DecodeArgs& a, int64_t capacity = 0) {
   const int nb = std::min(a.num_seqs, kSeqsPerLaunch);
   const int64_t max_tokens = static_cast<int64_t>(nb) * a.max_blocks_per_seq * a.block_size;
   const int64_t groups = (a.num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
   const int64_t most = std::max<int64_t>(1, resident_for<FUSED>(a.num_q_heads / a.num_kv_heads) / groups);
   const int64_t fine = std::min(most, range_cap(max_tokens, kStep));
-  if (decode_workspace_need(nb, a.num_q_heads, fine) <= capacity) return Split{fine, 1};
-  return Split{std::min(most, range_cap(max_tokens, kWorkspaceRangeTokens)), kWorkspaceRangeTokens / kStep};
+  if (FUSED && decode_workspace_need(nb, a.num_q_heads, fine) <= capacity) return fine;
+  return std::min(most, range_cap(max_tokens, kWorkspaceRangeTokens));
 }
 
 // Enqueues the decode of a checked batch on `s` with `ws` as workspace (ws_bytes must
@@ -996,10 +993,9 @@ static Split batch_split(const DecodeArgs& a, int64_t capacity) {
 // the LDS prefix table run as consecutive launches of up to 1024 sequences; they reuse
 // the workspace in stream order.
 template <bool FUSED>
-static int enqueue_decode(const char* fn, const DecodeArgs& a, const Split& split, char* ws, hipStream_t s,
+static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, char* ws, hipStream_t s,
                           const DecodeParams* fused = nullptr) {
   const int G = a.num_q_heads / a.num_kv_heads;
-  const int64_t ranges = split.ranges;
   for (int b0 = 0; b0 < a.num_seqs; b0 += kSeqsPerLaunch) {
     const int nb = std::min(kSeqsPerLaunch, a.num_seqs - b0);
     DecodeParams p = fused ? *fused : DecodeParams{};
@@ -1026,7 +1022,6 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, const Split& spli
     p.num_kv_heads = a.num_kv_heads;
     p.block_size = a.block_size;
     p.max_blocks = a.max_blocks_per_seq;
-    p.min_steps = split.min_steps;
     p.div_block = divisor(static_cast<uint32_t>(a.block_size));
     p.scale_log2 = a.softmax_scale * 1.4426950408889634f;
     p.out = static_cast<uint16_t*>(a.out) + b0 * a.out_seq_stride;
@@ -1130,7 +1125,7 @@ extern "C" int kvp_paged_decode_bf16(const void* q, int64_t q_seq_stride, int64_
     return fail(KVP_EWORKSPACE, "%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, need);
   if (reinterpret_cast<uintptr_t>(workspace) & 255u)
     return fail(KVP_EINVAL, "%s: workspace must be 256-byte aligned", fn);
-  return enqueue_decode<false>(fn, a, batch_split(a, static_cast<int64_t>(workspace_bytes)), static_cast<char*>(workspace),
+  return enqueue_decode<false>(fn, a, batch_ranges(a), static_cast<char*>(workspace),
                                static_cast<hipStream_t>(stream));
 }
 
@@ -1155,11 +1150,8 @@ extern "C" int kvp_paged_decode_bf16_noalloc(const void* q, int64_t q_seq_stride
   int rc = check_decode_args(fn, a);
   if (rc != KVP_OK) return rc;
   if (num_seqs == 0) return KVP_OK;
-  // cut as with a workspace of the formula's size, so that both entry points agree bit for bit
-  const int64_t formula =
-      decode_workspace_bound(std::min(num_seqs, kHeaderSeqs), num_q_heads, max_blocks_per_seq, block_size);
-  const Split split = batch_split(a, formula);
-  const int64_t need = decode_workspace_need(std::min(num_seqs, kHeaderSeqs), num_q_heads, split.ranges);
+  const int64_t ranges = batch_ranges(a);
+  const int64_t need = decode_workspace_need(std::min(num_seqs, kHeaderSeqs), num_q_heads, ranges);
   if (need > static_cast<int64_t>(kScratchBytes))
     return fail(KVP_EWORKSPACE,
                 "%s: %d sequences x %d query heads need %lld bytes of decode scratch; the static scratch "
@@ -1168,7 +1160,7 @@ extern "C" int kvp_paged_decode_bf16_noalloc(const void* q, int64_t q_seq_stride
   char* ws = nullptr;
   rc = scratch_address(fn, static_cast<hipStream_t>(stream), &ws);
   if (rc != KVP_OK) return rc;
-  return enqueue_decode<false>(fn, a, split, ws, static_cast<hipStream_t>(stream));
+  return enqueue_decode<false>(fn, a, ranges, ws, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int kvp_paged_decode_fused_bf16(
@@ -1223,6 +1215,6 @@ extern "C" int kvp_paged_decode_fused_bf16(
   f.eps = eps;
   f.slot_mapping = slot_mapping;
   f.num_cache_slots = static_cast<int64_t>(num_cache_blocks) * block_size;
-  return enqueue_decode<true>(fn, a, batch_split<true>(a, static_cast<int64_t>(workspace_bytes)), static_cast<char*>(workspace),
-                              static_cast<hipStream_t>(stream), &f);
+  return enqueue_decode<true>(fn, a, batch_ranges<true>(a, static_cast<int64_t>(workspace_bytes)),
+                              static_cast<char*>(workspace), static_cast<hipStream_t>(stream), &f);
 }

@@ -51,12 +51,12 @@ def _args(d, out):
             ctypes.c_float(SCALE), out.data_ptr(), out.stride(0), out.stride(1)]
 
 
-def _workspace_call(dev, d):
+def _workspace_call(dev, d, times=1):
     lib = _lib.lib()
     B, hq, D = d["q"].shape
     bs, width = d["kc"].shape[1], d["bt"].shape[1]
     out_ws = torch.empty((B, hq, D), dtype=torch.bfloat16, device=dev)
-    nbytes = lib.kvp_decode_workspace_bytes(B, hq, D, width, bs)
+    nbytes = times * lib.kvp_decode_workspace_bytes(B, hq, D, width, bs)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     rc = lib.kvp_paged_decode_bf16(*_args(d, out_ws), ws.data_ptr(), nbytes,
                                    torch.cuda.current_stream(dev).cuda_stream)
@@ -103,6 +103,21 @@ def test_noalloc_decode_gqa_shapes(cuda_device, B, hq, hkv, bs, lo, hi):
     host, d = _inputs(cuda_device, 33 + hq + hkv, B=B, hq=hq, hkv=hkv, bs=bs, lo=lo, hi=hi)
     got, want = _run_both(cuda_device, d)
     assert bits_equal(got, want)
+    oracle = ref.paged_decode(host["q"], host["kc"], host["vc"], host["bt"], host["ctx"], SCALE)
+    torch.testing.assert_close(got.float(), oracle, **TOL)
+
+
+@pytest.mark.parametrize("B,hq,hkv,lo,hi", [(1, 16, 8, 611, 611), (37, 16, 8, 17, 118), (2, 64, 8, 3000, 4000),
+                                            (8, 40, 8, 600, 3000)])
+def test_decode_gives_the_same_bits_in_any_workspace(cuda_device, B, hq, hkv, lo, hi):
+    """A batch is cut by its shape, not by the bytes at hand: a workspace of the stated size,
+    larger ones and the static scratch give the same output.  The batches are small, where
+    more room could hold more ranges."""
+    host, d = _inputs(cuda_device, 60 + B, B=B, hq=hq, hkv=hkv, bs=256, lo=lo, hi=hi)
+    got, want = _run_both(cuda_device, d)
+    assert bits_equal(got, want)
+    for times in (2, 4, 20):
+        assert bits_equal(_workspace_call(cuda_device, d, times), want)
     oracle = ref.paged_decode(host["q"], host["kc"], host["vc"], host["bt"], host["ctx"], SCALE)
     torch.testing.assert_close(got.float(), oracle, **TOL)
 
