@@ -126,8 +126,9 @@ def reserve_decode_workspace(max_num_seqs: int, num_q_heads: int, head_dim: int,
             raise RuntimeError(
                 "the paged-decode workspace must be reserved before graph capture "
                 f"({nbytes} bytes needed): call reserve_decode_workspace() first")
-        if ws is not None:
+        if ws is not None:  # at least double, so that all that is retired is less than what is held
             _retired_workspaces.append(ws)
+            nbytes = max(nbytes, 2 * ws.numel())
         ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
         _workspaces[dev.index] = ws
     return ws
