@@ -20,6 +20,7 @@ import torch
 from torch import nn
 
 from kavor_amd._lib import check, lib
+from kavor_amd.layers.workspace import Workspaces, retired
 from kavor_amd.utils.context import get_context
 
 __all__ = [
@@ -92,10 +93,9 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
 
 # ----------------------------------------------------------------------------- decode
 
-_workspaces: dict[int, torch.Tensor] = {}
-# Outgrown workspaces are kept, never freed: a graph captured before the growth still
-# launches the decode on the old buffer, and freed memory would be handed to new tensors.
-_retired_workspaces: list[torch.Tensor] = []
+_decode_workspaces = Workspaces("paged-decode", "reserve_decode_workspace")
+_workspaces = _decode_workspaces.default
+_retired_workspaces = retired
 
 
 @lru_cache(maxsize=1024)  # arithmetic on the sizes
@@ -108,35 +108,20 @@ def decode_workspace_bytes(max_num_seqs: int, num_q_heads: int, head_dim: int,
 def reserve_decode_workspace(max_num_seqs: int, num_q_heads: int, head_dim: int,
                              max_blocks_per_seq: int, block_size: int,
                              device: torch.device | str | int) -> torch.Tensor:
-    """Allocates (or grows) the per-device decode workspace.  Call before graph capture
-    with the largest batch a captured graph will use; an eager call that needs more grows
-    the workspace without freeing the one the graphs hold.  It holds the states of
-    one-step (32-token) ranges, four times as many as kvp_decode_workspace_bytes counts
-    for the same block table: a small batch runs faster in them."""
-    nbytes = decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim, 4 * max_blocks_per_seq, block_size)
-    dev = torch.device(device) if not isinstance(device, int) else torch.device("cuda", device)
-    if dev.index is None:
-        dev = torch.device("cuda", torch.cuda.current_device())
-    ws = _workspaces.get(dev.index)
-    if ws is None or ws.numel() < nbytes:
-        if torch.cuda.is_current_stream_capturing():
-            least = decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim, max_blocks_per_seq, block_size)
-            if ws is not None and ws.numel() >= least:
-                return ws  # enough for longer ranges
-            raise RuntimeError(
-                "the paged-decode workspace must be reserved before graph capture "
-                f"({nbytes} bytes needed): call reserve_decode_workspace() first")
-        if ws is not None:  # at least double, so that all that is retired is less than what is held
-            _retired_workspaces.append(ws)
-            nbytes = max(nbytes, 2 * ws.numel())
-        ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
-        _workspaces[dev.index] = ws
-    return ws
+    """Allocates (or grows) the current stream's decode workspace on a device.  Call before graph
+    capture with the largest batch a captured graph will use: the capture takes the buffer over,
+    and eager calls, which need no reservation, go on in another.  It holds the states of
+    one-step (32-token) ranges, four times as many as kvp_decode_workspace_bytes counts for the
+    same block table: the one-launch step runs a small batch faster in them."""
+    return _decode_workspaces.get(
+        device, decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim, 4 * max_blocks_per_seq, block_size),
+        decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim, max_blocks_per_seq, block_size))
 
 
 # ----------------------------------------------------------------------------- prefill workspace
 
-_prefill_workspaces: dict[int, torch.Tensor] = {}
+_prefill_pool = Workspaces("prefill", "reserve_prefill_workspace")
+_prefill_workspaces = _prefill_pool.default
 
 
 @lru_cache(maxsize=1024)
@@ -151,29 +136,15 @@ def _prefill_split_bytes(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num
 
 def reserve_prefill_workspace(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int,
                               device: torch.device | str | int) -> torch.Tensor:
-    """Allocates (or grows) the per-device prefill workspace: the work list of a launch and
-    the partial states of a batch whose keys are split
+    """Allocates (or grows) the current stream's prefill workspace on a device: the work list of a
+    launch and the partial states of a batch whose keys are split
     (kvp_prefill_split_workspace_bytes).  A caller that captures prefill into a graph reserves
-    the largest batch first; an eager call that needs more grows the workspace without
-    freeing the one a graph holds."""
+    the largest batch first: the capture takes the buffer over, and eager calls, which need no
+    reservation, go on in another."""
     nbytes = _prefill_split_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads)
-    dev = torch.device(device) if not isinstance(device, int) else torch.device("cuda", device)
-    if dev.index is None:
-        dev = torch.device("cuda", torch.cuda.current_device())
-    ws = _prefill_workspaces.get(dev.index)
-    if ws is None or ws.numel() < nbytes:
-        if torch.cuda.is_current_stream_capturing():
-            if ws is not None and ws.numel() >= prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads):
-                return ws  # enough without the partial states
-            raise RuntimeError(
-                "the prefill workspace must be reserved before graph capture "
-                f"({nbytes} bytes needed): call reserve_prefill_workspace() first")
-        if ws is not None:
-            _retired_workspaces.append(ws)
-        # a power of two, so that batches of growing size retire few buffers
-        ws = torch.empty(1 << (nbytes - 1).bit_length(), dtype=torch.uint8, device=dev)
-        _prefill_workspaces[dev.index] = ws
-    return ws
+    # a power of two, so that batches of growing size allocate few buffers
+    return _prefill_pool.get(device, 1 << max(0, nbytes - 1).bit_length(),
+                             prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
 
 
 def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,

@@ -15,6 +15,7 @@ from __future__ import annotations
 import torch
 
 from kavor_amd._lib import check, lib
+from kavor_amd.layers.workspace import Workspaces
 
 __all__ = ["rms_norm", "add_rms_norm", "qk_norm_rope_append", "qk_norm_rope", "silu_and_mul",
            "greedy_argmax"]
@@ -178,24 +179,16 @@ def silu_and_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None) -> torc
     return out
 
 
-_argmax_workspaces: dict[int, torch.Tensor] = {}
+_argmax_pool = Workspaces("argmax", "argmax_workspace")
 # The largest split-row workspace any batch needs (fewer than 192 rows, up to 16 segments
-# of one 8-byte key each, at most 1024 keys); reserved once per device.
+# of one 8-byte key each, at most 1024 keys).
 _ARGMAX_WORKSPACE_BYTES = 16384
 
 
 def argmax_workspace(device: torch.device) -> torch.Tensor:
-    """The per-device workspace of the split-row argmax, allocated on first use (which the
-    engine makes before any graph capture)."""
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    ws = _argmax_workspaces.get(index)
-    if ws is None:
-        if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError("the argmax workspace must be reserved before graph capture: "
-                               "call argmax_workspace(device) first")
-        ws = torch.empty(_ARGMAX_WORKSPACE_BYTES, dtype=torch.uint8, device=torch.device("cuda", index))
-        _argmax_workspaces[index] = ws
-    return ws
+    """The current stream's workspace of the split-row argmax on a device, allocated on first use
+    (which the engine makes before any graph capture)."""
+    return _argmax_pool.get(device, _ARGMAX_WORKSPACE_BYTES)
 
 
 def greedy_argmax(logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
