@@ -270,12 +270,20 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const Prefil
 // the same keys at about the same time.  A tile of one chunk writes its output directly.
 // The chunk length C is the one of least estimated cost, in key tiles: the longest unit
 // where every unit has a workgroup slot (two per CU), otherwise the mean load of a slot and
-// half the longest unit (units go out longest first), plus the partial states' traffic
-// (66 KB written and read each, about 1/48 key tile) and the merge.
+// half the longest unit (units go out longest first), but no less than the K/V of all
+// sequences take to arrive (some 300 key tiles of a kv head in the time of one), plus the
+// partial states' traffic (66 KB written and read each, about 1/48 key tile) and the merge.
+// Without the bound by arrival, 32 sequences of 60 new tokens on 2048 (16q/8kv) were cut in
+// two: 81 -> 93 us.
 // Measured against the uncut launch, whole calls with the append: 3 sequences of 17-300 new
 // tokens on 2048-8192 cached (32q/8kv) 156 -> 64 us; 32 new on 4096 (16q/8kv) 83 -> 32 us; 4 of
 // 200-700 on 500-3000 81 -> 60 us; one prompt of 2000 without a prefix 60 -> 46 us, of 3000
 // 82 -> 69 us.
+// Neighbouring tiles of a sequence rank side by side, as the pairs of the uncut launch do, so
+// that two workgroups of an XCD read their keys at the same time (32 sequences of 100 new
+// tokens on 2048, nothing cut: 100.0 us with the tiles apart, 93.8 side by side, 89.6 uncut).
+// A plan that cuts nothing costs 3 to 4 us over the uncut launch's plan, most of it the launch
+// of a merge that finds no work.
 // A unit: s, tile, q start, q length, k start, k length, first key tile | end << 16 (-1: all
 // key tiles, and the tiles tile_slots apart), partial slot (-1: none).
 // A merge: tile, q start, q length, first partial slot, parts.
@@ -288,9 +296,11 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
   __shared__ int hist[kSplitLevels];
   __shared__ int s_n[kSplitTiles], s_nm[kSplitTiles];  // key tiles of a tile, and of its sequence
   __shared__ int s_cost[kCandidates];
-  __shared__ int s_longest;
+  __shared__ int s_longest, s_keys;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int J = p.tile_slots, T = p.num_seqs * J;
+  // A thread's tiles are neighbours of one sequence: an odd count of tile slots is made even
+  // where the table holds it.
+  const int J = p.tile_slots, E = (J & 1) && p.num_seqs * (J + 1) <= kSplitTiles ? J + 1 : J, T = p.num_seqs * E;
   const int slots = kSplitTiles / p.num_kv_heads, most = kSplitItems / p.num_kv_heads;  // T <= slots
   int flip = 0;
   // exclusive prefix sum over the threads and the total (a barrier; the buffers alternate)
@@ -312,16 +322,16 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
     return before;
   };
   if (tid < 8) p.ws[kClaimStride * tid] = 0;
-  if (tid == 0) s_longest = 1;
+  if (tid == 0) s_longest = 1, s_keys = 0;
   if (tid < kCandidates) s_cost[tid] = 0x7fffffff;
   for (int i = tid; i < kSplitLevels; i += kPlanThreads) hist[i] = 0;
   int sq[U], ti[U], q0[U], ql[U], k0[U], kl[U], n[U], nm[U];
-  int work = 0, longest = 1;
+  int work = 0, longest = 1, keys = 0;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int idx = U * tid + u;
-    sq[u] = idx / J;
-    ti[u] = idx - sq[u] * J;
+    sq[u] = idx / E;
+    ti[u] = idx - sq[u] * E;
     q0[u] = ql[u] = k0[u] = kl[u] = n[u] = 0;
     nm[u] = 1;
     if (idx < T) {
@@ -331,7 +341,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
       kl[u] = p.cu_k[sq[u] + 1] - k0[u];
     }
     const int nt = (ql[u] + TOK - 1) / TOK;
-    if (idx < T && ti[u] < nt) {
+    if (idx < T && ti[u] < min(nt, J)) {
       const int end = min(kl[u], min(ql[u], (ti[u] + 1) * TOK) + kl[u] - ql[u]);  // keys the tile sees
       n[u] = max(1, (end + kKeyTile - 1) / kKeyTile);
       nm[u] = max(1, (kl[u] + kKeyTile - 1) / kKeyTile);
@@ -339,14 +349,18 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
     }
     s_n[idx] = n[u];
     s_nm[idx] = nm[u];
+    if (n[u] > 0 && ti[u] == 0) keys += nm[u];  // once per sequence
     work += n[u];
     longest = max(longest, nm[u]);
   }
   __syncthreads();
   if (longest > 1) atomicMax(&s_longest, longest);
+  if (keys > 0) atomicAdd(&s_keys, keys);
   u32 total;
   scan(static_cast<u32>(work), total);
   longest = __builtin_amdgcn_readfirstlane(s_longest);
+  // the time in which all K/V arrive, in key tiles (sequences x kv heads <= 512, of 2^15 each)
+  const int arrive = __builtin_amdgcn_readfirstlane(s_keys) * p.num_kv_heads / 300;
   // chunks of a tile at chunk length C: the sequence's keys in equal chunks of at most C
   auto chunk_of = [](int nm, int C) { const int k = (nm + C - 1) / C; return (nm + k - 1) / k; };
   // Candidates for C: half the longest, then down by quarters while C stays above a quarter
@@ -365,14 +379,15 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
       const int sum = __builtin_amdgcn_readlane(wave_incl_scan(packed), 63);
       const int units = sum & 0xffff, partial = sum >> 16;
       const int cost =
-          (units <= slots ? C : static_cast<int>(total) / slots + C / 2) + partial * p.num_kv_heads / 48 + 4;
+          max(arrive, units <= slots ? C : static_cast<int>(total) / slots + C / 2) +
+          partial * p.num_kv_heads / 48 + 4;
       if (lane == 0 && units <= most) s_cost[k] = cost;
     }
   }
   __syncthreads();
   int C = longest;
   {
-    int best_cost = longest, c = (longest + 1) / 2;
+    int best_cost = max(longest, arrive), c = (longest + 1) / 2;
     for (int k = 0; k < kCandidates && c >= floor_c; ++k, c -= max(1, c >> 2)) {
       const int cost = __builtin_amdgcn_readfirstlane(s_cost[k]);
       if (cost < best_cost) {
@@ -388,13 +403,21 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
     cs[u] = chunk_of(nm[u], C);
     np[u] = (n[u] + cs[u] - 1) / cs[u];
     mine += static_cast<u32>(np[u]);
-    if (np[u] > 1) {
-      mine += (static_cast<u32>(np[u]) << 11) + (1u << 22);
-      // the tile's units by length: np - 1 of cs key tiles, and the rest
-      atomicAdd(&hist[min(cs[u], kSplitLevels - 1)], np[u] - 1);
-    }
-    if (np[u] > 0) atomicAdd(&hist[min(n[u] - (np[u] - 1) * cs[u], kSplitLevels - 1)], 1);
+    if (np[u] > 1) mine += (static_cast<u32>(np[u]) << 11) + (1u << 22);
   }
+  // Chunk i of the thread's two tiles, which read the same keys if they are of one sequence,
+  // ranks as one entry at the longer one's length, so that neighbours are claimed one after the
+  // other.  The first `full` entries are of the chunk length, one placement for all of them (a
+  // tile without chunks has n = np = 0).
+  static_assert(U == 2, "two tiles per thread");
+  auto chunk_len = [&](int u, int i) { return i < np[u] ? min(n[u] - i * cs[u], cs[u]) : 0; };
+  auto level = [&](int i) { return min(max(chunk_len(0, i), chunk_len(1, i)), kSplitLevels - 1); };
+  const int chunks = max(np[0], np[1]);
+  auto whole = [&](int u) { return np[u] * cs[u] == n[u] ? np[u] : np[u] - 1; };  // chunks of the chunk length
+  const int full = !np[0] || !np[1] || cs[0] == cs[1] ? max(whole(0), whole(1)) : 0;
+  const int full_units = min(np[0], full) + min(np[1], full);
+  if (full > 0) atomicAdd(&hist[level(0)], full_units);
+  for (int i = full; i < chunks; ++i) atomicAdd(&hist[level(i)], (i < np[0]) + (i < np[1]));
   u32 sums;
   const u32 mark = scan(mine, sums);
   int slot = static_cast<int>(mark >> 11) & 0x7ff, mat = static_cast<int>(mark >> 22);
@@ -417,19 +440,27 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
   }
   __syncthreads();
   int* const list = p.split + kSplitUnitsInt;
+  int first[U];  // partial slots
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    if (np[u] > 1) {
-      int* const m = p.split + kSplitMergesInt + kUnitInts * mat++;
-      *reinterpret_cast<int4*>(m) = make_int4(ti[u], q0[u], ql[u], slot);
-      m[4] = np[u];
-    }
-    for (int i = 0; i < np[u]; ++i) {
+    first[u] = slot;
+    if (np[u] <= 1) continue;
+    int* const m = p.split + kSplitMergesInt + kUnitInts * mat++;
+    *reinterpret_cast<int4*>(m) = make_int4(ti[u], q0[u], ql[u], slot);
+    m[4] = np[u];
+    slot += np[u];
+  }
+  int at = full > 0 ? atomicAdd(&hist[level(0)], full_units) : 0;
+  for (int i = 0; i < chunks; ++i) {
+    if (i >= full) at = atomicAdd(&hist[level(i)], (i < np[0]) + (i < np[1]));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i >= np[u]) continue;
       const int t0 = i * cs[u], t1 = min(n[u], t0 + cs[u]);
-      const int at = atomicAdd(&hist[min(t1 - t0, kSplitLevels - 1)], 1);
       *reinterpret_cast<int4*>(list + kUnitInts * at) = make_int4(sq[u], ti[u], q0[u], ql[u]);
       *reinterpret_cast<int4*>(list + kUnitInts * at + 4) =
-          make_int4(k0[u], kl[u], np[u] > 1 ? t0 | (t1 << 16) : -1, np[u] > 1 ? slot++ : -1);
+          make_int4(k0[u], kl[u], np[u] > 1 ? t0 | (t1 << 16) : -1, np[u] > 1 ? first[u] + i : -1);
+      ++at;
     }
   }
   if (tid == 0) {
@@ -1015,8 +1046,8 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(const Pr
   constexpr int D = kPrefillHeadDim;
   constexpr int TOK = kPrefillRows / G;
   const int hk = blockIdx.x >> 2, quarter = blockIdx.x & 3;  // rows 32 quarter .. + 31
+  if (hk >= __builtin_amdgcn_readfirstlane(p.split[1]) * p.num_kv_heads) return;
   const int e = hk / p.num_kv_heads, kvh = hk - e * p.num_kv_heads;
-  if (e >= p.split[1]) return;
   const int lane = threadIdx.x & 63, mb = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int* cut = p.split + kSplitMergesInt + kUnitInts * e;
   const int np = __builtin_amdgcn_readfirstlane(cut[4]);

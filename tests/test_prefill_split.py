@@ -61,6 +61,34 @@ def _run(dev, q, k, v, bt, cq, ck, max_q, small=False):
     return out.cpu()
 
 
+def _launch(dev, q, k, v, bt, cq, ck, max_q, split=True):
+    """The C entry point in a workspace with or without the split area: the output, and the
+    split plan's units and cut tiles (None: the launch was not a split one)."""
+    lib = _lib.lib()
+    n, (Tq, hq, D), hkv = cq.numel() - 1, q.shape, k.shape[-2]
+    plain = lib.kvp_prefill_workspace_bytes(n, max_q, hq, hkv)
+    size = lib.kvp_prefill_split_workspace_bytes(n, max_q, hq, hkv) if split else plain
+    ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=dev)
+    q, k, v, cq, ck = (t.to(dev) for t in (q, k, v, cq, ck))
+    out = torch.empty_like(q)
+    if bt is None:
+        ks, vs, table = (0, k.stride(0), k.stride(1)), (0, v.stride(0), v.stride(1)), (0, 0, 0, 0, 0)
+    else:
+        bt = bt.to(dev)
+        ks, vs = k.stride()[:3], v.stride()[:3]
+        table = bt.data_ptr(), bt.stride(0), k.shape[0], k.shape[1], bt.shape[1]
+    _lib.check("prefill", lib.kvp_varlen_prefill_bf16(
+        q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), *ks, v.data_ptr(), *vs, *table, cq.data_ptr(),
+        ck.data_ptr(), n, max_q, hq, hkv, D, SCALE, 1, out.data_ptr(), out.stride(0), out.stride(1), ws.data_ptr(),
+        size, torch.cuda.current_stream(dev).cuda_stream))
+    torch.cuda.synchronize()
+    at = -(-plain // 256) * 256  # the split area: unit and cut counts, from int 64 the units, 8 ints each
+    area = ws[at:at + 4 * (64 + 8 * 1024)].view(torch.int32).tolist() if split else [-1]
+    if area[0] < 0:
+        return out.cpu(), None, None
+    return out.cpu(), [area[64 + 8 * i:72 + 8 * i] for i in range(area[0] // hkv)], area[1]
+
+
 CASES = [
     # one tile on many keys, one row past a tile, a tile of one row; chunks off block borders
     (2, 8, 256, [64], [4000]), (2, 8, 64, [65], [1500]), (4, 8, 192, [1], [3000]),
@@ -167,3 +195,32 @@ def test_smaller_workspace_is_accepted_inside_a_capture(cuda_device):
         attention._prefill_workspaces.pop(d.index, None)
         if kept is not None:
             attention._prefill_workspaces[d.index] = kept
+
+
+@pytest.mark.parametrize("qlens,prefixes", [([128] * 8, [1024] * 8), ([100] * 16, [1024] * 16),
+                                            ([700, 690, 650, 700], [512] * 4), ([120, 1900], [64, 0])])
+def test_neighbouring_tiles_rank_side_by_side(cuda_device, qlens, prefixes):
+    """Tiles 2j and 2j + 1 of a sequence, and their chunks where they are cut alike, follow each
+    other in the plan's list, as the pairs of an uncut launch do, so that they are claimed one
+    after the other on one XCD and read their keys together."""
+    q, kc, vc, bt, cq, ck = _paged(33, qlens, prefixes, 2, 8, 64)
+    _, units, _ = _launch(cuda_device, q, kc, vc, bt, cq, ck, max(qlens))
+    where = {}
+    for i, (s, tile, _, _, _, _, keys, _) in enumerate(units):
+        where.setdefault((s, tile), {})[-1 if keys < 0 else (keys & 0xFFFF)] = i
+    assert sorted(where) == [(s, t) for s, n in enumerate(qlens) for t in range(-(-n // 64))]
+    for (s, tile), at in where.items():
+        for start, i in at.items():
+            other = where.get((s, tile ^ 1), {})
+            if start in other:
+                assert abs(other[start] - i) == 1, (s, tile, start)
+
+
+def test_a_batch_bound_by_its_keys_arrival_is_not_cut(cuda_device):
+    """32 one-tile sequences on 33 key tiles of their own: two chunks each would fit the workgroup
+    slots, but the K/V take longer to arrive than the longest unit to compute."""
+    args = _paged(34, [60] * 32, [2048] * 32, 2, 8, 256)
+    _, units, cuts = _launch(cuda_device, *args, 60)
+    assert cuts == 0 and len(units) == 32
+    _, units, cuts = _launch(cuda_device, *_paged(35, [60] * 8, [2048] * 8, 2, 8, 256), 60)
+    assert cuts == 8 and len(units) > 16
