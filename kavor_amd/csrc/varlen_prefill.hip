@@ -279,9 +279,11 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const Prefil
 // tokens on 2048-8192 cached (32q/8kv) 156 -> 64 us; 32 new on 4096 (16q/8kv) 83 -> 32 us; 4 of
 // 200-700 on 500-3000 81 -> 60 us; one prompt of 2000 without a prefix 60 -> 46 us, of 3000
 // 82 -> 69 us.
-// Neighbouring tiles of a sequence rank side by side, as the pairs of the uncut launch do, so
-// that two workgroups of an XCD read their keys at the same time (32 sequences of 100 new
-// tokens on 2048, nothing cut: 100.0 us with the tiles apart, 93.8 side by side, 89.6 uncut).
+// Where nothing is cut, neighbouring tiles of a sequence rank side by side, as the pairs of the
+// uncut launch do, so that two workgroups of an XCD read their keys at the same time (32
+// sequences of 100 new tokens on 2048: 100.0 us with the tiles apart, 93.8 side by side, 89.6
+// uncut).  Chunks are placed by length alone: in pairs, the 440 of 3 sequences of 17-300 new
+// tokens on 2048-8192 took 64.2 us against 63.4.
 // A plan that cuts nothing costs 3 to 4 us over the uncut launch's plan, most of it the launch
 // of a merge that finds no work.
 // A unit: s, tile, q start, q length, k start, k length, first key tile | end << 16 (-1: all
@@ -405,19 +407,21 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
     mine += static_cast<u32>(np[u]);
     if (np[u] > 1) mine += (static_cast<u32>(np[u]) << 11) + (1u << 22);
   }
-  // Chunk i of the thread's two tiles, which read the same keys if they are of one sequence,
-  // ranks as one entry at the longer one's length, so that neighbours are claimed one after the
-  // other.  The first `full` entries are of the chunk length, one placement for all of them (a
-  // tile without chunks has n = np = 0).
+  // Where nothing is cut, a thread's two tiles rank as one entry at the longer one's length, so
+  // that neighbours are claimed one after the other.
   static_assert(U == 2, "two tiles per thread");
-  auto chunk_len = [&](int u, int i) { return i < np[u] ? min(n[u] - i * cs[u], cs[u]) : 0; };
-  auto level = [&](int i) { return min(max(chunk_len(0, i), chunk_len(1, i)), kSplitLevels - 1); };
-  const int chunks = max(np[0], np[1]);
-  auto whole = [&](int u) { return np[u] * cs[u] == n[u] ? np[u] : np[u] - 1; };  // chunks of the chunk length
-  const int full = !np[0] || !np[1] || cs[0] == cs[1] ? max(whole(0), whole(1)) : 0;
-  const int full_units = min(np[0], full) + min(np[1], full);
-  if (full > 0) atomicAdd(&hist[level(0)], full_units);
-  for (int i = full; i < chunks; ++i) atomicAdd(&hist[level(i)], (i < np[0]) + (i < np[1]));
+  const bool paired = C == longest;  // uniform
+  const int pair_level = min(max(n[0], n[1]), kSplitLevels - 1), pair_units = np[0] + np[1];
+  if (paired) {
+    if (pair_units > 0) atomicAdd(&hist[pair_level], pair_units);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // the tile's units by length: np - 1 of cs key tiles, and the rest
+      if (np[u] > 1) atomicAdd(&hist[min(cs[u], kSplitLevels - 1)], np[u] - 1);
+      if (np[u] > 0) atomicAdd(&hist[min(n[u] - (np[u] - 1) * cs[u], kSplitLevels - 1)], 1);
+    }
+  }
   u32 sums;
   const u32 mark = scan(mine, sums);
   int slot = static_cast<int>(mark >> 11) & 0x7ff, mat = static_cast<int>(mark >> 22);
@@ -440,26 +444,20 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_split_plan_kernel(const 
   }
   __syncthreads();
   int* const list = p.split + kSplitUnitsInt;
-  int first[U];  // partial slots
+  int at = paired && pair_units > 0 ? atomicAdd(&hist[pair_level], pair_units) : 0;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    first[u] = slot;
-    if (np[u] <= 1) continue;
-    int* const m = p.split + kSplitMergesInt + kUnitInts * mat++;
-    *reinterpret_cast<int4*>(m) = make_int4(ti[u], q0[u], ql[u], slot);
-    m[4] = np[u];
-    slot += np[u];
-  }
-  int at = full > 0 ? atomicAdd(&hist[level(0)], full_units) : 0;
-  for (int i = 0; i < chunks; ++i) {
-    if (i >= full) at = atomicAdd(&hist[level(i)], (i < np[0]) + (i < np[1]));
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (i >= np[u]) continue;
+    if (np[u] > 1) {
+      int* const m = p.split + kSplitMergesInt + kUnitInts * mat++;
+      *reinterpret_cast<int4*>(m) = make_int4(ti[u], q0[u], ql[u], slot);
+      m[4] = np[u];
+    }
+    for (int i = 0; i < np[u]; ++i) {
       const int t0 = i * cs[u], t1 = min(n[u], t0 + cs[u]);
+      if (!paired) at = atomicAdd(&hist[min(t1 - t0, kSplitLevels - 1)], 1);
       *reinterpret_cast<int4*>(list + kUnitInts * at) = make_int4(sq[u], ti[u], q0[u], ql[u]);
       *reinterpret_cast<int4*>(list + kUnitInts * at + 4) =
-          make_int4(k0[u], kl[u], np[u] > 1 ? t0 | (t1 << 16) : -1, np[u] > 1 ? first[u] + i : -1);
+          make_int4(k0[u], kl[u], np[u] > 1 ? t0 | (t1 << 16) : -1, np[u] > 1 ? slot++ : -1);
       ++at;
     }
   }

@@ -197,23 +197,20 @@ def test_smaller_workspace_is_accepted_inside_a_capture(cuda_device):
             attention._prefill_workspaces[d.index] = kept
 
 
-@pytest.mark.parametrize("qlens,prefixes", [([128] * 8, [1024] * 8), ([100] * 16, [1024] * 16),
-                                            ([700, 690, 650, 700], [512] * 4), ([120, 1900], [64, 0])])
+@pytest.mark.parametrize("qlens,prefixes", [([250] * 8, [1024] * 8), ([100] * 32, [2048] * 32),
+                                            ([500, 490, 450, 500], [512] * 4), ([1300] * 3, [0] * 3)])
 def test_neighbouring_tiles_rank_side_by_side(cuda_device, qlens, prefixes):
-    """Tiles 2j and 2j + 1 of a sequence, and their chunks where they are cut alike, follow each
-    other in the plan's list, as the pairs of an uncut launch do, so that they are claimed one
-    after the other on one XCD and read their keys together."""
+    """Where the plan cuts nothing, tiles 2j and 2j + 1 of a sequence follow each other in its list,
+    as the pairs of an uncut launch do, so that they are claimed one after the other on one XCD
+    and read their keys together."""
     q, kc, vc, bt, cq, ck = _paged(33, qlens, prefixes, 2, 8, 64)
-    _, units, _ = _launch(cuda_device, q, kc, vc, bt, cq, ck, max(qlens))
-    where = {}
-    for i, (s, tile, _, _, _, _, keys, _) in enumerate(units):
-        where.setdefault((s, tile), {})[-1 if keys < 0 else (keys & 0xFFFF)] = i
-    assert sorted(where) == [(s, t) for s, n in enumerate(qlens) for t in range(-(-n // 64))]
-    for (s, tile), at in where.items():
-        for start, i in at.items():
-            other = where.get((s, tile ^ 1), {})
-            if start in other:
-                assert abs(other[start] - i) == 1, (s, tile, start)
+    _, units, cuts = _launch(cuda_device, q, kc, vc, bt, cq, ck, max(qlens))
+    assert cuts == 0
+    at = {(s, tile): i for i, (s, tile, *_) in enumerate(units)}
+    assert len(at) == len(units) and sorted(at) == [(s, t) for s, n in enumerate(qlens) for t in range(-(-n // 64))]
+    for (s, tile), i in at.items():
+        if (s, tile ^ 1) in at:
+            assert abs(at[s, tile ^ 1] - i) == 1, (s, tile)
 
 
 def test_a_batch_bound_by_its_keys_arrival_is_not_cut(cuda_device):
