@@ -122,6 +122,7 @@ def reserve_decode_workspace(max_num_seqs: int, num_q_heads: int, head_dim: int,
 
 _prefill_pool = Workspaces("prefill", "reserve_prefill_workspace")
 _prefill_workspaces = _prefill_pool.default
+_split_pool = Workspaces("split prefill", "reserve_prefill_workspace")
 
 
 @lru_cache(maxsize=1024)
@@ -131,20 +132,46 @@ def prefill_workspace_bytes(num_seqs: int, max_seqlen_q: int, num_q_heads: int, 
 
 @lru_cache(maxsize=1024)
 def _prefill_split_bytes(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int) -> int:
-    return int(lib().kvp_prefill_split_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
+    nbytes = int(lib().kvp_prefill_split_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
+    return -(-nbytes // (1 << 20)) << 20  # one size for all launches that can be split: their work lists are small
+
+
+# Query tiles x kv heads of a launch that may be split, at most, and keys from which one may be.
+_SPLIT_TILES, _SPLIT_MIN_KEYS = 512, 1024
+
+
+def _may_split(num_seqs: int, max_seqlen_q: int, max_keys: int, num_q_heads: int, num_kv_heads: int) -> bool:
+    """Whether the kernel may cut the keys of such a batch, given room for the partial states."""
+    group = num_q_heads // num_kv_heads if num_kv_heads else 0
+    if max_keys < _SPLIT_MIN_KEYS or group not in (1, 2, 4, 5, 8):
+        return False
+    return 0 < num_seqs * -(-max_seqlen_q // (128 // group)) * num_kv_heads <= _SPLIT_TILES
 
 
 def reserve_prefill_workspace(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int,
                               device: torch.device | str | int) -> torch.Tensor:
-    """Allocates (or grows) the current stream's prefill workspace on a device: the work list of a
-    launch and the partial states of a batch whose keys are split
-    (kvp_prefill_split_workspace_bytes).  A caller that captures prefill into a graph reserves
-    the largest batch first: the capture takes the buffer over, and eager calls, which need no
-    reservation, go on in another."""
-    nbytes = _prefill_split_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads)
+    """Allocates (or grows) the current stream's prefill workspaces on a device: the work list of a
+    launch, which is returned, and the partial states of a batch whose keys are split
+    (kvp_prefill_split_workspace_bytes, 69 MB).  A caller that captures prefill into a graph
+    reserves the largest batch first: the capture takes the buffers over.  Eager calls need no
+    reservation, and hold partial states only once a batch may be split."""
+    _split_pool.get(device, _prefill_split_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
+    return _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, device)
+
+
+def _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, device) -> torch.Tensor:
+    nbytes = prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads)
     # a power of two, so that batches of growing size allocate few buffers
-    return _prefill_pool.get(device, 1 << max(0, nbytes - 1).bit_length(),
-                             prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
+    return _prefill_pool.get(device, 1 << max(4095, nbytes - 1).bit_length(), nbytes)
+
+
+def _prefill_workspace(num_seqs, max_seqlen_q, max_keys, num_q_heads, num_kv_heads, device) -> torch.Tensor:
+    if _may_split(num_seqs, max_seqlen_q, max_keys, num_q_heads, num_kv_heads):
+        ws = _split_pool.get(device, _prefill_split_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads),
+                             optional=True)
+        if ws is not None:  # inside a capture without it the launch is not split
+            return ws
+    return _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, device)
 
 
 def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -264,10 +291,9 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, max_seqlen
     kavor/layers/attention/flash_attention_kvcache.py:76-79: q is [Tq, Hq, D]; with
     block_table None, k / v are [Tk, Hkv, D] rows addressed through cu_seqlens_k; with
     a block_table they are the paged caches [num_blocks, block_size, Hkv, D].  The
-    causal mask is bottom-right aligned.  Returns [Tq, Hq, D] bf16.  max_seqlen_k is
-    accepted for signature compatibility (the kernel reads lengths on the device).
+    causal mask is bottom-right aligned.  Returns [Tq, Hq, D] bf16.  The kernel reads lengths
+    on the device; max_seqlen_k (0 or no int: unknown) only helps to choose the launch.
     """
-    del max_seqlen_k
     Tq, Hq, D = q.shape
     _require_cuda_bf16("q", q)
     _require_cuda_bf16("k", k)
@@ -301,7 +327,12 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, max_seqlen
         bt_ptr, bt_stride, max_blocks = block_table.data_ptr(), block_table.stride(0), block_table.shape[1]
     if k.shape[-1] != D:
         raise ValueError("head_dim mismatch between q and k")
-    ws = reserve_prefill_workspace(num_seqs, int(max_seqlen_q), Hq, Hkv, q.device) if num_seqs else None
+    ws = None
+    if num_seqs:
+        max_keys = max_blocks * block_size if block_table is not None else int(max_seqlen_q)
+        if isinstance(max_seqlen_k, int) and 0 < max_seqlen_k < max_keys:
+            max_keys = max_seqlen_k
+        ws = _prefill_workspace(num_seqs, int(max_seqlen_q), max_keys if causal else 0, Hq, Hkv, q.device)
     rc = lib().kvp_varlen_prefill_bf16(
         q.data_ptr(), q.stride(0), q.stride(1),
         k.data_ptr(), *kstr,

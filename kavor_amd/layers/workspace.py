@@ -29,10 +29,12 @@ class Workspaces:
         self.side: dict[tuple[int, int], torch.Tensor] = {}  # by device and stream handle
         self.captured: dict[int, torch.Tensor] = {}  # by device: the captured graphs'
 
-    def get(self, device: torch.device | str | int, nbytes: int, least: int | None = None) -> torch.Tensor:
+    def get(self, device: torch.device | str | int, nbytes: int, least: int | None = None,
+            optional: bool = False) -> torch.Tensor | None:
         """At least `nbytes` for calls on the device's current stream.  Inside a capture nothing
         is allocated: the largest buffer that the device has becomes the graphs' if it holds
-        `nbytes`, or `least` at least, and the eager calls that used it get another."""
+        `nbytes`, or `least` at least, and the eager calls that used it get another.  Without
+        such a buffer the capture fails, or gets None where the workspace is `optional`."""
         dev = torch.device(device) if not isinstance(device, int) else torch.device("cuda", device)
         i = dev.index if dev.index is not None else torch.cuda.current_device()
         stream = torch._C._cuda_getCurrentRawStream(i)
@@ -40,7 +42,7 @@ class Workspaces:
             ws = self.default.get(i)
             mine = ws is not self.captured.get(i)
         elif torch.cuda.is_current_stream_capturing():
-            return self._for_capture(i, nbytes, nbytes if least is None else least)
+            return self._for_capture(i, nbytes, nbytes if least is None else least, optional)
         else:
             ws = self.side.get((i, stream))
             mine = True
@@ -58,7 +60,7 @@ class Workspaces:
                     self.side.pop(old, None)
         return ws
 
-    def _for_capture(self, i: int, nbytes: int, least: int) -> torch.Tensor:
+    def _for_capture(self, i: int, nbytes: int, least: int, optional: bool) -> torch.Tensor | None:
         own = self.captured.get(i)
         if own is not None and own.numel() >= nbytes:
             return own
@@ -74,5 +76,7 @@ class Workspaces:
             return best
         if own is not None and own.numel() >= least:
             return own
+        if optional:
+            return None
         raise RuntimeError(f"the {self.what} workspace must be reserved before graph capture "
                            f"({nbytes} bytes needed): call {self.reserve}() first")

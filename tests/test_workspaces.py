@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 SCALE = 128 ** -0.5
 
 
-KINDS = (attention._decode_workspaces, attention._prefill_pool, fused._argmax_pool)
+KINDS = (attention._decode_workspaces, attention._prefill_pool, attention._split_pool, fused._argmax_pool)
 
 
 @pytest.fixture
@@ -86,6 +86,46 @@ def test_streams_have_buffers_of_their_own(fresh):
         last = fused.argmax_workspace(d)
         assert len(fused._argmax_pool.side) == workspace._SIDE_STREAMS
         assert fused.argmax_workspace(d).data_ptr() == last.data_ptr()
+
+
+def _prefill(d, num_seqs, new, keys, bs=256, max_seqlen_k=0, causal=True):
+    """An eager prefill of num_seqs sequences, 16 query heads over 8, on one shared prefix."""
+    g = gen(3)
+    kc, vc = (randn_bf16((2, bs, 8, 128), g).to(d) for _ in range(2))
+    bt = torch.zeros(num_seqs, -(-keys // bs), dtype=torch.int32, device=d)
+    cu = torch.arange(num_seqs + 1, dtype=torch.int32, device=d)
+    q = randn_bf16((num_seqs * new, 16, 128), g).to(d)
+    return attention.varlen_prefill(q, kc, vc, new, cu * new, max_seqlen_k, cu * keys, SCALE, causal=causal,
+                                    block_table=bt)
+
+
+def test_partial_states_are_held_only_where_a_batch_may_be_split(fresh):
+    """A launch of too many query tiles, one on few keys (by its table or by the stated length) and
+    one without the causal mask hold a work list alone; the launches that may be split share one
+    buffer of 69 MB."""
+    d, split, lists = fresh, attention._split_pool, attention._prefill_pool
+    _prefill(d, 33, 128, 2048)
+    _prefill(d, 2, 100, 700)
+    _prefill(d, 2, 100, 2048, max_seqlen_k=900)
+    _prefill(d, 2, 100, 2048, causal=False)
+    assert not split.default and lists.default[d.index].numel() <= 16384
+    _prefill(d, 2, 100, 2048)
+    held = split.default[d.index]
+    assert held.numel() <= 70 << 20
+    for n, new, keys in ((1, 1, 1024), (8, 512, 1024), (64, 60, 4096)):
+        _prefill(d, n, new, keys)
+        assert split.default[d.index] is held
+    assert lists.default[d.index].numel() <= 16384
+
+
+@pytest.mark.parametrize("heads", [(4, 8), (24, 8), (256, 1), (8, 0)])
+def test_head_counts_without_a_kernel_are_still_refused(fresh, heads):
+    hq, hkv = heads
+    q = torch.zeros(8, hq, 128, dtype=torch.bfloat16, device=fresh)
+    k = torch.zeros(8, hkv, 128, dtype=torch.bfloat16, device=fresh)
+    cu = torch.tensor([0, 8], dtype=torch.int32, device=fresh)
+    with pytest.raises(RuntimeError, match="kvp_varlen_prefill_bf16"):
+        attention.varlen_prefill(q, k, k, 2000, cu, None, cu, SCALE)
 
 
 def test_a_capture_takes_the_buffer_over(fresh):
