@@ -148,6 +148,46 @@ def _may_split(num_seqs: int, max_seqlen_q: int, max_keys: int, num_q_heads: int
     return 0 < num_seqs * -(-max_seqlen_q // (128 // group)) * num_kv_heads <= _SPLIT_TILES
 
 
+@lru_cache(maxsize=4096)  # the layers of a step share one answer
+def _split_pays(num_seqs: int, total_q: int, max_seqlen_q: int, max_keys: int, num_q_heads: int,
+                num_kv_heads: int) -> bool:
+    """Whether cutting the keys of a batch that may be split is likely to gain, from what the host
+    knows of its lengths.
+
+    The plan kernel decides by the lengths themselves, but a split launch in which it cuts nothing
+    costs 3 to 5 us over an uncut one (its plan, and a merge that finds no work): 4 prompts of
+    1024 tokens (16q/8kv) 45.6 -> 48.7 us, 4 of 700 on 2048 cached 84.8 -> 88.2, 2 of 750 on
+    15000 (32q/8kv) 408 -> 411.  So the plan's cost model runs here on an average tile first.  A
+    batch of about equal new lengths is taken to have equal cached ones, a ragged batch to have
+    0.6 of the longest on average; averages and thresholds are fitted over 900 shapes.  17 of them
+    are slower than uncut, by 4 us each (174 where every batch that may be split takes the split
+    launch); 50 of the 689 that would gain stay uncut, above all equal turns on very unequal
+    histories (4 of 509 tokens on 0 to 16384: 425 us against 301)."""
+    tok = 128 // (num_q_heads // num_kv_heads)
+    slots = _SPLIT_TILES / num_kv_heads
+    even = total_q >= 0.95 * num_seqs * max_seqlen_q
+    longest = -(-max_keys // 64)  # all in key tiles
+    own = max_seqlen_q / 64
+    cached = max(0.0, longest - own)
+    tiles = num_seqs * -(-max_seqlen_q // tok)
+    if not even:
+        tiles = min(tiles, total_q / tok + 0.5 * num_seqs)
+        cached, own = 0.6 * cached, 0.7 * own
+    mean = cached + own / 2
+    arrive = num_seqs * (cached + own) * num_kv_heads / 300
+    least = (1.0 if num_seqs == 1 else 0.95 if even else 0.9) * max(longest, arrive)
+    for parts in (2, 3, 4, 6, 8, 12, 16):
+        chunk = -(-longest // parts)
+        if chunk < 8:
+            break
+        units = tiles * min(parts, mean / chunk + 0.5)
+        busy = chunk if units <= slots else tiles * mean / slots + chunk / 2
+        whole = tiles * min(1.0, max(0.0, chunk - cached) / own)
+        if max(arrive, busy) + (units - whole) * num_kv_heads / 48 + 4 < least:
+            return True
+    return False
+
+
 def reserve_prefill_workspace(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int,
                               device: torch.device | str | int) -> torch.Tensor:
     """Allocates (or grows) the current stream's prefill workspaces on a device: the work list of a
@@ -165,8 +205,9 @@ def _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, device) -> tor
     return _prefill_pool.get(device, 1 << max(4095, nbytes - 1).bit_length(), nbytes)
 
 
-def _prefill_workspace(num_seqs, max_seqlen_q, max_keys, num_q_heads, num_kv_heads, device) -> torch.Tensor:
-    if _may_split(num_seqs, max_seqlen_q, max_keys, num_q_heads, num_kv_heads):
+def _prefill_workspace(num_seqs, total_q, max_seqlen_q, max_keys, num_q_heads, num_kv_heads, device) -> torch.Tensor:
+    if _may_split(num_seqs, max_seqlen_q, max_keys, num_q_heads, num_kv_heads) and \
+            _split_pays(num_seqs, total_q, max_seqlen_q, max_keys, num_q_heads, num_kv_heads):
         ws = _split_pool.get(device, _prefill_split_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads),
                              optional=True)
         if ws is not None:  # inside a capture without it the launch is not split
@@ -332,7 +373,7 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, max_seqlen
         max_keys = max_blocks * block_size if block_table is not None else int(max_seqlen_q)
         if isinstance(max_seqlen_k, int) and 0 < max_seqlen_k < max_keys:
             max_keys = max_seqlen_k
-        ws = _prefill_workspace(num_seqs, int(max_seqlen_q), max_keys if causal else 0, Hq, Hkv, q.device)
+        ws = _prefill_workspace(num_seqs, Tq, int(max_seqlen_q), max_keys if causal else 0, Hq, Hkv, q.device)
     rc = lib().kvp_varlen_prefill_bf16(
         q.data_ptr(), q.stride(0), q.stride(1),
         k.data_ptr(), *kstr,
