@@ -154,15 +154,15 @@ int kvp_paged_decode_fused_bf16(const void* qkv, int64_t qkv_tok_stride,
 
 /*
  * kvp_paged_decode_bf16 without a workspace argument: the decode's partial states live
- * in a static 32 MiB device array of the library (one per GPU, held until the process
+ * in a static 34 MiB device array of the library (one per GPU, held until the process
  * ends), so the call allocates nothing and needs no caller buffer.  No counterpart in
  * the reference: it is for callers that cannot allocate device memory (code under
  * hipGraph capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments, semantics and results as kvp_paged_decode_bf16 (bit for bit).  A batch
  * whose partial states do not fit (about (R + num_seqs) * num_q_heads * 520 bytes, where
  * R is the launch's range count: one workgroup per CU divided by ceil(num_kv_heads / 4), so
- * 128 with 8 kv heads and up to 256 with 4 or fewer on MI355X; Qwen3-0.6B at 512 sequences
- * takes 5.3 MB) returns KVP_EWORKSPACE before any
+ * 128 with 8 kv heads and up to 256 with 4 or fewer on MI355X, and twice that for 512 sequences
+ * or more of as many query heads as kv heads; Qwen3-0.6B at 512 sequences takes 5.3 MB) returns KVP_EWORKSPACE before any
  * launch.  Every call on one GPU shares that GPU's array, so calls that overlap on one
  * GPU (different streams or threads without ordering) race; calls ordered on one
  * stream do not.  The array needs no clearing between calls.  The array's device

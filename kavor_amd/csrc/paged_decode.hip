@@ -11,8 +11,8 @@
 //   Work is counted in steps of 32 tokens of one sequence; the steps of all sequences are
 //   laid end to end (prefix sums of ceil(ctx / 32), built in LDS by every workgroup from
 //   context_lens).  The grid is the number of workgroups the GPU holds at once (one of 4
-//   waves per CU), independent of the batch and of the block-table width, so a captured
-//   graph never launches empty workgroups.  A workgroup's waves are 4 kv heads;
+//   waves per CU; two for many sequences at G = 1, see steps_ahead), and no more than the
+//   block tables can hold steps for, so a captured graph launches few empty workgroups.  A workgroup's waves are 4 kv heads;
 //   ceil(Hkv / 4) workgroups walk one contiguous range of steps for all kv heads (kv heads
 //   of one token row share HBM pages and are fetched together).  Every range gets the same
 //   number of steps (exact balance whatever the context lengths).  A wave owns all
@@ -22,7 +22,7 @@
 // products, their lane sums and the P V products grow with G while the K/V bytes do not.
 // At G = 8 a wave needed more issue cycles for a step than HBM needs to deliver it, and the
 // registers that held the K/V double buffer were short.  Here both products run as
-// v_mfma_f32_16x16x32_bf16 with the G heads as columns, a fixed 24 (G <= 5) or 32 (G = 8)
+// v_mfma_f32_16x16x32_bf16 with the G heads as columns, a fixed 16 (G <= 5) or 24 (G = 8)
 // matrix instructions per step.  Measured against the vector-ALU kernel (MI355X, whole
 // calls, the two in turn): 64 sequences of 1000-9000 tokens at G = 8, one-launch step:
 // 382 -> 215 us (3.4 -> 6.1 TB/s); 128 sequences of 1024-32768 tokens at G = 4: 1300 ->
@@ -32,7 +32,13 @@
 // K and V rows go from memory into the wave's own LDS tiles (32 tokens x 256 bytes, two of
 // each) with direct-to-LDS buffer loads: no register holds them, no barrier is needed, and
 // a tile is refilled as soon as its step has read it, two steps ahead, so 24-32 KiB per
-// wave are in flight all the time.  They are read with the nontemporal hint; rows past the
+// wave are in flight all the time.  Where sequences are short, their starts and ends take
+// longer than their steps: a wave has one SIMD to itself and nothing to hide the vector work
+// behind.  So a sequence's lengths, block id and slot come from lanes (SeqWindow), its q and new
+// token with its first tiles, q and the new k share their norms and rotations, and the waits
+// count what is in flight exactly (see the loop): 4096 sequences of 1-60 tokens, one-launch step,
+// G = 2 223 -> 152 us, G = 1 219 -> 136; 1024 of 10-100 70.7 -> 63.2 and 68.2 -> 55.9; one of
+// 611 tokens, 28 layers 308 -> 292.  They are read with the nontemporal hint; rows past the
 // context are clamped onto its last token (masked in the softmax), so no branch guards a
 // load.
 //
@@ -47,10 +53,11 @@
 // mantissa each), and the 16 columns hold the parts of the G heads side by side (column n:
 // part n / G of head n % G; q is repeated, so every column forms its own part from its own
 // scores).  Three parts fit for G <= 5; G = 8 holds two and adds the third with a second
-// product.  The parts of a head are summed in fp32 when the state is written.  Tile rows are
+// product (8 more instructions).  The parts of a head are summed in fp32 when the state is written.  Tile rows are
 // swizzled by 16-byte chunks, K by row & 15 and V by 2 (row & 7), so neither the 16-byte
 // reads nor the transpose reads share a bank.  Softmax: online, base 2, scale*log2(e)
-// folded into the scores, one running (max, sum) per column and row group.
+// folded into the scores, one running max per column (over all row groups) and a running sum
+// per column and row group.
 //
 // Output: where a wave's range ends or a sequence ends its state is written; a sequence
 // covered by one range gives bf16 directly, otherwise each range writes (max, sum,
@@ -67,6 +74,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "common.h"
 
@@ -84,7 +92,20 @@ constexpr int kTileBytes = kStep * 256;  // one K or V tile
 // of 611 tokens 15.0 us with 128-token ranges, 12.2 us with one-step ranges; 37 sequences of
 // 17-118 tokens 20.9 and 12.5 us.  A large batch is split by the grid and sees no difference.
 constexpr int kWorkspaceRangeTokens = 128;
-constexpr int kSeqsPerLaunch = 1024;  // sequences per launch (LDS tables); more run as consecutive launches
+// Sequences per launch: as many as the step prefix has LDS for beside the tiles of `ahead` steps
+// and the sequences' inputs.  More run as consecutive launches.
+constexpr int seqs_per_launch(int g, bool fused, int ahead) {
+  if (ahead == 1) return 2048;
+  return fused ? (g <= 2 ? 4096 : g <= 5 ? 2048 : 1024) : (g <= 5 ? 4096 : 2048);
+}
+// Steps whose tiles a wave has in flight ahead of the one it computes: two, with one workgroup on
+// a CU; or one, with two workgroups, whose waves compute while the others wait, for batches of
+// many short sequences at G = 1, where a sequence's start and end take longer than its steps.
+// 8q/8kv, one-launch step, two steps ahead against one: 1024 sequences of 1-32 tokens 37.8 and
+// 30.3 us, 1024 of 10-100 59.7 and 55.9, 512 of 100-200 64.0 and 63.1, 1024 of 200-400 214.6 and
+// 215.7; 32 of 200-800 23.4 and 24.4, one of 20000 29.5 and 33.0, 128 of 1024-16384 667 and 673.
+constexpr int kManySeqs = 512;
+static int steps_ahead(int g, int num_seqs) { return g == 1 && num_seqs >= kManySeqs ? 1 : 2; }
 constexpr int kHeaderSeqs = 4096;     // sequences the workspace formula counts at most
 constexpr int64_t kMaxDmaRow = 1 << 24;  // row stride (elements) up to which 32 rows are addressed in 32 bits
 constexpr int kHeaderInts = 16;          // workspace header before the prefix table
@@ -119,7 +140,7 @@ struct DecodeParams {
   const int32_t* block_tables;
   int64_t bt_stride;
   const int32_t* context_lens;
-  int32_t num_seqs;  // <= kSeqsPerLaunch
+  int32_t num_seqs;  // <= seqs_per_launch
   int32_t num_q_heads;
   int32_t num_kv_heads;
   int32_t block_size;
@@ -179,10 +200,10 @@ __device__ __forceinline__ void fill_row(const DecodeParams& p, int b, int ctx) 
 // Keeps a load whose value is not used.
 __device__ __forceinline__ void keep(int x) { asm volatile("" ::"v"(x)); }
 
-// s_ctx[b] = context length, s_cum[b] = steps of sequences 0..b-1 (b = 0..num_seqs), built by
-// the whole workgroup: each thread sums a contiguous run of sequences, then the 256 run
-// totals are scanned with DPP within each wave and the 4 wave totals through LDS.
-__device__ __forceinline__ void build_step_prefix(const DecodeParams& p, int* s_cum, int* s_ctx, int* s_part) {
+// s_cum[b] = steps of sequences 0..b-1 (b = 0..num_seqs), built by the whole workgroup: each
+// thread sums a contiguous run of sequences, then the 256 run totals are scanned with DPP
+// within each wave and the 4 wave totals through LDS.
+__device__ __forceinline__ void build_step_prefix(const DecodeParams& p, int* s_cum, int* s_part) {
   const int tid = threadIdx.x;
   const int B = p.num_seqs;
   const int per = (B + kDecodeThreads - 1) / kDecodeThreads;
@@ -191,15 +212,22 @@ __device__ __forceinline__ void build_step_prefix(const DecodeParams& p, int* s_
   const int wg = blockIdx.y * gridDim.x + blockIdx.x, wgs = gridDim.x * gridDim.y;
   int local = 0;
 #pragma unroll 1
-  for (int b = j0; b < j1; ++b) {
-    const int ctx = p.context_lens[b];
-    const int steps = seq_steps(ctx, p);
-    s_ctx[b] = ctx;
-    local += steps;
-    if (steps == 0 && b % wgs == wg) fill_row(p, b, ctx);
-    // the first entry of a sequence's block-table row, so that the table read behind the
-    // prefix finds its line in L2; no entry is read of a row without steps
-    if (steps > 0 && per == 1) warm = p.block_tables[b * p.bt_stride];
+  for (int b0 = j0; b0 < j1; b0 += 4) {  // four lengths in flight
+    int ctx[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ctx[i] = p.context_lens[min(b0 + i, j1 - 1)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int b = b0 + i;
+      if (b >= j1) break;
+      const int steps = seq_steps(ctx[i], p);
+      s_cum[b] = steps;
+      local += steps;
+      if (steps == 0 && b % wgs == wg) fill_row(p, b, ctx[i]);
+      // the first entry of a sequence's block-table row, so that the table read behind the
+      // prefix finds its line in L2; no entry is read of a row without steps
+      if (steps > 0 && per == 1) warm = p.block_tables[b * p.bt_stride];
+    }
   }
   const int lane = tid & 63, wave = tid >> 6;
   const int incl = wave_incl_scan(local);
@@ -212,8 +240,9 @@ __device__ __forceinline__ void build_step_prefix(const DecodeParams& p, int* s_
   int run = before + incl - local;
 #pragma unroll 1
   for (int b = j0; b < j1; ++b) {
+    const int steps = s_cum[b];
     s_cum[b] = run;
-    run += seq_steps(s_ctx[b], p);
+    run += steps;
   }
   if (tid == kDecodeThreads - 1) s_cum[B] = before + incl;
   keep(warm);
@@ -231,23 +260,50 @@ struct StepCursor {
   int j;        // step within the sequence
   int nsteps;   // steps of sequence b
   int ctx;      // context length of sequence b
+  int slot;     // FUSED: where its new token goes
   int lblk;     // logical block whose id is cached in blk (-1: none)
   int blk;      // physical block id of lblk
   int pf_blk;   // id of block lblk + 1, loaded one block ahead (-1: not loaded)
+  int buf;      // which of the wave's input regions holds the sequence's q
   int bad;      // a needed block id was out of range (an int: the struct copies stay in registers)
+  int mark;     // vector memory operations issued up to the step's K tile (its V tile follows)
 };
 
-// The cursor of step S, which belongs to sequence b.
-__device__ __forceinline__ void cursor_start_seq(StepCursor& cur, const int* s_cum, const int* s_ctx, int b, int S) {
-  const int cum = __builtin_amdgcn_readfirstlane(s_cum[b]);
-  cur.b = b;
-  cur.j = S - cum;
-  cur.ctx = __builtin_amdgcn_readfirstlane(s_ctx[b]);
-  cur.nsteps = __builtin_amdgcn_readfirstlane(s_cum[b + 1]) - cum;
-  cur.lblk = -1;
-  cur.blk = 0;
-  cur.pf_blk = -1;
-  cur.bad = 0;
+// 64 consecutive sequences' metadata, one per lane, so that moving to the next sequence waits for
+// no memory and no LDS: lane i holds sequence base + i.
+struct SeqWindow {
+  int base;
+  uint64_t live;  // the lanes with steps
+  int ctx, blk, slot;  // length, first block id (0 without steps), FUSED: the new token's slot
+};
+template <bool FUSED>
+__device__ __forceinline__ void fill_window(const DecodeParams& p, const int* s_cum, int base, int lane, SeqWindow& w) {
+  const int b = min(base + lane, p.num_seqs - 1);
+  const bool has = base + lane < p.num_seqs && s_cum[b + 1] > s_cum[b];
+  w.base = base;
+  w.live = __ballot(has);
+  w.ctx = p.context_lens[b];
+  w.slot = FUSED ? p.slot_mapping[b] : 0;
+  w.blk = 0;
+  if (has) w.blk = p.block_tables[b * p.bt_stride];
+  // waited for here, so that no later read waits for what has been issued since
+  asm volatile("" : "+v"(w.ctx), "+v"(w.slot), "+v"(w.blk));
+}
+
+// The cursor of the first step of sequence base + i.
+__device__ __forceinline__ void cursor_start_seq(const DecodeParams& p, StepCursor& cur, const SeqWindow& w, int i,
+                                                 int buf) {
+  cur.buf = buf;
+  cur.b = w.base + i;
+  cur.j = 0;
+  cur.ctx = __builtin_amdgcn_readlane(w.ctx, i);
+  cur.slot = __builtin_amdgcn_readlane(w.slot, i);
+  cur.blk = __builtin_amdgcn_readlane(w.blk, i);
+  cur.nsteps = (cur.ctx + kStep - 1) / kStep;
+  cur.lblk = 0;
+  cur.bad = cur.blk < 0 || cur.blk >= p.num_cache_blocks;
+  if (cur.bad) cur.blk = 0;
+  cur.pf_blk = p.block_size < cur.ctx ? load_uniform(p.block_tables + cur.b * p.bt_stride, 1) : -1;
 }
 
 // Element offset of the cursor's step in the caches, and the number of valid tokens of the
@@ -274,13 +330,12 @@ __device__ __forceinline__ int64_t step_base(const DecodeParams& p, StepCursor& 
 
 // ---- fused q/k norm + RoPE + append (FUSED kernels)
 //
-// The inputs of the q of a sequence (its cos/sin row and raw q heads) and of its new token
-// (cos/sin row, raw k and v heads) reach a per-wave LDS region with direct-to-LDS buffer
-// loads one step before they are needed, so the wave never waits on a dependent load chain
-// at a sequence boundary and no VGPR holds them meanwhile.  The token's position is
+// The inputs of a sequence -- its cos/sin row, raw q heads, and its new token's raw k and v heads
+// -- reach one of two per-wave LDS regions with direct-to-LDS buffer loads, issued with the tiles
+// of the sequence's first step, two steps ahead, so the wave never waits on a dependent load
+// chain at a sequence boundary and no VGPR holds them meanwhile.  The token's position is
 // context_lens[b] - 1.
 constexpr int kFzRow = 512;  // bytes: one cos/sin row, 128 fp32
-constexpr int kFzNew = 1024;  // new token: cos/sin row | raw k head | raw v head
 __device__ __forceinline__ BufferRsrc cos_sin_rsrc(const DecodeParams& p) {
   return buffer_rsrc(p.cos_sin, static_cast<uint32_t>(p.max_position) * kFzRow);
 }
@@ -298,33 +353,40 @@ __device__ __forceinline__ void fz_issue_weights(const DecodeParams& p, int lane
   else if (lane < 32) lds_dma16(buffer_rsrc(p.k_weight, 256), 16 * (lane - 16), region);
 }
 
-// q inputs of sequence b (context ctx) for kv head kvh: the cos/sin row at bytes 0-511,
-// then the G q heads.
+// A sequence's region: the cos/sin row (bytes 0-511), the G raw q heads of kv head kvh, the raw k
+// head, the raw v head.  Instruction i of the qkv part fills bytes 1024 i .. + 1023 of the region.
 template <int G>
-__device__ __forceinline__ void fz_issue_q(const DecodeParams& p, int b, int ctx, int kvh, int lane, char* region) {
-  if (lane < 32) lds_dma16(cos_sin_rsrc(p), fz_row_bytes(p, ctx) + 16 * lane, region);
-  const int heads = (b * static_cast<int>(p.qkv_stride) + kvh * G * kRopeDim) * 2;
-#pragma unroll
-  for (int i = 0; i < (kFzRow + G * 256 + 1023) / 1024; ++i) {
-    const int byte = 1024 * i + 16 * lane;  // this lane's destination within the region
-    if (byte >= kFzRow && byte < kFzRow + G * 256) lds_dma16(qkv_rsrc(p), heads + byte - kFzRow, region + 1024 * i);
-  }
+struct FzRegion {
+  static constexpr int kNew = kFzRow + 256 * G;  // where the new token's k and v start
+  static constexpr int kBytes = kNew + 512;
+  static constexpr int kLoads = (kBytes + 1023) / 1024;
+  static constexpr int kOps = 1 + kLoads;  // vector memory operations
+};
+// Byte offset in a qkv row of what the lane loads in instruction i.
+template <int G>
+__device__ __forceinline__ int fz_row_offset(const DecodeParams& p, int kvh, int lane, int i) {
+  const int at = 1024 * i + 16 * lane;
+  const int head = at < FzRegion<G>::kNew         ? kvh * G + (at - kFzRow) / 256
+                   : at < FzRegion<G>::kNew + 256 ? p.num_q_heads + kvh
+                                                  : p.num_q_heads + p.num_kv_heads + kvh;
+  return head * 256 + at % 256;
 }
-
-// New-token inputs of sequence b (context ctx) for kv head kvh: the cos/sin row, then the
-// raw k head (bytes 512-767) and the raw v head (768-1023).
-__device__ __forceinline__ void fz_issue_new(const DecodeParams& p, int b, int ctx, int kvh, int lane, char* region) {
-  if (lane < 32) {
-    lds_dma16(cos_sin_rsrc(p), fz_row_bytes(p, ctx) + 16 * lane, region);
-  } else {
-    const int head = lane < 48 ? p.num_q_heads + kvh : p.num_q_heads + p.num_kv_heads + kvh;
-    lds_dma16(qkv_rsrc(p), (b * static_cast<int>(p.qkv_stride) + head * kRopeDim) * 2 + 16 * (lane & 15), region);
+template <int G>
+__device__ __forceinline__ void fz_issue(const DecodeParams& p, int b, int ctx, const int (&row_at)[FzRegion<G>::kLoads],
+                                         int lane, char* region) {
+  typedef __attribute__((address_space(3))) void* Lds;
+  if (lane < kFzRow / 16) raw_buffer_load_lds(cos_sin_rsrc(p), (Lds)region, 16, 16 * lane, fz_row_bytes(p, ctx), 0, 0);
+  const int row = b * static_cast<int>(p.qkv_stride) * 2;
+#pragma unroll
+  for (int i = 0; i < FzRegion<G>::kLoads; ++i) {
+    const int at = 1024 * i + 16 * lane;
+    if (at >= kFzRow && at < FzRegion<G>::kBytes)
+      raw_buffer_load_lds(qkv_rsrc(p), (Lds)(region + 1024 * i), 16, row_at[i], row, 0, 0);
   }
 }
 
 typedef __bf16 mfma_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float mfma_f32x4_t __attribute__((ext_vector_type(4)));
-
 
 __device__ __forceinline__ mfma_f32x4_t mfma16(u32x4_t a, u32x4_t b, mfma_f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mfma_bf16x8_t, a),
@@ -369,33 +431,33 @@ __device__ __forceinline__ void read_v_tile(const u32 (&a)[8], u32x2_t (&lo)[8],
       : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7])
       : "memory");
 }
-// A head's inputs for norm_rope_head: the lane's norm weights, cos and sin, and two 16-byte
-// chunks x0, x1.
-struct HeadInputs {
-  u32x4_t w, cos[2], sin[2], x0, x1;
-};
-__device__ __forceinline__ HeadInputs read_head(u32 w_at, u32 table_at, u32 x0_at, u32 x1_at) {
-  HeadInputs h;
+// A head's chunk normalised and rotated (chunk c of the head at x_at), by the norm weights at w_at
+// and the cos/sin row at table_at.
+__device__ __forceinline__ uint4 norm_rope_chunk(u32 w_at, u32 table_at, u32 x_at, int c, bool pos_ok, float eps) {
+  u32x4_t hw, hx, hc[2], hs[2];
   asm volatile(
-      "ds_read_b128 %0, %7\n\tds_read_b128 %1, %8\n\tds_read_b128 %2, %8 offset:16\n\t"
-      "ds_read_b128 %3, %8 offset:256\n\tds_read_b128 %4, %8 offset:272\n\t"
-      "ds_read_b128 %5, %9\n\tds_read_b128 %6, %10\n\ts_waitcnt lgkmcnt(0)"
-      : "=&v"(h.w), "=&v"(h.cos[0]), "=&v"(h.cos[1]), "=&v"(h.sin[0]), "=&v"(h.sin[1]), "=&v"(h.x0), "=&v"(h.x1)
-      : "v"(w_at), "v"(table_at), "v"(x0_at), "v"(x1_at)
+      "ds_read_b128 %0, %6\n\tds_read_b128 %1, %8\n\tds_read_b128 %2, %7\n\tds_read_b128 %3, %7 offset:16\n\t"
+      "ds_read_b128 %4, %7 offset:256\n\tds_read_b128 %5, %7 offset:272\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(hw), "=&v"(hx), "=&v"(hc[0]), "=&v"(hc[1]), "=&v"(hs[0]), "=&v"(hs[1])
+      : "v"(w_at), "v"(table_at), "v"(x_at)
       : "memory");
-  return h;
-}
-__device__ __forceinline__ uint4 norm_rope_chunk(const HeadInputs& h, u32x4_t raw, int c, bool pos_ok, float eps) {
   float w[8], x[8], cs[8], sn[8];
-  unpack8(__builtin_bit_cast(uint4, h.w), w);
-  unpack8(__builtin_bit_cast(uint4, raw), x);
+  unpack8(__builtin_bit_cast(uint4, hw), w);
+  unpack8(__builtin_bit_cast(uint4, hx), x);
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    cs[e] = __uint_as_float(h.cos[e >> 2][e & 3]);
-    sn[e] = __uint_as_float(h.sin[e >> 2][e & 3]);
+    cs[e] = __uint_as_float(hc[e >> 2][e & 3]);
+    sn[e] = __uint_as_float(hs[e >> 2][e & 3]);
   }
   norm_rope_head(x, w, cs, sn, c < 8, pos_ok, eps);
   return pack8(x);
+}
+// Two 16-byte chunks.
+__device__ __forceinline__ void read_pair(u32 a, u32 b, u32x4_t& x, u32x4_t& y) {
+  asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(x), "=&v"(y)
+               : "v"(a), "v"(b)
+               : "memory");
 }
 // q of one column in the B layout: 16 bytes at a, a + 64, a + 128, a + 192.
 __device__ __forceinline__ void read_q(u32 a, u32x4_t (&q)[4]) {
@@ -408,6 +470,32 @@ __device__ __forceinline__ void read_q(u32 a, u32x4_t (&q)[4]) {
 }
 __device__ __forceinline__ void write_tile16(u32 addr, uint4 v) {
   asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(__builtin_bit_cast(u32x4_t, v)) : "memory");
+}
+
+// Stores that the waits count: one instruction each.
+template <int OFFSET>
+__device__ __forceinline__ void store8(void* ptr, u32x2_t v) {
+  asm volatile("global_store_dwordx2 %0, %1, off offset:%2" ::"v"(ptr), "v"(v), "n"(OFFSET) : "memory");
+}
+template <int OFFSET>
+__device__ __forceinline__ void store16(void* ptr, u32x4_t v) {
+  asm volatile("global_store_dwordx4 %0, %1, off offset:%2" ::"v"(ptr), "v"(v), "n"(OFFSET) : "memory");
+}
+
+// Waits until at most `most` vector memory operations of the wave are in flight (uniform; rounded
+// down to a multiple of 8).
+__device__ __forceinline__ void wait_upto(int most) {
+  if (most >= 24) {
+    if (most >= 40) wait_vmem<40>();
+    else if (most >= 32) wait_vmem<32>();
+    else wait_vmem<24>();
+  } else if (most >= 16) {
+    wait_vmem<16>();
+  } else if (most >= 8) {
+    wait_vmem<8>();
+  } else {
+    wait_vmem<0>();
+  }
 }
 
 // x of the lane N places up in the 16-lane row (0 past its end).
@@ -451,6 +539,19 @@ __device__ __forceinline__ void issue_tile(const DecodeParams& p, const TileLane
   }
 }
 
+// f(0) .. f(7) with constant arguments.
+template <typename F>
+__device__ __forceinline__ void each8(F f) {
+  f(std::integral_constant<int, 0>{});
+  f(std::integral_constant<int, 1>{});
+  f(std::integral_constant<int, 2>{});
+  f(std::integral_constant<int, 3>{});
+  f(std::integral_constant<int, 4>{});
+  f(std::integral_constant<int, 5>{});
+  f(std::integral_constant<int, 6>{});
+  f(std::integral_constant<int, 7>{});
+}
+
 template <int G>
 struct State {
   float m, l;
@@ -470,13 +571,13 @@ __device__ __forceinline__ void reset_state(State<G>& st) {
 
 // The state of (b, kvh) for this range: the parts of each head summed, then the bf16
 // output when one range covers the sequence, otherwise an fp32 partial.
+// Returns its vector memory operations.
 template <int G>
-__device__ __forceinline__ void emit_state(const DecodeParams& p, int b, int kvh, int slot, bool single, bool bad,
+__device__ __forceinline__ int emit_state(const DecodeParams& p, int b, int kvh, int slot, bool single, bool bad,
                                           int n, int q4, const State<G>& st) {
   float l = xor32_sum(xor16_sum(st.l));
   if (bad) l = NAN;
-  float o[8][4];
-  bool nan = false;
+  float o[8][4], odd = 0.f;  // odd: NaN once a value is not finite
 #pragma unroll
   for (int mt = 0; mt < 8; ++mt) {
 #pragma unroll
@@ -485,10 +586,10 @@ __device__ __forceinline__ void emit_state(const DecodeParams& p, int b, int kvh
       o[mt][j] = a + row_up<G>(a);
       if (G <= 5) o[mt][j] += row_up<2 * (G <= 5 ? G : 1)>(a);
       else o[mt][j] += row_up<G>(st.acc2[mt][j]);
-      nan |= o[mt][j] != o[mt][j];
+      odd = fmaf(o[mt][j], 0.f, odd);
     }
   }
-  if (__any(nan)) {  // an infinite value in V: the first part has the result, the others inf - inf
+  if (__any(odd != odd)) {  // an infinite value in V: the first part has the result, the others inf - inf
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
@@ -498,35 +599,39 @@ __device__ __forceinline__ void emit_state(const DecodeParams& p, int b, int kvh
   if (single) {
     const float inv = 1.f / l;
     uint16_t* out = p.out + b * p.o_seq_stride + h * p.o_head_stride + 4 * q4;
-    if (n < G)
-#pragma unroll
-      for (int mt = 0; mt < 8; ++mt)
-        *reinterpret_cast<uint2*>(out + 16 * mt) =
-            make_uint2(pack_bf16x2(o[mt][0] * inv, o[mt][1] * inv), pack_bf16x2(o[mt][2] * inv, o[mt][3] * inv));
-  } else if (n < G) {
-    const int64_t row = static_cast<int64_t>(slot) * p.num_q_heads + h;
-    float* part = p.part_o + row * kDecodeHeadDim + 4 * q4;
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt)
-      *reinterpret_cast<float4*>(part + 16 * mt) = make_float4(o[mt][0], o[mt][1], o[mt][2], o[mt][3]);
-    if (q4 == 0) *reinterpret_cast<float2*>(p.part_ml + row * 2) = make_float2(st.m, l);
+    auto row = [&](auto mt_c) {
+      constexpr int mt = decltype(mt_c)::value;
+      store8<32 * mt>(out, u32x2_t{pack_bf16x2(o[mt][0] * inv, o[mt][1] * inv),
+                                   pack_bf16x2(o[mt][2] * inv, o[mt][3] * inv)});
+    };
+    if (n < G) each8(row);
+    return 8;
   }
+  const int64_t at = static_cast<int64_t>(slot) * p.num_q_heads + h;
+  float* part = p.part_o + at * kDecodeHeadDim + 4 * q4;
+  auto row = [&](auto mt_c) {
+    constexpr int mt = decltype(mt_c)::value;
+    store16<64 * mt>(part, u32x4_t{__float_as_uint(o[mt][0]), __float_as_uint(o[mt][1]), __float_as_uint(o[mt][2]),
+                                   __float_as_uint(o[mt][3])});
+  };
+  if (n < G) {
+    each8(row);
+    if (q4 == 0) store8<0>(p.part_ml + at * 2, u32x2_t{__float_as_uint(st.m), __float_as_uint(l)});
+  }
+  return 9;
 }
 
-template <int G, bool FUSED>
+template <int G, bool FUSED, int A>
 __global__ __launch_bounds__(kDecodeThreads)
 void paged_decode_kernel(const DecodeParams p) {
-  // per wave: K and V tiles of the steps of either parity
-  __shared__ __attribute__((aligned(16))) char s_tile[kDecodeWaves][2][2 * kTileBytes];
-  // per wave: q heads of the next sequence (FUSED: behind its cos/sin row); FUSED: norm
-  // weights, and cos/sin row, raw k and raw v of the new token
+  // per wave: K and V tiles of the steps in flight, and the inputs of as many sequences (FUSED:
+  // FzRegion, else the G q heads); FUSED: norm weights, which every wave loads (the same bytes)
+  __shared__ __attribute__((aligned(16))) char s_tile[kDecodeWaves][A][2 * kTileBytes];
   constexpr int kQRow = FUSED ? kFzRow : 0;
-  constexpr int kFzWaves = FUSED ? kDecodeWaves : 1;
-  __shared__ __attribute__((aligned(16))) char s_fq[kDecodeWaves][kQRow + 256 * G];
-  __shared__ __attribute__((aligned(16))) char s_fw[kFzWaves][FUSED ? 512 : 16];
-  __shared__ __attribute__((aligned(16))) char s_fn[kFzWaves][FUSED ? kFzNew : 16];
-  __shared__ int s_cum[kSeqsPerLaunch + 1];  // steps of sequences 0 .. b - 1
-  __shared__ int s_ctx[kSeqsPerLaunch];
+  constexpr int kQBytes = FUSED ? FzRegion<G>::kBytes : 256 * G;
+  __shared__ __attribute__((aligned(16))) char s_q[kDecodeWaves][A][kQBytes];
+  __shared__ __attribute__((aligned(16))) char s_fw[FUSED ? 512 : 16];
+  __shared__ int s_cum[seqs_per_launch(G, FUSED, A) + 1];  // steps of sequences 0 .. b - 1
   __shared__ int s_part[kDecodeWaves];
 
   const int tid = threadIdx.x;
@@ -534,7 +639,7 @@ void paged_decode_kernel(const DecodeParams p) {
   const int lane = tid & 63;
   const int n = lane & 15, q4 = lane >> 4;
 
-  build_step_prefix(p, s_cum, s_ctx, s_part);
+  build_step_prefix(p, s_cum, s_part);
   const int B = p.num_seqs;
   const int total_steps = __builtin_amdgcn_readfirstlane(s_cum[B]);  // uniform, and a scalar
   const int spr = max(1, div_by(total_steps + static_cast<int>(gridDim.y) - 1, p.div_ranges));
@@ -557,7 +662,6 @@ void paged_decode_kernel(const DecodeParams p) {
   }
   lo = __builtin_amdgcn_readfirstlane(lo);
   const int64_t head_off = static_cast<int64_t>(kvh) * p.head_stride;
-  const int fw = FUSED ? wave : 0;
   const int hg = n % G;     // this column's head and the part of P it holds
   const int part = n / G;
 
@@ -577,122 +681,132 @@ void paged_decode_kernel(const DecodeParams p) {
 #pragma unroll
   for (int mt = 0; mt < 8; ++mt) va[mt] = kTileBytes + 256 * vrow + 8 * (n & 3) + 32 * (mt ^ (vrow & 7));
 
-  auto seq_after = [&](int b, int S) {  // the first sequence with steps starting at S + 1
-    int nb = b + 1;
-    while (s_cum[nb + 1] == S + 1) ++nb;
-    return __builtin_amdgcn_readfirstlane(nb);
-  };
-
-  // q of a sequence reaches the wave's region one step ahead, then the B layout (column n is
-  // head hg, dims 32 kk + 8 q4 + e).  FUSED: the raw heads are normalised and rotated in
-  // place first (row group r takes heads r, r + 4).
-  auto issue_q = [&](int b, int ctx) {
+  // q of a sequence reaches the wave's region with the tiles of its first step, then the
+  // B layout (column n is head hg, dims 32 kk + 8 q4 + e).  FUSED: the raw heads are normalised
+  // and rotated in place first (row group r takes heads r, r + 4).  Returns the vector memory
+  // operations that the waits may count.
+  int row_at[FUSED ? FzRegion<G>::kLoads : 1] = {};
+  if constexpr (FUSED) {
+#pragma unroll
+    for (int i = 0; i < FzRegion<G>::kLoads; ++i) row_at[i] = fz_row_offset<G>(p, kvh, lane, i);
+  }
+  auto issue_q = [&](const StepCursor& c) {
+    char* region = s_q[wave][c.buf];
     if constexpr (FUSED) {
-      fz_issue_q<G>(p, b, ctx, kvh, lane, s_fq[wave]);
+      fz_issue<G>(p, c.b, c.ctx, row_at, lane, region);
+      return FzRegion<G>::kOps;
     } else {
-      const uint16_t* src = p.q + b * p.q_seq_stride + static_cast<int64_t>(kvh) * G * p.q_head_stride;
+      const uint16_t* src = p.q + c.b * p.q_seq_stride + static_cast<int64_t>(kvh) * G * p.q_head_stride;
 #pragma unroll
       for (int u = 0; u < (G + 3) / 4; ++u) {
         const int g = q4 + 4 * u;
         if (p.q_by_dma) {  // uniform
           const int head_bytes = static_cast<int>(p.q_head_stride) * 2;
           const BufferRsrc rsrc = buffer_rsrc(src, static_cast<uint32_t>((G - 1) * head_bytes + 256));
-          if (g < G) lds_dma16(rsrc, g * head_bytes + 16 * n, s_fq[wave] + 1024 * u);
+          if (g < G) lds_dma16(rsrc, g * head_bytes + 16 * n, region + 1024 * u);
         } else if (g < G) {
-          write_tile16(lds_addr(s_fq[wave]) + 256 * g + 16 * n, load16(src + g * p.q_head_stride + 8 * n));
+          write_tile16(lds_addr(region) + 256 * g + 16 * n, load16(src + g * p.q_head_stride + 8 * n));
         }
       }
+      return p.q_by_dma ? (G + 3) / 4 : 0;
     }
   };
-  const u32 q_at = lds_addr(s_fq[wave]), w_at = lds_addr(s_fw[fw]), new_at = lds_addr(s_fn[fw]);
-  auto finish_q = [&](int ctx, u32x4_t (&dst)[4]) {
-    if constexpr (FUSED) {
-      const bool pos_ok = ctx - 1 >= 0 && ctx - 1 < p.max_position;
-      const int g0 = min(q4, G - 1), g1 = min(q4 + 4, G - 1);
-      const u32 x0_at = q_at + kQRow + 256 * g0 + 16 * n, x1_at = q_at + kQRow + 256 * g1 + 16 * n;
-      const HeadInputs h = read_head(w_at + 16 * n, q_at + 32 * (n & 7), x0_at, x1_at);
-      const uint4 y0 = norm_rope_chunk(h, h.x0, n, pos_ok, p.eps);
-      if (q4 < G) write_tile16(x0_at, y0);
-      if (G > 4) {
-        const uint4 y1 = norm_rope_chunk(h, h.x1, n, pos_ok, p.eps);
-        if (q4 + 4 < G) write_tile16(x1_at, y1);
+  const u32 q_base = lds_addr(s_q[wave][0]), w_at = lds_addr(s_fw);
+  // At a range's first step of a sequence.  `ends`: the sequence's last step is in the range.
+  auto finish_q = [&](const StepCursor& c, bool ends, u32x4_t (&dst)[4]) {
+    const u32 q_at = q_base + kQBytes * c.buf;
+    if constexpr (FUSED) {  // four heads at a time; head G is the new token's k
+      const bool pos_ok = c.ctx - 1 >= 0 && c.ctx - 1 < p.max_position;
+#pragma unroll
+      for (int g0 = 0; g0 <= G; g0 += 4) {
+        if (g0 == G && !ends) break;
+        const int g = min(g0 + q4, G);
+        const u32 x_at = q_at + kQRow + 256 * g + 16 * n;
+        const uint4 y = norm_rope_chunk(w_at + (g == G ? 256 : 0) + 16 * n, q_at + 32 * (n & 7), x_at, n, pos_ok, p.eps);
+        if (g0 + q4 <= G) write_tile16(x_at, y);
       }
     }
     read_q(q_at + kQRow + 256 * hg + 16 * q4, dst);
   };
-  // FUSED: the new token of the sequence that ends at this step: k normalised and rotated,
-  // both rows appended at the slot and put into the step's tiles, where the loads left them
-  // out; the rows past it are cleared, so that no unwritten slot is multiplied.
+  // FUSED: the new token of the sequence that ends at this step: k (normalised and rotated with
+  // q) and v appended at the slot and put into the step's tiles, where the loads left them out;
+  // the rows of V past it are cleared, so that no unwritten slot is multiplied (those of K give
+  // scores that are masked).  Returns the vector memory operations.
   auto finish_new = [&](const StepCursor& c, int nv, u32 tile) {
-    const bool pos_ok = c.ctx - 1 >= 0 && c.ctx - 1 < p.max_position;
-    const int slot = load_uniform(p.slot_mapping, c.b);
-    const HeadInputs h =
-        read_head(w_at + 256 + 16 * n, new_at + 32 * (n & 7), new_at + kFzRow + 16 * n, new_at + kFzRow + 256 + 16 * n);
-    const uint4 knew = norm_rope_chunk(h, h.x0, n, pos_ok, p.eps);
-    const uint4 vnew = __builtin_bit_cast(uint4, h.x1);
-    if (q4 == 0 && slot >= 0 && slot < p.num_cache_slots) {
-      const int blk = slot / p.block_size, off = slot - blk * p.block_size;
+    const u32 new_at = q_base + kQBytes * c.buf + kQRow + 256 * G + 16 * n;
+    u32x4_t knew, vnew;
+    read_pair(new_at, new_at + 256, knew, vnew);
+    int ops = 0;
+    if (c.slot >= 0 && c.slot < p.num_cache_slots) {  // uniform
+      const int blk = div_by(c.slot, p.div_block), off = c.slot - blk * p.block_size;
       const int64_t at = static_cast<int64_t>(blk) * p.blk_stride + static_cast<int64_t>(off) * p.slot_stride +
                          head_off + 8 * n;
-      *reinterpret_cast<uint4*>(const_cast<uint16_t*>(p.k_cache) + at) = knew;
-      *reinterpret_cast<uint4*>(const_cast<uint16_t*>(p.v_cache) + at) = vnew;
+      if (q4 == 0) {
+        store16<0>(const_cast<uint16_t*>(p.k_cache) + at, knew);
+        store16<0>(const_cast<uint16_t*>(p.v_cache) + at, vnew);
+      }
+      ops = 2;
     }
-#pragma unroll 1
-    for (int row = q4; row < kStep; row += 4) {
-      if (row < nv - 1) continue;
-      const uint4 zero = make_uint4(0, 0, 0, 0);
-      write_tile16(tile + 256 * row + 16 * (n ^ (row & 15)), row == nv - 1 ? knew : zero);
-      write_tile16(tile + kTileBytes + 256 * row + 16 * (n ^ (2 * (row & 7))), row == nv - 1 ? vnew : zero);
-    }
+    const int last = nv - 1;
+    if (q4 == 0) write_tile16(tile + 256 * last + 16 * (n ^ (last & 15)), __builtin_bit_cast(uint4, knew));
+    for (int row = (last & ~3) + q4; row < kStep; row += 4)
+      if (row >= last)
+        write_tile16(tile + kTileBytes + 256 * row + 16 * (n ^ (2 * (row & 7))),
+                     row == last ? __builtin_bit_cast(uint4, vnew) : make_uint4(0, 0, 0, 0));
     wait_lds();
+    return ops;
   };
-
   // The rows of V past a sequence's end repeat its last token (see issue_tile); their weights
   // are 0, but 0 times an infinity is not: they are cleared.  (finish_new clears its own.)
   auto clear_past = [&](int nv, u32 tile) {
 #pragma unroll 1
-    for (int row = q4; row < kStep; row += 4)
+    for (int row = (nv & ~3) + q4; row < kStep; row += 4)
       if (row >= nv) write_tile16(tile + kTileBytes + 256 * row + 16 * n, make_uint4(0, 0, 0, 0));
     wait_lds();
   };
 
-  // The loop.  Iteration S computes step S and issues the tiles of step S + 2; the first two
-  // iterations (S < S0) only issue.  c0, c1, c2: cursors of steps S, S + 1, S + 2.  Loads
-  // complete in issue order, which is, per iteration: what the sequence end at step S + 1
-  // needs (q of the sequence after it, FUSED its new token), K of S + 2, V of S + 2; the
-  // first sequence's q goes before the tiles of S0.  The waits count from that order; other
-  // operations in flight (stores) only make them stricter.
-  StepCursor c0{}, c1{}, c2{};
-  int nv0 = 0, nv1 = 0, nv2 = 0;
-  u32x4_t qv[4] = {}, qn[4] = {};
+  // The loop.  Iteration S computes step S and issues the tiles of step S + A, each as soon as its
+  // tile has been read, with the inputs of the sequence before them if it starts one; the first A
+  // iterations (S < S0) only issue.  c[i]: cursor of step S + i.  Vector memory operations
+  // complete in issue order, so the waits count back from the operations issued so far to the
+  // mark of what they need; an operation that is not counted only makes them stricter.
+  StepCursor c[A + 1] = {};
+  StepCursor &c0 = c[0], &cn = c[A];
+  u32x4_t qv[4] = {};
   State<G> st;
   reset_state<G>(st);
-  if (FUSED) fz_issue_weights(p, lane, s_fw[fw]);
-  const u32 tile_base = lds_addr(s_tile[wave][0]);
-  for (int S = S0 - 2; S < S1; ++S) {
-    const int par = (S - S0) & 1;
-    const u32 tile = tile_base + 2 * kTileBytes * par;
-    const bool live = S >= S0, has1 = S + 1 >= S0 && S + 1 < S1, has2 = S + 2 < S1;
+  int issued = 0;
+  const int tile_ops = p.rows_by_dma ? 8 : 0;
+  if (FUSED) fz_issue_weights(p, lane, s_fw);
+  // The first step, from a window that starts at its sequence; its block, if not the sequence's
+  // first, is loaded with the window.
+  const int j0 = S0 - __builtin_amdgcn_readfirstlane(s_cum[lo]);
+  const int lblk0 = div_by(j0 * kStep, p.div_block);
+  int blk0 = 0;
+  if (lblk0 > 0) blk0 = load_uniform(p.block_tables + lo * p.bt_stride, lblk0);
+  SeqWindow win;
+  fill_window<FUSED>(p, s_cum, lo, lane, win);
+  cursor_start_seq(p, cn, win, 0, 0);
+  cn.j = j0;
+  if (lblk0 > 0) {
+    cn.lblk = lblk0 - 1;  // step_base takes the block over as one loaded ahead
+    cn.bad = 0;
+    cn.pf_blk = blk0;
+  }
+  for (int S = S0 - A; S < S1; ++S) {
+    char* const tiles = s_tile[wave][(S - S0) & (A - 1)];
+    const u32 tile = lds_addr(tiles);
+    const bool live = S >= S0, issue = S + A < S1;
     const bool seq_end = live && c0.j + 1 == c0.nsteps;
-    const bool end1 = has1 && c1.j + 1 == c1.nsteps;  // a sequence ends at S + 1
-    const bool new_q = has1 && (!live || seq_end);    // S + 1 starts with another q
-    if (seq_end || new_q) {
-      if (has1) wait_vmem<16>();  // all but the tiles of S + 1
-      else wait_vmem<0>();
-      if (seq_end) {
-        if constexpr (FUSED) finish_new(c0, nv0, tile);
-        else if (nv0 < kStep) clear_past(nv0, tile);
-      }
-      if (new_q) finish_q(c1.ctx, qn);
-    } else if (live) {
-      if (has1) wait_vmem<24>();  // all but this step's V and the tiles of S + 1
-      else wait_vmem<8>();
-    }
-    if (end1) {
-      if (FUSED && live) fz_issue_new(p, c1.b, c1.ctx, kvh, lane, s_fn[fw]);
-      if (has2) {
-        const int nb = seq_after(c1.b, S + 1);
-        issue_q(nb, FUSED ? __builtin_amdgcn_readfirstlane(s_ctx[nb]) : 0);
+    const int nv0 = min(kStep, c0.ctx - c0.j * kStep);
+    const bool starts = S == S0 || c0.j == 0;
+    const bool early_v = seq_end && (FUSED || nv0 < kStep);  // the tile's last rows are rewritten
+    if (live) {
+      wait_upto(issued - c0.mark - (early_v ? tile_ops : 0));
+      if (starts) finish_q(c0, c0.nsteps - c0.j <= S1 - S, qv);
+      if (early_v) {
+        if constexpr (FUSED) issued += finish_new(c0, nv0, tile);
+        else clear_past(nv0, tile);
       }
     }
 
@@ -705,24 +819,31 @@ void paged_decode_kernel(const DecodeParams p) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) s[i & 1] = mfma16(k[i], qv[i >> 1], s[i & 1]);
     }
-    int64_t base2 = 0;
-    int rows2 = 0;
-    if (has2) {  // K has been read: its tile takes step S + 2
-      if (S + 2 == S0) {
-        cursor_start_seq(c2, s_cum, s_ctx, lo, S0);
-        issue_q(c2.b, c2.ctx);
-        if (FUSED && c2.j + 1 == c2.nsteps) fz_issue_new(p, c2.b, c2.ctx, kvh, lane, s_fn[fw]);
-      } else if (c1.j + 1 == c1.nsteps) {
-        cursor_start_seq(c2, s_cum, s_ctx, seq_after(c1.b, S + 1), S + 2);
-      } else {
-        c2 = c1;
-        c2.j = c1.j + 1;
+    int64_t base = 0;
+    int rows = 0;
+    if (issue) {  // K has been read: its tile takes step S + A
+      const StepCursor& prev = c[A - 1];
+      const bool next_seq = S + A != S0 && prev.j + 1 == prev.nsteps;
+      if (next_seq) {
+        int at = prev.b + 1 - win.base;
+        while (at >= 64 || (win.live >> at) == 0) {  // a sequence with steps follows
+          fill_window<FUSED>(p, s_cum, win.base + 64, lane, win);
+          at = 0;
+        }
+        cursor_start_seq(p, cn, win, at + __builtin_ctzll(win.live >> at), A == 2 ? prev.buf ^ 1 : 0);
+      } else if (S + A != S0) {
+        cn = prev;
+        cn.j = prev.j + 1;
       }
-      base2 = step_base(p, c2, head_off, nv2);
+      if (S + A == S0 || next_seq) issued += issue_q(cn);
+      int nv;
+      base = step_base(p, cn, head_off, nv);
       // FUSED: a sequence's final step holds the token this launch appends, whose slot is
       // not written yet; its row is filled by finish_new
-      rows2 = FUSED && c2.j + 1 == c2.nsteps && nv2 > 1 ? nv2 - 1 : nv2;
-      issue_tile<false>(p, ln, base2, rows2, s_tile[wave][par]);
+      rows = FUSED && cn.j + 1 == cn.nsteps && nv > 1 ? nv - 1 : nv;
+      issue_tile<false>(p, ln, base, rows, tiles);
+      issued += tile_ops;
+      cn.mark = issued;
     }
     u32 pk[4] = {}, pk2[4] = {};
     if (live) {
@@ -738,7 +859,7 @@ void paged_decode_kernel(const DecodeParams p) {
       const float m_new = fmaxf(st.m, mx);
       const float alpha = fast_exp2(st.m - m_new);
       st.m = m_new;
-      if (__any(alpha != 1.f)) {
+      if (!starts && __any(alpha != 1.f)) {  // a new state is zero
         st.l *= alpha;
 #pragma unroll
         for (int mt = 0; mt < 8; ++mt) {
@@ -762,9 +883,7 @@ void paged_decode_kernel(const DecodeParams p) {
         if (G > 5) pk2[e >> 1] = pack_bf16x2(w[0], w[1]);
       }
       // ---- O^T += V^T P^T
-      if (has2) wait_vmem<24>();  // all but the tiles of S + 1 and the K tile of S + 2
-      else if (has1) wait_vmem<16>();
-      else wait_vmem<0>();
+      if (!early_v) wait_upto(issued - c0.mark - tile_ops);
       u32x2_t vlo[8], vhi[8];
       const u32 at[8] = {tile + va[0], tile + va[1], tile + va[2], tile + va[3],
                          tile + va[4], tile + va[5], tile + va[6], tile + va[7]};
@@ -777,20 +896,17 @@ void paged_decode_kernel(const DecodeParams p) {
         if (G > 5) st.acc2[mt] = mfma16(vt, pf2, st.acc2[mt]);
       }
     }
-    if (has2) issue_tile<true>(p, ln, base2, rows2, s_tile[wave][par] + kTileBytes);
-    if (seq_end || (live && !has1)) {
+    if (issue) {
+      issue_tile<true>(p, ln, base, rows, tiles + kTileBytes);
+      issued += tile_ops;
+    }
+    if (seq_end || S + 1 == S1) {
       // the whole sequence in this range: it ends here and began here
-      emit_state<G>(p, c0.b, kvh, range + c0.b, seq_end && S + 1 - c0.nsteps >= S0, c0.bad, n, q4, st);
+      issued += emit_state<G>(p, c0.b, kvh, range + c0.b, seq_end && S + 1 - c0.nsteps >= S0, c0.bad, n, q4, st);
       reset_state<G>(st);
     }
-    if (new_q) {
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) qv[kk] = qn[kk];
-    }
-    c0 = c1;
-    nv0 = nv1;
-    c1 = c2;
-    nv1 = nv2;
+    for (int i = 0; i < A; ++i) c[i] = c[i + 1];
   }
 }
 // Combines the per-range partial states of sequences that span several ranges.
@@ -879,9 +995,25 @@ static int64_t decode_workspace_bound(int64_t seqs, int64_t q_heads, int64_t max
   return decode_workspace_need(seqs, q_heads, ranges);
 }
 
+// f(G, A) with constants for a batch of num_seqs sequences at GQA ratio g.
+template <typename F>
+static auto with_variant(int g, int num_seqs, F f) {
+  using std::integral_constant;
+  const integral_constant<int, 2> two;
+  switch (g) {
+    case 1:
+      if (steps_ahead(1, num_seqs) == 1) return f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+      return f(integral_constant<int, 1>{}, two);
+    case 2: return f(integral_constant<int, 2>{}, two);
+    case 4: return f(integral_constant<int, 4>{}, two);
+    case 5: return f(integral_constant<int, 5>{}, two);
+    default: return f(integral_constant<int, 8>{}, two);
+  }
+}
+
 // Workgroups of the kernel resident on the whole current device (cached per device once
 // the queries succeed), capped at kMaxDecodeGrid.
-template <int G, bool FUSED>
+template <int G, bool FUSED, int A>
 static int resident_workgroups() {
   static std::atomic<int> cached[16];
   int dev = 0;
@@ -891,7 +1023,7 @@ static int resident_workgroups() {
   int cus = 0, per_cu = 0;
   bool ok = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0;
   if (!ok) cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, paged_decode_kernel<G, FUSED>, kDecodeThreads, 0) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, paged_decode_kernel<G, FUSED, A>, kDecodeThreads, 0) !=
           hipSuccess || per_cu <= 0) {
     per_cu = 1;
     ok = false;
@@ -901,23 +1033,12 @@ static int resident_workgroups() {
   return v;
 }
 
-template <bool FUSED>
-static int resident_for(int G) {
-  switch (G) {
-    case 1: return resident_workgroups<1, FUSED>();
-    case 2: return resident_workgroups<2, FUSED>();
-    case 4: return resident_workgroups<4, FUSED>();
-    case 5: return resident_workgroups<5, FUSED>();
-    default: return resident_workgroups<8, FUSED>();
-  }
-}
-
-template <int G, bool FUSED>
+template <int G, bool FUSED, int A>
 static void launch_decode(DecodeParams p, int64_t ranges, hipStream_t s) {
   const int64_t groups_per_range = (p.num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
   p.div_ranges = divisor(static_cast<uint32_t>(ranges));
   const dim3 grid(static_cast<unsigned>(groups_per_range), static_cast<unsigned>(ranges));
-  hipLaunchKernelGGL((paged_decode_kernel<G, FUSED>), grid, dim3(kDecodeThreads), 0, s, p);
+  hipLaunchKernelGGL((paged_decode_kernel<G, FUSED, A>), grid, dim3(kDecodeThreads), 0, s, p);
   hipLaunchKernelGGL(decode_merge_kernel, dim3((p.num_q_heads + kMergeHeads - 1) / kMergeHeads, p.num_seqs),
                      dim3(kMergeThreads), 0, s, p);
 }
@@ -979,10 +1100,14 @@ static int check_decode_args(const char* fn, const DecodeArgs& a) {
 // every step of its tables where `capacity` bytes hold their states.
 template <bool FUSED = false>
 static int64_t batch_ranges(const DecodeArgs& a, int64_t capacity = 0) {
-  const int nb = std::min(a.num_seqs, kSeqsPerLaunch);
+  const int g = a.num_q_heads / a.num_kv_heads;
+  const int nb = std::min(a.num_seqs, seqs_per_launch(g, FUSED, steps_ahead(g, a.num_seqs)));
   const int64_t max_tokens = static_cast<int64_t>(nb) * a.max_blocks_per_seq * a.block_size;
   const int64_t groups = (a.num_kv_heads + kDecodeWaves - 1) / kDecodeWaves;
-  const int64_t most = std::max<int64_t>(1, resident_for<FUSED>(a.num_q_heads / a.num_kv_heads) / groups);
+  const int resident = with_variant(g, a.num_seqs, [](auto G, auto A) {
+    return resident_workgroups<decltype(G)::value, FUSED, decltype(A)::value>();
+  });
+  const int64_t most = std::max<int64_t>(1, resident / groups);
   const int64_t fine = std::min(most, range_cap(max_tokens, kStep));
   if (FUSED && decode_workspace_need(nb, a.num_q_heads, fine) <= capacity) return fine;
   return std::min(most, range_cap(max_tokens, kWorkspaceRangeTokens));
@@ -990,14 +1115,15 @@ static int64_t batch_ranges(const DecodeArgs& a, int64_t capacity = 0) {
 
 // Enqueues the decode of a checked batch on `s` with `ws` as workspace (ws_bytes must
 // cover decode_workspace_need of every launch; checked by the callers).  Batches beyond
-// the LDS prefix table run as consecutive launches of up to 1024 sequences; they reuse
-// the workspace in stream order.
+// the LDS prefix table run as consecutive launches of up to seqs_per_launch sequences; they
+// reuse the workspace in stream order.
 template <bool FUSED>
 static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, char* ws, hipStream_t s,
                           const DecodeParams* fused = nullptr) {
-  const int G = a.num_q_heads / a.num_kv_heads;
-  for (int b0 = 0; b0 < a.num_seqs; b0 += kSeqsPerLaunch) {
-    const int nb = std::min(kSeqsPerLaunch, a.num_seqs - b0);
+  const int g = a.num_q_heads / a.num_kv_heads;
+  const int most = seqs_per_launch(g, FUSED, steps_ahead(g, a.num_seqs));
+  for (int b0 = 0; b0 < a.num_seqs; b0 += most) {
+    const int nb = std::min(most, a.num_seqs - b0);
     DecodeParams p = fused ? *fused : DecodeParams{};
     if (FUSED) {  // this chunk's rows of the per-sequence inputs
       p.qkv += b0 * p.qkv_stride;
@@ -1030,13 +1156,9 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, c
     p.header = reinterpret_cast<int32_t*>(ws);
     p.part_o = reinterpret_cast<float*>(ws + kHeaderBytes);
     p.part_ml = p.part_o + static_cast<size_t>(ranges + nb) * a.num_q_heads * kDecodeHeadDim;
-    switch (G) {
-      case 1: launch_decode<1, FUSED>(p, ranges, s); break;
-      case 2: launch_decode<2, FUSED>(p, ranges, s); break;
-      case 4: launch_decode<4, FUSED>(p, ranges, s); break;
-      case 5: launch_decode<5, FUSED>(p, ranges, s); break;
-      default: launch_decode<8, FUSED>(p, ranges, s); break;
-    }
+    with_variant(g, a.num_seqs, [&](auto G, auto A) {
+      launch_decode<decltype(G)::value, FUSED, decltype(A)::value>(p, ranges, s);
+    });
     const int rc = launch_status(fn);
     if (rc != KVP_OK) return rc;
   }
@@ -1046,7 +1168,7 @@ static int enqueue_decode(const char* fn, const DecodeArgs& a, int64_t ranges, c
 // ---------------------------------------------------------------- no-allocation variant
 
 // Workspace of kvp_paged_decode_bf16_noalloc: one per device, held until the process ends.
-constexpr size_t kScratchBytes = 32u << 20;
+constexpr size_t kScratchBytes = 34u << 20;
 static __device__ __align__(256) char scratch[kScratchBytes];
 
 // Device address of this device's `scratch`, looked up once per device with that device

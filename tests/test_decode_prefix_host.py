@@ -79,13 +79,13 @@ int main(int argc, char** argv) {  // stride, max_blocks, block_size, then the c
   std::mutex lock;
   std::vector<uint16_t> out(B * 128, 1);
   DecodeParams p{ctx.data(), Table{&seen, &lock}, atoi(argv[1]), B, 1, atoi(argv[2]), atoi(argv[3]), out.data(), 128, 128};
-  std::vector<int> s_cum(B + 1, -1), s_ctx(B, -1);
+  std::vector<int> s_cum(B + 1, -1);
   int s_part[kDecodeWaves];
   std::vector<std::thread> ts;
   for (int t = 0; t < kDecodeThreads; ++t)
     ts.emplace_back([&, t] {
       threadIdx = {t, 0};
-      build_step_prefix(p, s_cum.data(), s_ctx.data(), s_part);
+      build_step_prefix(p, s_cum.data(), s_part);
     });
   for (auto& t : ts) t.join();
   for (int v : s_cum) printf("%d ", v);

@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from oracle import kvpath_oracle as ref
+from oracle import layers_oracle as lref
 from tests.helpers import TOL, contiguous_caches, gen, random_block_tables, randn_bf16
 from tests.test_fused_decode import _case as fused_case, _fused, _separate
 from tests.test_paged_decode import SCALE, _case as decode_case, _check, _decode
@@ -62,6 +63,55 @@ def test_more_sequences_than_one_launch(cuda_device):
     kc, vc = contiguous_caches(nb, bs, hkv, 128, g)
     bt = random_block_tables([int(c) for c in ctx], bs, nb, g)
     _check(cuda_device, randn_bf16((B, 4 * hkv, 128), g), kc, vc, bt, ctx)
+
+
+@pytest.mark.parametrize("G,hkv,B", [(1, 32, 2300), (2, 32, 2300), (8, 8, 2100)])
+def test_many_short_sequences_per_wave(cuda_device, G, hkv, B):
+    """More sequences than a wave's window of 64 holds and than a launch's tables, with runs of
+    empty ones across the windows' borders.  All sequences share eight pages."""
+    g, bs = gen(12 + G), 64
+    ctx = torch.randint(0, 41, (B,), generator=g, dtype=torch.int32)
+    ctx[100:300] = 0
+    ctx[1000:1064] = 0
+    ctx[B - 70:] = 0
+    kc, vc = contiguous_caches(8, bs, hkv, 128, g)
+    bt = torch.randint(0, 8, (B, 1), generator=g, dtype=torch.int32)
+    d = cuda_device
+    q = randn_bf16((B, G * hkv, 128), g)
+    out = _decode(q.to(d), kc.to(d), vc.to(d), ctx.to(d), bt.to(d)).cpu().float()
+    # all pages' keys at once, masked per sequence: [B, heads, 8 * bs]
+    qd, kd, vd = q.to(d).float(), kc.to(d).float(), vc.to(d).float()
+    s = torch.stack([torch.mm(qd[:, h], kd[:, :, h // G].reshape(-1, 128).t().contiguous()) for h in range(G * hkv)], 1)
+    at = torch.arange(8 * bs, device=d)
+    seen = (at[None] // bs == bt.to(d)) & (at[None] % bs < ctx.to(d)[:, None])
+    w = torch.softmax((s * SCALE).masked_fill(~seen[:, None], -math.inf), -1).nan_to_num(0.0)
+    want = torch.stack([torch.mm(w[:, h], vd[:, :, h // G].reshape(-1, 128)) for h in range(G * hkv)], 1)
+    torch.testing.assert_close(out, want.cpu(), **TOL)
+    assert torch.count_nonzero(out[ctx == 0]) == 0
+
+
+@pytest.mark.parametrize("G,hkv,B", [(1, 32, 2300), (2, 32, 1500), (8, 8, 1100)])
+def test_one_launch_step_of_many_short_sequences(cuda_device, G, hkv, B):
+    """The same for the one-launch step, against the separate launches: a page per sequence."""
+    d, g, hq, bs = cuda_device, gen(40 + G), G * hkv, 64
+    ctx = torch.randint(1, 41, (B,), generator=g, dtype=torch.int32)
+    ctx[90:170] = 0
+    pages = torch.randperm(B, generator=g).to(torch.int32)
+    slots = torch.where(ctx > 0, pages * bs + ctx - 1, -1)
+    dg = torch.Generator(device=d).manual_seed(G)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=dg, device=d, dtype=torch.bfloat16)
+
+    d1 = dict(pool=rand(B, 2 * bs * hkv * 128).view(torch.uint8), qkv=rand(B, (hq + 2 * hkv) * 128), qw=rand(128),
+              kw=rand(128), table=lref.rope_table(128, 64, 1e6).to(d), bt=pages[:, None].contiguous().to(d),
+              ctx=ctx.to(d), pos=(ctx - 1).clamp(min=0).to(d), slots=slots.to(torch.int32).to(d))
+    d2 = {k: v.clone() for k, v in d1.items()}
+    sep, one = _separate(d1, hq, hkv, bs), _fused(d2, hq, hkv, bs)
+    torch.cuda.synchronize()
+    assert torch.equal(d1["pool"], d2["pool"])
+    torch.testing.assert_close(one.float(), sep.float(), **TOL)
+    assert torch.count_nonzero(one[90:170]) == 0
 
 
 def test_strides_beyond_32_bit_offsets(cuda_device):
