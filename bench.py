@@ -861,9 +861,9 @@ def summarize_prefill_pmc(dir_a: str, dir_b: str, dir_c: str) -> int:
 
 # (profile file, kernel-name prefix, which occurrence group, algorithmic bytes or flops, unit)
 PROFILE_KERNELS = [
-    ("paged_decode_qwen3_0.6b", "void kvp::paged_decode_kernel<2, false>", "decode_0.6b"),
-    ("paged_decode_fused_qwen3_0.6b", "void kvp::paged_decode_kernel<2, true>", "decode_fused_0.6b"),
-    ("paged_decode_qwen3_8b", "void kvp::paged_decode_kernel<4, false>", "decode_8b"),
+    ("paged_decode_qwen3_0.6b", "void kvp::paged_decode_kernel<2, false, 2>", "decode_0.6b"),
+    ("paged_decode_fused_qwen3_0.6b", "void kvp::paged_decode_kernel<2, true, 2>", "decode_fused_0.6b"),
+    ("paged_decode_qwen3_8b", "void kvp::paged_decode_kernel<4, false, 2>", "decode_8b"),
     ("kv_append_4096tok", "void kvp::kv_append_kernel<128", "append"),
     ("varlen_prefill_prefix_32seq", "void kvp::varlen_prefill_kernel<2, true, true, false>", "prefill"),
     ("varlen_prefill_dense_32seq", "void kvp::varlen_prefill_kernel<2, false, true, false>", "prefill_dense"),

@@ -118,6 +118,14 @@ def reserve_decode_workspace(max_num_seqs: int, num_q_heads: int, head_dim: int,
         decode_workspace_bytes(max_num_seqs, num_q_heads, head_dim, max_blocks_per_seq, block_size))
 
 
+def _decode_workspace(index, stream, num_seqs, num_q_heads, head_dim, max_blocks, block_size) -> torch.Tensor:
+    nbytes = decode_workspace_bytes(num_seqs, num_q_heads, head_dim, 4 * max_blocks, block_size)
+    ws = _decode_workspaces.ready(index, stream, nbytes)
+    if ws is None:
+        ws = reserve_decode_workspace(num_seqs, num_q_heads, head_dim, max_blocks, block_size, index)
+    return ws
+
+
 # ----------------------------------------------------------------------------- prefill workspace
 
 _prefill_pool = Workspaces("prefill", "reserve_prefill_workspace")
@@ -148,7 +156,6 @@ def _may_split(num_seqs: int, max_seqlen_q: int, max_keys: int, num_q_heads: int
     return 0 < num_seqs * -(-max_seqlen_q // (128 // group)) * num_kv_heads <= _SPLIT_TILES
 
 
-@lru_cache(maxsize=4096)  # the layers of a step share one answer
 def _split_pays(num_seqs: int, total_q: int, max_seqlen_q: int, max_keys: int, num_q_heads: int,
                 num_kv_heads: int) -> bool:
     """Whether cutting the keys of a batch that may be split is likely to gain, from what the host
@@ -199,20 +206,37 @@ def reserve_prefill_workspace(num_seqs: int, max_seqlen_q: int, num_q_heads: int
     return _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, device)
 
 
-def _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, device) -> torch.Tensor:
+@lru_cache(maxsize=1024)
+def _work_list_bytes(num_seqs: int, max_seqlen_q: int, num_q_heads: int, num_kv_heads: int) -> int:
     nbytes = prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads)
-    # a power of two, so that batches of growing size allocate few buffers
-    return _prefill_pool.get(device, 1 << max(4095, nbytes - 1).bit_length(), nbytes)
+    return 1 << max(4095, nbytes - 1).bit_length()  # so that batches of growing size allocate few buffers
 
 
-def _prefill_workspace(num_seqs, total_q, max_seqlen_q, max_keys, num_q_heads, num_kv_heads, device) -> torch.Tensor:
+def _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, device) -> torch.Tensor:
+    return _prefill_pool.get(device, _work_list_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads),
+                             prefill_workspace_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
+
+
+@lru_cache(maxsize=4096)  # the layers of a step share one answer
+def _split_room(num_seqs, total_q, max_seqlen_q, max_keys, num_q_heads, num_kv_heads) -> int:
+    """Bytes of the workspace that a split launch of such a batch takes; 0 for an uncut one."""
     if _may_split(num_seqs, max_seqlen_q, max_keys, num_q_heads, num_kv_heads) and \
             _split_pays(num_seqs, total_q, max_seqlen_q, max_keys, num_q_heads, num_kv_heads):
-        ws = _split_pool.get(device, _prefill_split_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads),
-                             optional=True)
+        return _prefill_split_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads)
+    return 0
+
+
+def _prefill_workspace(index, stream, num_seqs, total_q, max_seqlen_q, max_keys, num_q_heads,
+                       num_kv_heads) -> torch.Tensor:
+    room = _split_room(num_seqs, total_q, max_seqlen_q, max_keys, num_q_heads, num_kv_heads)
+    if room:
+        ws = _split_pool.ready(index, stream, room)
+        if ws is None:
+            ws = _split_pool.get(index, room, optional=True)
         if ws is not None:  # inside a capture without it the launch is not split
             return ws
-    return _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, device)
+    ws = _prefill_pool.ready(index, stream, _work_list_bytes(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads))
+    return ws if ws is not None else _work_list(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads, index)
 
 
 def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -258,7 +282,8 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         if out3.shape != (B, Hq, D) or out3.dtype != torch.bfloat16 or out3.stride(2) != 1:
             raise ValueError("out must be bf16 [B, 1, Hq, D] or [B, Hq, D] with contiguous head_dim")
     max_blocks = block_table.shape[1]
-    ws = reserve_decode_workspace(B, Hq, D, max_blocks, block_size, q3.device)
+    stream = _stream(q3)
+    ws = _decode_workspace(q3.get_device(), stream, B, Hq, D, max_blocks, block_size)
     rc = lib().kvp_paged_decode_bf16(
         q3.data_ptr(), q_str[0], q_str[1],
         k_cache.data_ptr(), v_cache.data_ptr(),
@@ -267,7 +292,7 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         cache_seqlens.data_ptr(), B, Hq, Hkv, D, block_size, max_blocks,
         float(softmax_scale),
         out3.data_ptr(), out3.stride(0), out3.stride(1),
-        ws.data_ptr(), ws.numel(), _stream(q3))
+        ws.data_ptr(), ws.numel(), stream)
     check("kvp_paged_decode_bf16", rc)
     return out
 
@@ -306,7 +331,8 @@ def paged_decode_fused(qkv: torch.Tensor, cos_sin: torch.Tensor,
     if out is None:
         out = torch.empty(B, num_q_heads, D, dtype=torch.bfloat16, device=qkv.device)
     max_blocks = block_table.shape[1]
-    ws = reserve_decode_workspace(B, num_q_heads, D, max_blocks, block_size, qkv.device)
+    stream = _stream(qkv)
+    ws = _decode_workspace(qkv.get_device(), stream, B, num_q_heads, D, max_blocks, block_size)
     rc = lib().kvp_paged_decode_fused_bf16(
         qkv.data_ptr(), qkv.stride(0), cos_sin.data_ptr(), cos_sin.shape[0],
         q_norm_weight.data_ptr(), k_norm_weight.data_ptr(), float(eps),
@@ -314,7 +340,7 @@ def paged_decode_fused(qkv: torch.Tensor, cos_sin: torch.Tensor,
         num_blocks, slot_mapping.data_ptr(), block_table.data_ptr(), block_table.stride(0),
         cache_seqlens.data_ptr(), B, num_q_heads, num_kv_heads, D, block_size, max_blocks,
         float(softmax_scale), out.data_ptr(), out.stride(0), out.stride(1),
-        ws.data_ptr(), ws.numel(), _stream(qkv))
+        ws.data_ptr(), ws.numel(), stream)
     check("kvp_paged_decode_fused_bf16", rc)
     return out
 
@@ -368,12 +394,13 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, max_seqlen
         bt_ptr, bt_stride, max_blocks = block_table.data_ptr(), block_table.stride(0), block_table.shape[1]
     if k.shape[-1] != D:
         raise ValueError("head_dim mismatch between q and k")
-    ws = None
+    ws, stream = None, _stream(q)
     if num_seqs:
         max_keys = max_blocks * block_size if block_table is not None else int(max_seqlen_q)
         if isinstance(max_seqlen_k, int) and 0 < max_seqlen_k < max_keys:
             max_keys = max_seqlen_k
-        ws = _prefill_workspace(num_seqs, Tq, int(max_seqlen_q), max_keys if causal else 0, Hq, Hkv, q.device)
+        ws = _prefill_workspace(q.get_device(), stream, num_seqs, Tq, int(max_seqlen_q), max_keys if causal else 0, Hq,
+                                Hkv)
     rc = lib().kvp_varlen_prefill_bf16(
         q.data_ptr(), q.stride(0), q.stride(1),
         k.data_ptr(), *kstr,
@@ -382,7 +409,7 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, max_seqlen
         cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), num_seqs, int(max_seqlen_q),
         Hq, Hkv, D, float(softmax_scale), 1 if causal else 0,
         out.data_ptr(), out.stride(0), out.stride(1),
-        ws.data_ptr() if ws is not None else 0, ws.numel() if ws is not None else 0, _stream(q))
+        ws.data_ptr() if ws is not None else 0, ws.numel() if ws is not None else 0, stream)
     check("kvp_varlen_prefill_bf16", rc)
     return out
 

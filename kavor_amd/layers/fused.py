@@ -200,12 +200,15 @@ def greedy_argmax(logits: torch.Tensor, out: torch.Tensor | None = None) -> torc
         out = torch.empty(logits.shape[0], dtype=torch.int64, device=logits.device)
     if out.dtype != torch.int64 or not out.is_contiguous() or out.numel() != logits.shape[0]:
         raise ValueError("out must be a contiguous int64 tensor with one entry per row")
-    ws = argmax_workspace(logits.device)
+    stream = _stream(logits)
+    ws = _argmax_pool.ready(logits.get_device(), stream, _ARGMAX_WORKSPACE_BYTES)
+    if ws is None:
+        ws = argmax_workspace(logits.device)
     need = lib().kvp_argmax_workspace_bytes(logits.shape[0])
     if need > ws.numel():
         raise RuntimeError(f"argmax workspace of {ws.numel()} bytes, {need} needed")
     rc = lib().kvp_argmax_bf16(logits.data_ptr(), logits.stride(0), logits.shape[0], logits.shape[1],
-                               out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(logits))
+                               out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
     check("kvp_argmax_bf16", rc)
     return out
 
@@ -229,12 +232,15 @@ def sample(logits: torch.Tensor, temperatures: torch.Tensor, seed: torch.Tensor,
         out = torch.empty(n, dtype=torch.int64, device=logits.device)
     if out.dtype != torch.int64 or not out.is_contiguous() or out.numel() != n:
         raise ValueError("out must be a contiguous int64 tensor with one entry per row")
-    ws = argmax_workspace(logits.device)
+    stream = _stream(logits)
+    ws = _argmax_pool.ready(logits.get_device(), stream, _ARGMAX_WORKSPACE_BYTES)
+    if ws is None:
+        ws = argmax_workspace(logits.device)
     need = lib().kvp_argmax_workspace_bytes(n)
     if need > ws.numel():
         raise RuntimeError(f"argmax workspace of {ws.numel()} bytes, {need} needed")
     seed.add_(1)
     rc = lib().kvp_sample_bf16(logits.data_ptr(), logits.stride(0), n, logits.shape[1], temperatures.data_ptr(),
-                               seed.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(logits))
+                               seed.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
     check("kvp_sample_bf16", rc)
     return out

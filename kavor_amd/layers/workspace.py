@@ -29,6 +29,15 @@ class Workspaces:
         self.side: dict[tuple[int, int], torch.Tensor] = {}  # by device and stream handle
         self.captured: dict[int, torch.Tensor] = {}  # by device: the captured graphs'
 
+    def ready(self, index: int, stream: int, nbytes: int) -> torch.Tensor | None:
+        """The buffer of an eager call on the default stream, if it is there and large enough: what
+        nearly every call finds.  get() alone made host-bound calls 0.6 us slower (14.9 -> 15.6)."""
+        if stream == 0:
+            ws = self.default.get(index)
+            if ws is not None and ws.numel() >= nbytes and ws is not self.captured.get(index):
+                return ws
+        return None
+
     def get(self, device: torch.device | str | int, nbytes: int, least: int | None = None,
             optional: bool = False) -> torch.Tensor | None:
         """At least `nbytes` for calls on the device's current stream.  Inside a capture nothing
