@@ -290,6 +290,15 @@ __device__ __forceinline__ void fill_window(const DecodeParams& p, const int* s_
   asm volatile("" : "+v"(w.ctx), "+v"(w.slot), "+v"(w.blk));
 }
 
+// Puts the cursor into logical block lblk, whose id is blk, and loads the next one's ahead.
+__device__ __forceinline__ void cursor_enter_block(const DecodeParams& p, StepCursor& cur, int lblk, int blk) {
+  const int bad = blk < 0 || blk >= p.num_cache_blocks;
+  cur.bad |= bad;
+  cur.blk = bad ? 0 : blk;
+  cur.lblk = lblk;
+  cur.pf_blk = (lblk + 1) * p.block_size < cur.ctx ? load_uniform(p.block_tables + cur.b * p.bt_stride, lblk + 1) : -1;
+}
+
 // The cursor of the first step of sequence base + i.
 __device__ __forceinline__ void cursor_start_seq(const DecodeParams& p, StepCursor& cur, const SeqWindow& w, int i,
                                                  int buf) {
@@ -298,12 +307,9 @@ __device__ __forceinline__ void cursor_start_seq(const DecodeParams& p, StepCurs
   cur.j = 0;
   cur.ctx = __builtin_amdgcn_readlane(w.ctx, i);
   cur.slot = __builtin_amdgcn_readlane(w.slot, i);
-  cur.blk = __builtin_amdgcn_readlane(w.blk, i);
   cur.nsteps = (cur.ctx + kStep - 1) / kStep;
-  cur.lblk = 0;
-  cur.bad = cur.blk < 0 || cur.blk >= p.num_cache_blocks;
-  if (cur.bad) cur.blk = 0;
-  cur.pf_blk = p.block_size < cur.ctx ? load_uniform(p.block_tables + cur.b * p.bt_stride, 1) : -1;
+  cur.bad = 0;
+  cursor_enter_block(p, cur, 0, __builtin_amdgcn_readlane(w.blk, i));
 }
 
 // Element offset of the cursor's step in the caches, and the number of valid tokens of the
@@ -312,17 +318,10 @@ __device__ __forceinline__ void cursor_start_seq(const DecodeParams& p, StepCurs
 __device__ __forceinline__ int64_t step_base(const DecodeParams& p, StepCursor& cur, int64_t head_off, int& nvalid) {
   const int t0 = cur.j * kStep;
   const int lblk = div_by(t0, p.div_block);
-  if (lblk != cur.lblk) {
-    const int32_t* row = p.block_tables + cur.b * p.bt_stride;
-    int blk = (cur.lblk >= 0 && lblk == cur.lblk + 1 && cur.pf_blk != -1) ? cur.pf_blk : load_uniform(row, lblk);
-    if (blk < 0 || blk >= p.num_cache_blocks) {
-      cur.bad = 1;
-      blk = 0;
-    }
-    cur.blk = blk;
-    cur.lblk = lblk;
-    cur.pf_blk = (lblk + 1) * p.block_size < cur.ctx ? load_uniform(row, lblk + 1) : -1;
-  }
+  if (lblk != cur.lblk)
+    cursor_enter_block(p, cur, lblk, lblk == cur.lblk + 1 && cur.pf_blk != -1
+                                         ? cur.pf_blk
+                                         : load_uniform(p.block_tables + cur.b * p.bt_stride, lblk));
   nvalid = min(kStep, cur.ctx - t0);
   return static_cast<int64_t>(cur.blk) * p.blk_stride +
          static_cast<int64_t>(t0 - lblk * p.block_size) * p.slot_stride + head_off;
@@ -431,26 +430,42 @@ __device__ __forceinline__ void read_v_tile(const u32 (&a)[8], u32x2_t (&lo)[8],
       : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7])
       : "memory");
 }
-// A head's chunk normalised and rotated (chunk c of the head at x_at), by the norm weights at w_at
-// and the cos/sin row at table_at.
-__device__ __forceinline__ uint4 norm_rope_chunk(u32 w_at, u32 table_at, u32 x_at, int c, bool pos_ok, float eps) {
-  u32x4_t hw, hx, hc[2], hs[2];
-  asm volatile(
-      "ds_read_b128 %0, %6\n\tds_read_b128 %1, %8\n\tds_read_b128 %2, %7\n\tds_read_b128 %3, %7 offset:16\n\t"
-      "ds_read_b128 %4, %7 offset:256\n\tds_read_b128 %5, %7 offset:272\n\ts_waitcnt lgkmcnt(0)"
-      : "=&v"(hw), "=&v"(hx), "=&v"(hc[0]), "=&v"(hc[1]), "=&v"(hs[0]), "=&v"(hs[1])
-      : "v"(w_at), "v"(table_at), "v"(x_at)
-      : "memory");
-  float w[8], x[8], cs[8], sn[8];
-  unpack8(__builtin_bit_cast(uint4, hw), w);
-  unpack8(__builtin_bit_cast(uint4, hx), x);
+// N (1 or 2) heads' chunks normalised and rotated: chunk c of the head at x_at[i], by the norm
+// weights at w_at[i] and the cos/sin row at table_at.
+template <int N>
+__device__ __forceinline__ void norm_rope_chunks(const u32 (&w_at)[N], u32 table_at, const u32 (&x_at)[N], int c,
+                                                 bool pos_ok, float eps, uint4 (&out)[N]) {
+  u32x4_t hw[2], hx[2], hc[2], hs[2];
+  if constexpr (N == 1) {
+    asm volatile(
+        "ds_read_b128 %0, %6\n\tds_read_b128 %1, %8\n\tds_read_b128 %2, %7\n\tds_read_b128 %3, %7 offset:16\n\t"
+        "ds_read_b128 %4, %7 offset:256\n\tds_read_b128 %5, %7 offset:272\n\ts_waitcnt lgkmcnt(0)"
+        : "=&v"(hw[0]), "=&v"(hx[0]), "=&v"(hc[0]), "=&v"(hc[1]), "=&v"(hs[0]), "=&v"(hs[1])
+        : "v"(w_at[0]), "v"(table_at), "v"(x_at[0])
+        : "memory");
+  } else {
+    asm volatile(
+        "ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\tds_read_b128 %2, %11\n\tds_read_b128 %3, %12\n\t"
+        "ds_read_b128 %4, %10\n\tds_read_b128 %5, %10 offset:16\n\tds_read_b128 %6, %10 offset:256\n\t"
+        "ds_read_b128 %7, %10 offset:272\n\ts_waitcnt lgkmcnt(0)"
+        : "=&v"(hw[0]), "=&v"(hw[1]), "=&v"(hx[0]), "=&v"(hx[1]), "=&v"(hc[0]), "=&v"(hc[1]), "=&v"(hs[0]), "=&v"(hs[1])
+        : "v"(w_at[0]), "v"(w_at[1]), "v"(table_at), "v"(x_at[0]), "v"(x_at[1])
+        : "memory");
+  }
+  float cs[8], sn[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     cs[e] = __uint_as_float(hc[e >> 2][e & 3]);
     sn[e] = __uint_as_float(hs[e >> 2][e & 3]);
   }
-  norm_rope_head(x, w, cs, sn, c < 8, pos_ok, eps);
-  return pack8(x);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    float w[8], x[8];
+    unpack8(__builtin_bit_cast(uint4, hw[i]), w);
+    unpack8(__builtin_bit_cast(uint4, hx[i]), x);
+    norm_rope_head(x, w, cs, sn, c < 8, pos_ok, eps);
+    out[i] = pack8(x);
+  }
 }
 // Two 16-byte chunks.
 __device__ __forceinline__ void read_pair(u32 a, u32 b, u32x4_t& x, u32x4_t& y) {
@@ -715,16 +730,28 @@ void paged_decode_kernel(const DecodeParams p) {
   // At a range's first step of a sequence.  `ends`: the sequence's last step is in the range.
   auto finish_q = [&](const StepCursor& c, bool ends, u32x4_t (&dst)[4]) {
     const u32 q_at = q_base + kQBytes * c.buf;
-    if constexpr (FUSED) {  // four heads at a time; head G is the new token's k
+    if constexpr (FUSED) {  // four heads to a pass, two passes interleaved; head G is the new token's k
       const bool pos_ok = c.ctx - 1 >= 0 && c.ctx - 1 < p.max_position;
+      auto passes = [&](auto n_c, int g0) {  // heads g0 + q4, and g0 + 4 + q4
+        constexpr int N = decltype(n_c)::value;
+        u32 x[N], w[N];
+        uint4 y[N];
 #pragma unroll
-      for (int g0 = 0; g0 <= G; g0 += 4) {
-        if (g0 == G && !ends) break;
-        const int g = min(g0 + q4, G);
-        const u32 x_at = q_at + kQRow + 256 * g + 16 * n;
-        const uint4 y = norm_rope_chunk(w_at + (g == G ? 256 : 0) + 16 * n, q_at + 32 * (n & 7), x_at, n, pos_ok, p.eps);
-        if (g0 + q4 <= G) write_tile16(x_at, y);
-      }
+        for (int i = 0; i < N; ++i) {
+          const int g = min(g0 + 4 * i + q4, G);
+          x[i] = q_at + kQRow + 256 * g + 16 * n;
+          w[i] = w_at + (g == G ? 256 : 0) + 16 * n;
+        }
+        norm_rope_chunks<N>(w, q_at + 32 * (n & 7), x, n, pos_ok, p.eps, y);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+          if (g0 + 4 * i + q4 <= G) write_tile16(x[i], y[i]);
+      };
+      constexpr std::integral_constant<int, 1> one{};
+      constexpr std::integral_constant<int, 2> two{};
+      if (G < 4 || (G == 4 && !ends)) passes(one, 0);
+      else passes(two, 0);
+      if (G == 8 && ends) passes(one, 8);
     }
     read_q(q_at + kQRow + 256 * hg + 16 * q4, dst);
   };
@@ -778,21 +805,20 @@ void paged_decode_kernel(const DecodeParams p) {
   int issued = 0;
   const int tile_ops = p.rows_by_dma ? 8 : 0;
   if (FUSED) fz_issue_weights(p, lane, s_fw);
-  // The first step, from a window that starts at its sequence; its block, if not the sequence's
-  // first, is loaded with the window.
-  const int j0 = S0 - __builtin_amdgcn_readfirstlane(s_cum[lo]);
-  const int lblk0 = div_by(j0 * kStep, p.div_block);
-  int blk0 = 0;
-  if (lblk0 > 0) blk0 = load_uniform(p.block_tables + lo * p.bt_stride, lblk0);
-  SeqWindow win;
-  fill_window<FUSED>(p, s_cum, lo, lane, win);
-  cursor_start_seq(p, cn, win, 0, 0);
-  cn.j = j0;
-  if (lblk0 > 0) {
-    cn.lblk = lblk0 - 1;  // step_base takes the block over as one loaded ahead
-    cn.bad = 0;
-    cn.pf_blk = blk0;
-  }
+  // The first step, and, if the range goes on into other sequences, their window: all of it loaded
+  // together.  (The first sequence from the window as well: one of 19008 tokens, a step or five to
+  // a range, 25.9 -> 26.3 us per layer.)
+  const int cum_lo = __builtin_amdgcn_readfirstlane(s_cum[lo]), cum_hi = __builtin_amdgcn_readfirstlane(s_cum[lo + 1]);
+  cn.b = lo;
+  cn.j = S0 - cum_lo;
+  cn.nsteps = cum_hi - cum_lo;
+  cn.ctx = load_uniform(p.context_lens, lo);
+  cn.slot = FUSED ? load_uniform(p.slot_mapping, lo) : 0;
+  const int lblk0 = div_by(cn.j * kStep, p.div_block);
+  const int blk0 = load_uniform(p.block_tables + lo * p.bt_stride, lblk0);
+  SeqWindow win{};
+  if (cum_hi < S1) fill_window<FUSED>(p, s_cum, lo + 1, lane, win);
+  cursor_enter_block(p, cn, lblk0, blk0);
   for (int S = S0 - A; S < S1; ++S) {
     char* const tiles = s_tile[wave][(S - S0) & (A - 1)];
     const u32 tile = lds_addr(tiles);
