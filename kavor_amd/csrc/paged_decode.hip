@@ -12,11 +12,12 @@
 //   laid end to end (prefix sums of ceil(ctx / 32), built in LDS by every workgroup from
 //   context_lens).  The grid is the number of workgroups the GPU holds at once (one of 4
 //   waves per CU; two for many sequences at G = 1, see steps_ahead), and no more than the
-//   block tables can hold steps for, so a captured graph launches few empty workgroups.  A workgroup's waves are 4 kv heads;
-//   ceil(Hkv / 4) workgroups walk one contiguous range of steps for all kv heads (kv heads
-//   of one token row share HBM pages and are fetched together).  Every range gets the same
-//   number of steps (exact balance whatever the context lengths).  A wave owns all
-//   G = Hq / Hkv query heads of its kv head, so GQA costs no extra KV traffic.
+//   block tables can hold steps for, so a captured graph launches few empty workgroups.  A
+//   workgroup's waves are 4 kv heads; ceil(Hkv / 4) workgroups walk one contiguous range of
+//   steps for all kv heads (kv heads of one token row share HBM pages and are fetched
+//   together).  Every range gets the same number of steps (exact balance whatever the context
+//   lengths).  A wave owns all G = Hq / Hkv query heads of its kv head, so GQA costs no extra
+//   KV traffic.
 //
 // Why the matrix cores, although the work is HBM-bound: on the vector ALUs the q.k dot
 // products, their lane sums and the P V products grow with G while the K/V bytes do not.
@@ -25,9 +26,10 @@
 // v_mfma_f32_16x16x32_bf16 with the G heads as columns, a fixed 16 (G <= 5) or 24 (G = 8)
 // matrix instructions per step.  Measured against the vector-ALU kernel (MI355X, whole
 // calls, the two in turn): 64 sequences of 1000-9000 tokens at G = 8, one-launch step:
-// 382 -> 215 us (3.4 -> 6.1 TB/s); 128 sequences of 1024-32768 tokens at G = 4: 1300 ->
-// 1269 us (7.0 TB/s); 256 sequences of 100-2048 tokens at G = 2, with the append: 182 ->
-// 177 us; 8 sequences of 600-3000 tokens at G = 2: 22.8 -> 21.8 us per layer.
+// 382 -> 215 us (3.4 -> 6.1 TB/s); 256 sequences of 100-2048 tokens at G = 2, with the append:
+// 182 -> 177 us; 8 sequences of 600-3000 tokens at G = 2: 22.8 -> 20.5 us per layer.  128
+// sequences of 1024-32768 tokens at G = 4 take what a streaming read takes (1.27 ms, 7.0 TB/s)
+// with either.
 //
 // K and V rows go from memory into the wave's own LDS tiles (32 tokens x 256 bytes, two of
 // each) with direct-to-LDS buffer loads: no register holds them, no barrier is needed, and
@@ -36,11 +38,11 @@
 // longer than their steps: a wave has one SIMD to itself and nothing to hide the vector work
 // behind.  So a sequence's lengths, block id and slot come from lanes (SeqWindow), its q and new
 // token with its first tiles, q and the new k share their norms and rotations, and the waits
-// count what is in flight exactly (see the loop): 4096 sequences of 1-60 tokens, one-launch step,
+// count what is in flight (see the loop): 4096 sequences of 1-60 tokens, one-launch step,
 // G = 2 223 -> 152 us, G = 1 219 -> 136; 1024 of 10-100 70.7 -> 63.2 and 68.2 -> 55.9; one of
-// 611 tokens, 28 layers 308 -> 292.  They are read with the nontemporal hint; rows past the
-// context are clamped onto its last token (masked in the softmax), so no branch guards a
-// load.
+// 611 tokens, 28 layers 307 -> 288.  The rows are read with the nontemporal hint.  Those past
+// the context are clamped onto its last token, so no branch guards a load; the softmax masks
+// them, and their V is cleared (0 times an infinity is a NaN).
 //
 // Layouts (lane l: n = l % 16, q4 = l / 16).  S = K Q^T: A is the K tile (row n of 16
 // tokens, dims 8 q4 + e of each 32), B is q (column n); the lane gets the scores of tokens

@@ -126,7 +126,7 @@ struct PrefillParams {
 // SPT sequences per thread: 1 up to kPlanThreads sequences, otherwise as many as a launch
 // may have.  With one, the hash table is small and the placement, a chain of LDS atomics per
 // sequence, is spread over a wave: 32 sequences of up to 8 pairs 6.3 -> 5.2 us, 2 of 128 pairs
-// 11.0 -> 4.8 us (the whole call of two 8192-token prompts 1002 -> 995 us).
+// 11.0 -> 4.8 us.
 template <int G, int SPT>
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const PrefillParams p) {
   constexpr int TOK = kPrefillRows / G;
@@ -1275,7 +1275,8 @@ extern "C" int kvp_varlen_prefill_bf16(const void* q, int64_t q_tok_stride, int6
   // partial states.  The tile count is a bound, exact for one sequence: its tiles all walk a
   // long cached prefix, and from about 3/4 of the slots on two halves of each take as long as
   // the whole (1500 new tokens on 15000 cached, 376 tiles: 406 us unsplit, 413 us with the
-  // split plan, which then cuts nothing).
+  // split plan, which then cuts nothing).  A caller that knows its lengths, and that nothing will
+  // be cut, passes a workspace without the partial states.
   const int64_t most_keys = paged ? static_cast<int64_t>(max_blocks_per_seq) * block_size : max_seqlen_q;
   p.tile_slots = static_cast<int32_t>(split_tile_slots(num_seqs, max_seqlen_q, G, num_kv_heads));
   p.split = nullptr;
